@@ -1,0 +1,677 @@
+"""The framework's work as its users ask for it, through its public entry points, to time and to compare.
+
+What a program does with the rasteriser: draw one frame of a packed cloud
+(TileRasterizer.render), a batch of views of it (render_views), a frame over an
+under-layer with points among the splats (render with points and under), a cut
+of its levels of detail (lod_select, then render), train a cloud's FP32 parameters
+from one view or from many (autograd.rasterize, rasterize_views), and sort pairs
+(radix_sort). listed() has the sizes of the repository's own workloads and small
+and odd ones beside them; draw() spreads over the ranges between.
+
+exact() is the image definition again in float64, in plain torch: the EWA
+projection, the splats in (24-bit depth key, index) order, and every pixel's
+front-to-back sum over the splats of its tile; gradients by torch's autograd.
+"""
+import math
+
+import numpy as np
+import torch
+
+from lucabrtrender_amd import autograd, raster
+
+NEAR, FAR, HAPERTURE = 0.1, 10000.0, 24.576
+REST = (0, 3, 8, 15)                      # rest coefficients a colour at each degree
+SH_C0 = 0.28209479177387814
+VIEW_SIZES = ((256, 256), (512, 384), (960, 540), (1280, 720), (1920, 1080))
+PARAMS = ("means", "log_scales", "quats", "opacity_logits", "sh")
+
+
+# ---- the cases ---------------------------------------------------------------
+
+def _frame(name, scene, splats, width, height, degree, **more):
+    case = dict(name=name, kind="frame", scene=scene, splats=splats, width=width, height=height, degree=degree,
+                antialias=True, filter3d=False, dilation=0.3, depth_mode=0, linearise=True, background=0.0)
+    case.update(more)
+    return case
+
+
+def listed():
+    return [
+        # A thumbnail of a small asset: launches and waits are all there is.
+        _frame("frame-2k-160x120", "cube", 2048, 160, 120, 0),
+        # The small workload of the benchmark: one object, no harmonics.
+        _frame("frame-65k-640x480", "cube", 65536, 640, 480, 0),
+        # An odd window size, the other options: no antialiasing, the depth where
+        # the coverage passes a half, a background, encoded colours.
+        _frame("frame-1M-1571x877", "cube", 1_000_000, 1571, 877, 2, antialias=False, depth_mode=1, linearise=False,
+               background=0.5),
+        # The headline frame: an interactive view of a captured scene.
+        _frame("frame-3M-1080p", "clusters", 3_000_000, 1920, 1080, 3, filter3d=True, dilation=0.1),
+        # Splats close to a 4K camera, each over hundreds of tiles: the sort.
+        _frame("frame-6M-2160p", "stress", 6_000_000, 3840, 2160, 3),
+        # A dataset's views, rendered at once (evaluation, serving), replayed as a graph.
+        dict(name="views-2M-64", kind="views", splats=2_000_000, views=64, degree=3, graph=True),
+        # One step of training a small object at an odd size, from one view.
+        dict(name="train-30k-489x363", kind="train", scene="cube", splats=30_001, width=489, height=363, degree=1),
+        # One step of training a scene, from one view.
+        dict(name="train-1M-720p", kind="train", scene="cube", splats=1_000_000, width=1280, height=720, degree=3),
+        # One step of training a scene, from a batch of views of several sizes.
+        dict(name="train-1M-24views", kind="train_views", splats=1_000_000, views=24, degree=3),
+        # Splats with a point cloud among them, over a rendered layer.
+        dict(name="points-3M+1M-1080p", kind="composite", splats=3_000_000, points=1_000_000, width=1920, height=1080,
+             degree=3),
+        # A far view through the levels of detail: the cut, then its frame.
+        dict(name="lod-2M-1080p", kind="lod", splats=2_000_000, width=1920, height=1080, degree=3, pixels=4.0),
+        # A caller's own pairs, 40 key bits.
+        dict(name="sort-30M-40bit", kind="sort", pairs=30_000_001, bits=40),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(("frame",) * 5 + ("train",) * 2 + ("views", "train_views", "composite", "lod", "sort"))
+    degree = rng.choice((0, 1, 2, 3, 3))
+    width = _log(rng, 160, 3840)
+    height = max(90, min(2160, int(width * rng.uniform(0.5, 1.0))))
+    if kind == "frame":
+        case = _frame("", rng.choice(("cube", "clusters")), _log(rng, 2000, 3_000_000), width, height, degree,
+                      antialias=rng.random() < 0.7, filter3d=rng.random() < 0.5, dilation=rng.choice((0.1, 0.3)),
+                      depth_mode=rng.choice((0, 0, 1)), linearise=rng.random() < 0.7,
+                      background=rng.choice((0.0, 0.0, 0.5)))
+        del case["name"]
+        return case
+    if kind == "train":
+        width = min(width, 1920)
+        return dict(kind=kind, scene=rng.choice(("cube", "clusters")), splats=_log(rng, 5000, 1_500_000), width=width,
+                    height=min(height, 1080), degree=degree)
+    if kind == "views":
+        return dict(kind=kind, splats=_log(rng, 20_000, 2_000_000), views=rng.randint(4, 64), degree=degree,
+                    graph=rng.random() < 0.5)
+    if kind == "train_views":
+        return dict(kind=kind, splats=_log(rng, 20_000, 1_000_000), views=rng.randint(3, 24), degree=degree)
+    if kind == "composite":
+        return dict(kind=kind, splats=_log(rng, 20_000, 3_000_000), points=_log(rng, 5000, 1_000_000), width=width,
+                    height=height, degree=degree)
+    if kind == "lod":
+        return dict(kind=kind, splats=_log(rng, 50_000, 2_000_000), width=width, height=height, degree=degree,
+                    pixels=rng.choice((2.0, 4.0, 8.0)))
+    return dict(kind=kind, pairs=_log(rng, 2000, 60_000_000), bits=rng.randint(16, 48))
+
+
+# ---- inputs ------------------------------------------------------------------
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _cloud(scene, n, degree, g):
+    """A cloud's values before packing, float32 on the GPU, as scenes.py lays its scenes out: positions (the
+    camera of "cube" and "stress" is at the origin looking down -z, that of "clusters" orbits the origin),
+    log-scales, quaternions x y z w, opacities, base colours and rest coefficients [n, rest, 3]."""
+    def normal(*shape):
+        return torch.randn(shape, generator=g, device="cuda")
+
+    def uniform(*shape):
+        return torch.rand(shape, generator=g, device="cuda")
+
+    logits = normal(n)
+    if scene == "clusters":
+        centres, sds = 20.0 * uniform(256, 3) - 10.0, 0.05 + 0.95 * uniform(256, 3)
+        member = torch.randint(0, 256, (n,), generator=g, device="cuda")
+        xyz = centres[member] + normal(n, 3) * sds[member]
+        log_scales = -5.0 + 0.8 * normal(n, 3)
+    else:
+        xyz = 2.0 * uniform(n, 3) - 1.0
+        xyz[:, 2] -= 4.0
+        log_scales = -4.0 + 0.5 * normal(n, 3)
+        if scene == "stress":   # a fifth of them pulled toward the camera
+            near = uniform(n) < 0.2
+            xyz = torch.where(near[:, None], xyz * (0.2 + 0.8 * uniform(n, 1)), xyz)
+            log_scales = torch.where(near[:, None], -3.6 + 0.3 * normal(n, 3), log_scales)
+            logits = logits + 1.0
+    rest = normal(n, REST[degree], 3)
+    band = torch.tensor([1.0] * 3 + [2.0] * 5 + [3.0] * 7, device="cuda")[:REST[degree]]
+    return dict(xyz=xyz, log_scales=log_scales, quats=normal(n, 4), logits=logits, base=uniform(n, 3),
+                rest=rest * (0.3 / band[None, :, None]))
+
+
+def _pack(c):
+    """The packed cloud (positions, shape, sh) of the values: opacities in positions.w, halves two a word, the
+    quaternion as its three smallest components in ten bits each."""
+    n = c["xyz"].shape[0]
+    positions = torch.cat([c["xyz"], torch.sigmoid(c["logits"])[:, None]], 1).contiguous()
+    q = torch.nn.functional.normalize(c["quats"], dim=1)
+    largest = q.abs().argmax(1)
+    q = q * torch.where(q.gather(1, largest[:, None]) < 0, -1.0, 1.0)
+    at = torch.tensor([[1, 2, 3], [0, 2, 3], [0, 1, 3], [0, 1, 2]], device="cuda")[largest]
+    unit = (q.gather(1, at) / 0.70710678 * 0.5 + 0.5).clamp(0.0, 1.0)
+    ten = torch.round(unit * 1023.0).to(torch.int64)
+    word = (ten[:, 0] << 22) | (ten[:, 1] << 12) | (ten[:, 2] << 2) | largest
+    word = torch.where(word >= 1 << 31, word - (1 << 32), word).to(torch.int32)
+    halves = torch.cat([c["log_scales"], c["base"]], 1).to(torch.float16).contiguous().view(torch.int32)
+    shape = torch.cat([word[:, None], halves], 1).contiguous()
+    rest = c["rest"].shape[1]
+    sh = None
+    if rest:
+        flat = torch.zeros((n, (rest * 3 + 1) // 2 * 2), dtype=torch.float16, device="cuda")
+        flat[:, :rest * 3] = c["rest"].reshape(n, -1).to(torch.float16)
+        sh = flat.view(torch.int32)
+    return positions, shape, sh
+
+
+def _filter3d(xyz, cameras, width):
+    """Mip-Splatting's 3D filter size a splat: sqrt(0.2) times its least depth / focal over the cameras in front of it."""
+    best = torch.full((xyz.shape[0],), math.inf, device="cuda")
+    for cam in cameras:
+        m = torch.tensor(_camera_numbers(cam, width, width)["m"][2], dtype=torch.float32, device="cuda")
+        z = xyz @ m[:3] + m[3]
+        best = torch.where(z > 0.2, torch.minimum(best, z), best)
+    best = torch.where(torch.isfinite(best), best, torch.ones_like(best))
+    return (best * (math.sqrt(0.2) / _focal(width))).contiguous()
+
+
+def _focal(width):
+    return width / (2.0 * math.tan(math.radians(30.0)))   # 60 degrees across the frame
+
+
+def _looking(eye, target, up=(0.0, 1.0, 0.0)):
+    """A camera as plain numbers: where it is, what it looks at, what is up."""
+    return tuple(eye), tuple(target), tuple(up)
+
+
+def _to_camera(cam):
+    out = raster.Camera.looking_at(*cam)
+    out.lens = raster.Lens(focal=HAPERTURE / (2.0 * math.tan(math.radians(30.0))), near_z=NEAR, far_z=FAR)
+    return out
+
+
+def _scene_camera(scene, angle=0.0):
+    if scene in ("cube", "stress"):
+        return _looking((0.0, 0.0, 0.0), (0.0, 0.0, -1.0))
+    a = math.radians(angle)
+    return _looking((15.0 * math.sin(a), 0.0, 15.0 * math.cos(a)), (0.0, 0.0, 0.0))
+
+
+def _sphere_views(count):
+    """Cameras on a sphere of radius 12 about the origin (a Fibonacci lattice), their sizes in turn from VIEW_SIZES."""
+    views = []
+    for k in range(count):
+        y = 1.0 - 2.0 * (k + 0.5) / count
+        r, a = math.sqrt(1.0 - y * y), math.pi * (3.0 - math.sqrt(5.0)) * k
+        up = (0.0, 0.0, 1.0) if abs(y) > 0.95 else (0.0, 1.0, 0.0)
+        views.append((_looking((12.0 * r * math.cos(a), 12.0 * y, 12.0 * r * math.sin(a)), (0.0, 0.0, 0.0), up),
+                      VIEW_SIZES[(k * 7 + 3) % len(VIEW_SIZES)]))
+    return views
+
+
+def _flat_targets(sizes):
+    """Every view's images in two buffers, as a program that fetches them at once keeps them."""
+    pixels = sum(w * h for w, h in sizes)
+    colour = torch.zeros((pixels, 4), dtype=torch.float32, device="cuda")
+    depth = torch.zeros((pixels,), dtype=torch.float32, device="cuda")
+    targets, at = [], 0
+    for w, h in sizes:
+        t = raster.RenderTargets(1, 1)
+        t.width, t.height = w, h
+        t.colour, t.depth = colour[at:at + w * h].view(h, w, 4), depth[at:at + w * h].view(h, w)
+        targets.append(t)
+        at += w * h
+    return colour, depth, targets
+
+
+def _values(case, seed):
+    """The values of a case's cloud, its points and its under-layer: what prepare() packs and exact() starts from."""
+    g = _generator(seed)
+    kind = case["kind"]
+    scene = case.get("scene", "clusters")
+    v = dict(cloud=_cloud(scene, case["splats"], case["degree"], g))
+    if kind == "composite":
+        # A point cloud about some of the splats' places, and a layer rendered behind part of the frame.
+        n, h, w = case["points"], case["height"], case["width"]
+        pick = torch.randint(0, case["splats"], (n,), generator=g, device="cuda")
+        v["points"] = v["cloud"]["xyz"][pick] + 0.05 * torch.randn((n, 3), generator=g, device="cuda")
+        v["point_rgb"] = torch.rand((n, 3), generator=g, device="cuda")
+        y, x = torch.meshgrid(torch.arange(h, device="cuda"), torch.arange(w, device="cuda"), indexing="ij")
+        z = 15.0 + 4.0 * torch.sin(x * (9.0 / w)) * torch.cos(y * (7.0 / h))
+        v["under_depth"] = torch.where((x * 3 + y * 2) % 640 < 480, z, torch.zeros_like(z)).float().contiguous()
+        v["under_colour"] = torch.rand((h, w, 4), generator=g, device="cuda")
+    if kind in ("train", "train_views"):
+        sizes = [(case["width"], case["height"])] if kind == "train" else [s for _, s in _sphere_views(case["views"])]
+        v["grads"] = [torch.randn((h, w, 4), generator=g, device="cuda") for w, h in sizes]
+    return v
+
+
+def _settings(case):
+    return raster.RenderSettings(width=case.get("width", 16), height=case.get("height", 16),
+                                 antialias=case.get("antialias", True), filter3d=case.get("filter3d", False),
+                                 dilation=case.get("dilation", 0.3), depth_mode=case.get("depth_mode", 0),
+                                 linearise=case.get("linearise", True),
+                                 background=(case.get("background", 0.0),) * 4, use_graph=case.get("graph", False))
+
+
+def _sort_inputs(case, seed):
+    g = _generator(seed)
+    keys = torch.randint(0, 1 << case["bits"], (case["pairs"],), generator=g, device="cuda")
+    return keys, torch.arange(case["pairs"], dtype=torch.int32, device="cuda")
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "sort":
+        keys, values = _sort_inputs(case, seed)
+        return dict(kind=kind, rast=raster.TileRasterizer(), bits=case["bits"], given=(keys, values),
+                    pairs=(keys.clone(), values.clone()), scratch=(torch.empty_like(keys), torch.empty_like(values)))
+    v = _values(case, seed)
+    state = dict(kind=kind, rast=raster.TileRasterizer(), settings=_settings(case))
+    if kind in ("train", "train_views"):
+        c = v["cloud"]
+        sh = torch.cat([((c["base"] - 0.5) / SH_C0)[:, None, :], c["rest"]], 1).contiguous()
+        params = (c["xyz"].contiguous(), c["log_scales"], c["quats"], c["logits"], sh)
+        state["params"] = [p.clone().requires_grad_() for p in params]
+        state["grads"] = v["grads"]
+        if kind == "train":
+            state["camera"] = _to_camera(_scene_camera(case["scene"], 20.0))
+        else:
+            views = _sphere_views(case["views"])
+            state["cameras"], state["sizes"] = [_to_camera(c) for c, _ in views], [s for _, s in views]
+        return state
+    positions, shape, sh = _pack(v["cloud"])
+    f3 = None
+    if case.get("filter3d"):
+        f3 = _filter3d(v["cloud"]["xyz"], _filter_cameras(case), case["width"])
+    cloud = raster.GpuSplats(positions, shape, sh, REST[case["degree"]], f3)
+    state["instances"] = [raster.SplatInstance(cloud)]
+    if kind == "views":
+        views = _sphere_views(case["views"])
+        state["colour"], state["depth"], targets = _flat_targets([s for _, s in views])
+        state["views"] = [raster.View(_to_camera(c), t) for (c, _), t in zip(views, targets)]
+        return state
+    state["targets"] = raster.RenderTargets(case["width"], case["height"])
+    if kind == "frame":
+        state["camera"] = _to_camera(_scene_camera(case["scene"], 20.0))
+    elif kind == "composite":
+        state["camera"] = _to_camera(_scene_camera("clusters", 20.0))
+        xyz1 = torch.cat([v["points"], torch.ones_like(v["points"][:, :1])], 1).contiguous()
+        rgb1 = torch.cat([v["point_rgb"], torch.ones_like(v["point_rgb"][:, :1])], 1).to(torch.float16).contiguous()
+        points = raster.GpuPoints(xyz1, rgb1.view(torch.int32))
+        style = raster.PointStyle(size_mode=raster.PointStyle.PIXELS, size=2.0)
+        state["points"] = [raster.PointInstance(points, style=style)]
+        under = raster.RenderTargets(1, 1)
+        under.width, under.height = case["width"], case["height"]
+        under.colour, under.depth = v["under_colour"], v["under_depth"]
+        state["under"] = under
+    else:
+        state["camera"] = _to_camera(_looking((0.0, 0.0, 60.0), (0.0, 0.0, 0.0)))
+        state["lod"] = [raster.LodInstance(state["rast"].lod_build(cloud))]
+        state["pixels"] = case["pixels"]
+    return state
+
+
+def _filter_cameras(case):
+    if case["scene"] == "cube":
+        return [_scene_camera("cube")]
+    return [_scene_camera("clusters", 360.0 * k / 16.0) for k in range(16)]
+
+
+# ---- one pass ----------------------------------------------------------------
+
+def _stats(st):
+    return {"visible": st.visible, "pairs": st.pairs}
+
+
+def run(state):
+    kind, rast = state["kind"], state["rast"]
+    if kind == "sort":
+        for to, given in zip(state["pairs"], state["given"]):
+            to.copy_(given)   # the sort works in place: the pairs of this pass
+        swapped = rast.radix_sort(*state["pairs"], *state["scratch"], state["bits"])
+        keys, values = state["scratch"] if swapped else state["pairs"]
+        return {"keys": keys, "values": values}
+    if kind == "train":
+        colour = autograd.rasterize(*state["params"], rast, state["camera"], state["settings"])
+        grads = torch.autograd.grad(colour, state["params"], state["grads"][0])
+        return {"colour": colour.detach(), **dict(zip(PARAMS, grads))}
+    if kind == "train_views":
+        colours = autograd.rasterize_views(*state["params"], rast, state["cameras"], state["sizes"], state["settings"])
+        grads = torch.autograd.grad(colours, state["params"], state["grads"])
+        return {"colours": [c.detach() for c in colours], **dict(zip(PARAMS, grads))}
+    if kind == "views":
+        st = rast.render_views(state["views"], state["instances"], state["settings"])
+        return {"colour": state["colour"], "depth": state["depth"], **_stats(st)}
+    t = state["targets"]
+    if kind == "composite":
+        st = rast.render(state["camera"], state["instances"], state["settings"], t, state["points"], state["under"])
+    elif kind == "lod":
+        drawn, cut = rast.lod_select(state["camera"], state["lod"], state["pixels"], state["settings"])
+        st = rast.render(state["camera"], drawn, state["settings"], t)
+        return {"colour": t.colour, "depth": t.depth, "splats": cut[0].splats, "merged": cut[0].merged, **_stats(st)}
+    else:
+        st = rast.render(state["camera"], state["instances"], state["settings"], t)
+    return {"colour": t.colour, "depth": t.depth, **_stats(st)}
+
+
+def work(case):
+    """Inputs read once and outputs written once; the projection's and the harmonics' arithmetic a splat, and
+    the arithmetic of a few dozen splats a pixel."""
+    kind = case["kind"]
+    if kind == "sort":
+        return {"bytes": 24.0 * case["pairs"], "flops": 0.0}
+    n, rest = case["splats"], REST[case["degree"]]
+    if kind in ("views", "train_views"):
+        sizes = [s for _, s in _sphere_views(case["views"])]
+    else:
+        sizes = [(case["width"], case["height"])]
+    pixels = sum(w * h for w, h in sizes)
+    flops = len(sizes) * n * (300.0 + 12.0 * rest) + pixels * 30 * 22.0
+    if kind in ("train", "train_views"):
+        floats = 3 + 3 + 4 + 1 + 3 * (1 + rest)
+        return {"bytes": 8.0 * floats * n + 32.0 * pixels, "flops": 3.0 * flops}
+    cloud = n * (32.0 + 4.0 * ((rest * 3 + 1) // 2) + (4.0 if case.get("filter3d") else 0.0))
+    if kind == "composite":
+        cloud += 24.0 * case["points"] + 20.0 * pixels
+    return {"bytes": cloud + 20.0 * pixels, "flops": flops}
+
+
+def tolerance(case):
+    """About four times what exact() is off by: a splat at its cutoff, at the 1/255 floor, at a pixel's last place or at
+    the threshold depth that falls the other way moves a pixel (and the gradients through it) by a whole contribution,
+    and with discs by a whole colour; everything else is 32-bit sums, 1e-6 and below. Seen: rel 5e-5 on a frame,
+    3e-3 where the depth is the threshold's, 4e-4 on views, 6e-4 and 3e-3 on the gradients of one view and of many
+    (sums of terms of either sign), 1.2e-3 with discs."""
+    kind = case["kind"]
+    if kind == "sort":
+        return "exact"
+    if kind == "frame" and case["depth_mode"] == 1:
+        return {"rel": 1.3e-2, "max": 0.99}
+    return {"frame": {"rel": 4e-4, "max": 0.3}, "lod": {"rel": 4e-4, "max": 0.3}, "views": {"rel": 1.6e-3, "max": 0.99},
+            "train": {"rel": 2.5e-3, "max": 0.8}, "train_views": {"rel": 1.2e-2, "max": 0.8},
+            "composite": {"rel": 5e-3, "max": 0.99}}[kind]
+
+
+# ---- the same in 64 bits -----------------------------------------------------
+
+def _camera_numbers(cam, width, height):
+    eye, target, up = (np.array(x, dtype=np.float64) for x in cam)
+    z = (eye - target) / np.linalg.norm(target - eye)
+    x = np.cross(up, z)
+    x /= np.linalg.norm(x)
+    y = np.cross(z, x)
+    rows = np.stack([x, y, -z])   # view space: x right, y up, z into the scene
+    m = np.concatenate([rows, -(rows @ eye)[:, None]], 1)
+    return dict(m=m, eye=eye, focal=_focal(width), width=width, height=height)
+
+
+def _harmonics(rest, d):
+    """The view-dependent colour of the rest coefficients [n, k, 3] in the directions d [n, 3]."""
+    x, y, z = d[:, 0], d[:, 1], d[:, 2]
+    b = []
+    if rest.shape[1] >= 3:
+        b += [-0.4886025119029199 * y, 0.4886025119029199 * z, -0.4886025119029199 * x]
+    if rest.shape[1] >= 8:
+        b += [1.0925484305920792 * x * y, -1.0925484305920792 * y * z,
+              0.31539156525252005 * (2 * z * z - x * x - y * y), -1.0925484305920792 * x * z,
+              0.5462742152960396 * (x * x - y * y)]
+    if rest.shape[1] >= 15:
+        b += [-0.5900435899266435 * y * (3 * x * x - y * y), 2.890611442640554 * x * y * z,
+              -0.4570457994644658 * y * (4 * z * z - x * x - y * y),
+              0.3731763325901154 * z * (2 * z * z - 3 * x * x - 3 * y * y),
+              -0.4570457994644658 * x * (4 * z * z - x * x - y * y), 1.445305721320277 * z * (x * x - y * y),
+              -0.5900435899266435 * x * (x * x - 3 * y * y)]
+    return sum(w[:, None] * rest[:, k] for k, w in enumerate(b)) if b else torch.zeros_like(d)
+
+
+def _depth_keys(cam, xyz32):
+    """The rasteriser's depth keys: bits 7..30 of the view depth as 32-bit sums give it."""
+    m = torch.tensor(cam["m"][2], dtype=torch.float32, device="cuda")
+    z = m[0] * xyz32[:, 0] + m[1] * xyz32[:, 1] + m[2] * xyz32[:, 2] + m[3]
+    return z.view(torch.int32).to(torch.int64) >> 7
+
+
+def _project(cam, s, opts):
+    """The footprints of the splats s (float64: xyz, scales, quats of any length, opacity, base, rest, filter3d or
+    None) in the camera: a dict of their screen values, and which of them are drawn."""
+    m = torch.tensor(cam["m"], device="cuda")
+    f, w, h = cam["focal"], cam["width"], cam["height"]
+    t = s["xyz"] @ m[:, :3].T + m[:, 3]
+    z = t[:, 2]
+    drawn = (z > NEAR) & (z <= FAR)
+    z = torch.where(drawn, z, torch.ones_like(z))
+    scales, opacity = s["scales"], s["opacity"]
+    if s["filter3d"] is not None:
+        wide = (scales ** 2 + s["filter3d"][:, None] ** 2).sqrt()
+        opacity = opacity * (scales / wide).prod(1)
+        scales = wide
+    q = s["quats"] / s["quats"].norm(dim=1, keepdim=True)
+    x, y, k, r = q.unbind(1)
+    rot = torch.stack([1 - 2 * (y * y + k * k), 2 * (x * y - r * k), 2 * (x * k + r * y),
+                       2 * (x * y + r * k), 1 - 2 * (x * x + k * k), 2 * (y * k - r * x),
+                       2 * (x * k - r * y), 2 * (y * k + r * x), 1 - 2 * (x * x + y * y)], 1).view(-1, 3, 3)
+    shape = rot * scales[:, None, :]
+    ux = (t[:, 0] / z).clamp((-0.15 * w - w / 2) / f, (1.15 * w - w / 2) / f)
+    uy = (t[:, 1] / z).clamp((-0.15 * h - h / 2) / f, (1.15 * h - h / 2) / f)
+    to_x = (m[0, :3] - ux[:, None] * m[2, :3]) * (f / z)[:, None]
+    to_y = (m[1, :3] - uy[:, None] * m[2, :3]) * (f / z)[:, None]
+    ax, ay = (to_x[:, :, None] * shape).sum(1), (to_y[:, :, None] * shape).sum(1)
+    a, b, c = (ax * ax).sum(1), (ax * ay).sum(1), (ay * ay).sum(1)
+    before = a * c - b * b
+    a, c = a + opts["dilation"], c + opts["dilation"]
+    det = a * c - b * b
+    drawn = drawn & (det > 1e-12)
+    alpha = opacity
+    if opts["antialias"]:
+        alpha = alpha * (before.clamp(min=1e-300) / det).sqrt()
+    drawn = drawn & (alpha >= 1.0 / 255.0)
+    cutoff = (2.0 * (255.0 * alpha.detach()).clamp(min=1.0001).log()).clamp(max=9.0)
+    cx, cy = f * t[:, 0] / z + w / 2, f * t[:, 1] / z + h / 2
+    ex, ey = (cutoff * a.detach()).sqrt(), (cutoff * c.detach()).sqrt()
+    drawn = drawn & (cx + ex >= 0) & (cy + ey >= 0) & (cx - ex < w) & (cy - ey < h)
+    away = s["xyz"] - torch.tensor(cam["eye"], device="cuda")
+    rgb = (s["base"] + _harmonics(s["rest"], away / away.norm(dim=1, keepdim=True))).clamp(min=0.0)
+    v = dict(cx=cx, cy=cy, ca=c / det, cb=-b / det, cc=a / det, alpha=alpha, z=z, rgb=rgb)
+    fixed = dict(cutoff=cutoff, ex=ex, ey=ey, disc=torch.zeros_like(cx))
+    return v, fixed, drawn.nonzero()[:, 0]
+
+
+def _tile_lists(fixed, v, keys, w, h):
+    """Each 16-pixel tile's splats in (key, index) order: (splats, first, count)."""
+    def tile(x, most):
+        return (x.clamp(0, most - 1).long() >> 4)
+
+    order = torch.sort(keys, stable=True)[1]
+    x0, x1 = tile((v["cx"] - fixed["ex"])[order], w), tile((v["cx"] + fixed["ex"])[order], w)
+    y0, y1 = tile((v["cy"] - fixed["ey"])[order], h), tile((v["cy"] + fixed["ey"])[order], h)
+    wide = x1 - x0 + 1
+    area = wide * (y1 - y0 + 1)
+    owner = torch.repeat_interleave(torch.arange(len(order), device="cuda"), area)
+    k = torch.arange(len(owner), device="cuda") - (area.cumsum(0) - area)[owner]
+    tiles_x, tiles_y = (w + 15) // 16, (h + 15) // 16
+    at = (y0[owner] + k // wide[owner]) * tiles_x + x0[owner] + k % wide[owner]
+    at, by_tile = torch.sort(at, stable=True)
+    count = torch.bincount(at, minlength=tiles_x * tiles_y)
+    return order[owner[by_tile]], count.cumsum(0) - count, count
+
+
+def _linear(c):
+    return torch.where(c <= 0.04045, c / 12.92, ((c.clamp(min=0.04) + 0.055) / 1.055) ** 2.4)
+
+
+def _chunks(lists, w, h):
+    """The tiles in groups of like length: (tile indices, the splats of each [tiles, longest], a place past the last
+    for none), at most about 24 million (pixel, splat) places a group."""
+    splats, first, count = lists
+    order = torch.argsort(count)
+    lengths = count[order].tolist()
+    at = 0
+    while at < len(lengths):
+        n = 1
+        while at + n < len(lengths) and (n + 1) * 256 * max(lengths[at + n], 1) <= 24_000_000:
+            n += 1
+        tiles = order[at:at + n]
+        longest = max(lengths[at + n - 1], 1)
+        k = torch.arange(longest, device="cuda")
+        inside = k < count[tiles][:, None]
+        if len(splats):
+            listed_ = splats[(first[tiles][:, None] + k).clamp(max=len(splats) - 1)]
+            yield tiles, torch.where(inside, listed_, torch.full_like(listed_, -1))
+        else:
+            yield tiles, torch.full((n, longest), -1, dtype=torch.int64, device="cuda")
+        at += n
+
+
+def _blend(v, fixed, tiles, idx, w, h, opts, under):
+    """The finished pixels of the tiles: (pixel indices, -1 past the frame [t, 256]; colour [t, 256, 4]; depth [t, 256])."""
+    tiles_x = (w + 15) // 16
+    p = torch.arange(256, device="cuda")
+    px, py = (tiles % tiles_x * 16)[:, None] + p % 16, (tiles // tiles_x * 16)[:, None] + p // 16
+    at = torch.where((px < w) & (py < h), py * w + px, torch.full_like(px, -1))
+
+    def of(x):
+        return x[idx.clamp(min=0)][:, None, :]
+
+    dx, dy = px[:, :, None] + 0.5 - of(v["cx"]), py[:, :, None] + 0.5 - of(v["cy"])
+    power = of(v["ca"]) * dx * dx + 2 * of(v["cb"]) * dx * dy + of(v["cc"]) * dy * dy
+    reach = (power <= of(fixed["cutoff"])) & (idx >= 0)[:, None, :]
+    disc = of(fixed["disc"]) > 0
+    alpha = (of(v["alpha"]) * torch.exp(-0.5 * power)).clamp(max=0.99)
+    alpha = torch.where(reach & (alpha >= 1.0 / 255.0) & ~disc, alpha, torch.zeros_like(alpha))
+    after = torch.cumprod(1.0 - alpha, 2)
+    ahead = torch.cat([torch.ones_like(after[:, :, :1]), after[:, :, :-1]], 2)
+    live = ahead >= 1e-4
+    z = torch.where(idx >= 0, v["z"][idx.clamp(min=0)], torch.zeros_like(idx, dtype=torch.float64))
+    hit = None
+    if under is not None:
+        discs = (disc & reach).long()
+        under_z = under["depth"].view(-1)[at.clamp(min=0)]
+        reached = torch.cummax(z.detach(), 1)[0][:, None, :] >= under_z[:, :, None]
+        live = live & (torch.cumsum(discs, 2) == discs) & ~(reached & (under_z > 0)[:, :, None])
+        hit = (discs.bool() & live).double()
+    weight = ahead * alpha * live
+    rgb = torch.bmm(weight, v["rgb"][idx.clamp(min=0)])
+    coverage = weight.sum(2)
+    t = 1.0 - coverage
+    if opts["linearise"]:
+        safe = coverage.clamp(min=1e-6)[:, :, None]
+        rgb = torch.where(coverage[:, :, None] > 1e-6, _linear(rgb / safe) * safe, rgb)
+    depth_sum = torch.bmm(weight, z[:, :, None])[:, :, 0].detach()
+    behind = torch.full_like(rgb[:, :, :1], opts["background"]).expand(-1, -1, 4)
+    total = coverage
+    if under is not None:
+        opaque = hit.sum(2) > 0
+        o_rgb = torch.bmm(hit, v["rgb"][idx.clamp(min=0)])
+        disc_behind = torch.cat([o_rgb, torch.ones_like(o_rgb[:, :, :1])], 2)
+        lower = under["colour"].view(-1, 4)[at.clamp(min=0)]
+        has_under = ~opaque & (under_z > 0)
+        behind = torch.where(opaque[:, :, None], disc_behind, torch.where(has_under[:, :, None], lower, behind))
+        back_z = torch.where(opaque, torch.bmm(hit, z[:, :, None])[:, :, 0], under_z)
+        depth_sum = torch.where(opaque | has_under, depth_sum + t * back_z, depth_sum)
+        total = torch.where(opaque | has_under, torch.ones_like(total), total)
+    colour = torch.cat([rgb + t[:, :, None] * behind[:, :, :3], (coverage + t * behind[:, :, 3])[:, :, None]], 2)
+    if opts["depth_mode"] == 0:
+        depth = torch.where(total > 1e-6, depth_sum / total.detach().clamp(min=1e-6), torch.zeros_like(t))
+    else:
+        past = (torch.cumsum(weight.detach(), 2) >= 0.5)
+        depth = torch.where(past[:, :, -1], z.gather(1, past.long().argmax(2)), torch.zeros_like(t))
+    return at, colour, depth.detach()
+
+
+def _render(cam, s, xyz32, opts, grad=None, discs=None, under=None):
+    """A frame in float64: (colour, depth). With grad, the dL/d(colour) image is taken back into s's leaves."""
+    w, h = cam["width"], cam["height"]
+    v, fixed, drawn = _project(cam, s, opts)
+    keys = _depth_keys(cam, xyz32)[drawn]
+    v, fixed = {k: x[drawn] for k, x in v.items()}, {k: x[drawn] for k, x in fixed.items()}
+    if discs is not None:
+        # Two-pixel discs: radius 1, no falloff.
+        m = torch.tensor(cam["m"], device="cuda")
+        t = discs["xyz"].double() @ m[:, :3].T + m[:, 3]
+        dz = t[:, 2]
+        cx, cy = cam["focal"] * t[:, 0] / dz + w / 2, cam["focal"] * t[:, 1] / dz + h / 2
+        ok = (dz > NEAR) & (dz <= FAR) & (cx >= -1) & (cy >= -1) & (cx < w + 1) & (cy < h + 1)
+        one = torch.ones_like(dz[ok])
+        more = dict(cx=cx[ok], cy=cy[ok], ca=one, cb=0 * one, cc=one, alpha=one, z=dz[ok], rgb=discs["rgb"][ok])
+        v = {k: torch.cat([x, more[k]]) for k, x in v.items()}
+        fixed = {k: torch.cat([x, one]) for k, x in fixed.items()}
+        keys = torch.cat([keys, _depth_keys(cam, discs["xyz"])[ok]])
+    flat = {k: x.detach().requires_grad_(grad is not None) for k, x in v.items()}
+    with torch.no_grad():
+        lists = _tile_lists(fixed, v, keys, w, h)
+    colour = torch.zeros((h * w, 4), dtype=torch.float64, device="cuda")
+    depth = torch.zeros((h * w,), dtype=torch.float64, device="cuda")
+    for tiles, idx in _chunks(lists, w, h):
+        with torch.set_grad_enabled(grad is not None):
+            at, c, d = _blend(flat, fixed, tiles, idx, w, h, opts, under)
+            inside = at >= 0
+            if grad is not None:
+                (c[inside] * grad.reshape(-1, 4)[at[inside]].double()).sum().backward()
+        colour[at[inside]], depth[at[inside]] = c[inside].detach(), d[inside]
+    if grad is not None:
+        kept = [k for k in v if v[k].requires_grad and flat[k].grad is not None]
+        torch.autograd.backward([v[k] for k in kept], [flat[k].grad for k in kept])
+    return colour.view(h, w, 4), depth.view(h, w)
+
+
+def _unpack(positions, shape, sh, filter3d):
+    """The float64 values that a packed cloud holds."""
+    halves = shape[:, 1:].contiguous().view(torch.float16).double()
+    word = shape[:, 0].long() & 0xFFFFFFFF
+    ten = torch.stack([(word >> 22) & 1023, (word >> 12) & 1023, (word >> 2) & 1023], 1).double()
+    small = (ten / 1023.0 * 2.0 - 1.0) * float(np.float32(0.70710678))
+    rest = (1.0 - (small ** 2).sum(1, keepdim=True)).clamp(min=0.0).sqrt()
+    four = torch.cat([rest, small], 1)
+    place = torch.tensor([[0, 1, 2, 3], [1, 0, 2, 3], [1, 2, 0, 3], [1, 2, 3, 0]], device="cuda")[word & 3]
+    n = positions.shape[0]
+    if sh is None:
+        coefficients = torch.zeros((n, 0, 3), dtype=torch.float64, device="cuda")
+    else:
+        k = sh.shape[1] * 2 // 3
+        coefficients = sh.view(torch.float16)[:, :k * 3].double().view(n, k, 3)
+    return dict(xyz=positions[:, :3].double(), opacity=positions[:, 3].double(), scales=halves[:, :3].exp(),
+                quats=four.gather(1, place), base=halves[:, 3:], rest=coefficients,
+                filter3d=None if filter3d is None else filter3d.double())
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind in ("sort", "lod") or case.get("scene") == "stress":
+        return None   # whole numbers; a merged cloud of its own; too many pairs
+    v = _values(case, seed)
+    opts = dict(dilation=case.get("dilation", 0.3), antialias=case.get("antialias", True),
+                linearise=case.get("linearise", True), depth_mode=case.get("depth_mode", 0),
+                background=case.get("background", 0.0))
+    if kind in ("train", "train_views"):
+        c = v["cloud"]
+        xyz32 = c["xyz"]
+        sh = torch.cat([((c["base"] - 0.5) / SH_C0)[:, None, :], c["rest"]], 1)
+        params = [p.double().requires_grad_() for p in (xyz32, c["log_scales"], c["quats"], c["logits"], sh)]
+        if kind == "train":
+            views = [(_scene_camera(case["scene"], 20.0), (case["width"], case["height"]))]
+        else:
+            views = _sphere_views(case["views"])
+        colours = []
+        for (cam, (w, h)), grad in zip(views, v["grads"]):
+            s = dict(xyz=params[0], scales=params[1].exp(), quats=params[2], opacity=torch.sigmoid(params[3]),
+                     base=0.5 + SH_C0 * params[4][:, 0], rest=params[4][:, 1:], filter3d=None)
+            colours.append(_render(_camera_numbers(cam, w, h), s, xyz32, opts, grad=grad)[0])
+        out = {"colour": colours[0]} if kind == "train" else {"colours": colours}
+        return {**out, **{k: p.grad for k, p in zip(PARAMS, params)}}
+    f3 = None
+    if case.get("filter3d"):
+        f3 = _filter3d(v["cloud"]["xyz"], _filter_cameras(case), case["width"])
+    s = _unpack(*_pack(v["cloud"]), f3)
+    xyz32 = v["cloud"]["xyz"]
+    counts = {"visible": None, "pairs": None}
+    with torch.no_grad():
+        if kind == "views":
+            images = [_render(_camera_numbers(cam, w, h), s, xyz32, opts) for cam, (w, h) in _sphere_views(case["views"])]
+            return {"colour": torch.cat([c.view(-1, 4) for c, _ in images]),
+                    "depth": torch.cat([d.view(-1) for _, d in images]), **counts}
+        discs = under = None
+        cam = _scene_camera(case.get("scene", "clusters"), 20.0)
+        if kind == "composite":
+            discs = dict(xyz=v["points"], rgb=v["point_rgb"].half().double())
+            under = dict(colour=v["under_colour"].double(), depth=v["under_depth"].double())
+        c, d = _render(_camera_numbers(cam, case["width"], case["height"]), s, xyz32, opts, discs=discs, under=under)
+        return {"colour": c, "depth": d, **counts}
