@@ -673,7 +673,9 @@ bool sortPairs(uint64_t* keys, uint32_t* values, uint64_t* keysAlt, uint32_t* va
                uint32_t bitLo, uint32_t keyBits, const SortWorkspace& ws, hipStream_t stream,
                hipEvent_t afterHistogram, const uint32_t* nDevice, TileDepthLayout depth, uint32_t* alsoZero,
                uint64_t alsoZeroWords, uint32_t radixBits) {
-    if ((nDevice == nullptr && n < 2) || n == 0 || keyBits == 0) {
+    // One pair is sorted as it is, but a sort that narrows still has to leave a u32 key.
+    const bool sorted = nDevice == nullptr && n < 2 && !sortNarrows(mode, keyBits, radixBits);
+    if (sorted || n == 0 || keyBits == 0) {
         if (alsoZero != nullptr) fill32(alsoZero, 0u, alsoZeroWords, stream);
         if (afterHistogram != nullptr) (void)hipEventRecord(afterHistogram, stream);
         return false;

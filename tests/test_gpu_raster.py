@@ -397,3 +397,23 @@ def test_every_half_pattern_decodes_as_the_oracle_does(rast):
     gpu = H.run_gpu(cam, s, inst, rast)
     ora = H.run_oracle(cam, s, inst)
     H.assert_bit_exact(gpu, ora)
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+def test_a_frame_of_one_pair_draws_it(rast, tile):
+    """One splat inside one tile: the sort has nothing to order, but its key is
+    still the narrowed one the ranges read."""
+    fields = np.zeros((1, 14), np.float32)
+    fields[0, :4] = (0.2, 0.2, 0.0, 0.9)
+    fields[0, 4:7] = -3.3
+    fields[0, 10] = 1.0
+    fields[0, 11:14] = (0.9, 0.5, 0.2)
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=60.0)
+    s = raster.RenderSettings(width=32, height=32, tile_size=tile)
+    inst = [(scenes.pack_splats(fields, 0), np.eye(4), raster.SplatEdit())]
+    gpu = H.run_gpu(cam, s, inst, rast)
+    ora = H.run_oracle(cam, s, inst)
+    assert ora["pairs"] == 1
+    H.assert_bit_exact(gpu, ora)
+    assert ora["colour"].max() > 0.1
+    np.testing.assert_allclose(gpu["colour"], ora["colour"], rtol=0, atol=2e-5)
