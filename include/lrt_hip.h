@@ -133,8 +133,9 @@ typedef struct {
     int32_t time_stages;          /* per-stage HIP event timing into lrt_frame_stats */
     float dilation;               /* 0.3 reproduces the reference */
     int32_t filter3d;             /* 1: read lrt_splats.filter3d */
-    uint32_t blend_batch;         /* records each 8x8 quadrant's LDS list holds: 64, 128 or 256 (0, the
-                                     default: 256; other values take the next of those up, 256 at most) */
+    uint32_t blend_batch;         /* 64, 128 or 256 (0, the default: 256): once the length of each
+                                     quadrant's list; accepted, and without effect since a block's
+                                     quadrants stage a round of a pair a lane together */
     int32_t tile_order;           /* 0: tile index order; 1 (default): heaviest tiles launched first */
     int32_t persistent_blend;     /* batches: 1 = a persistent blend taking quadrants from a queue */
     int32_t use_graph;            /* batches: 1 = capture the launch sequence once and replay it */
@@ -366,8 +367,7 @@ lrt_status lrt_raster_render_views(lrt_context* ctx, const lrt_view* views, uint
                                    const lrt_render_settings* settings, lrt_frame_stats* stats);
 
 /* The autotuner: times the batch under each launch choice this build offers
- * (tile size 8/16/32, list length 64/128/256, grid or persistent blend, graph
- * replay or not), then the sort's digit width (8/9/10 bits) under the fastest,
+ * (tile size 8/16/32, grid or persistent blend, graph replay or not), then the sort's digit width (8/9/10 bits) under the fastest,
  * and writes the winner into *settings (its other fields are kept). ms (host,
  * may be NULL) receives the winner's batch time. */
 lrt_status lrt_autotune_views(lrt_context* ctx, const lrt_view* views, uint32_t view_count,

@@ -1,36 +1,47 @@
-// Blend: one wave64 workgroup per 8x8 quadrant of a tile (a 16x16 tile has
-// four, an 8x8 one, a 32x32 sixteen), one lane per pixel. The wave walks its
-// tile's sorted pairs front to back in rounds of 128 (64 for 64-record lists):
-//   1. each lane takes two pairs of the round (one for 64-record lists; their
-//      records gathered one round ahead, so the loads are in flight while the
-//      previous round is worked)
-//      and tests each against the quadrant's pixel-centre box with a
-//      conservative bound on the Gaussian's power (quadrantReach);
-//   2. the pairs that pass are compacted (ballot + popcount) into the wave's
-//      own LDS list, records and all, in pair order, until the list is full or
-//      the pairs run out;
-//   3. the wave walks the list kGroup records at a time with a branch-free body
-//      (a skipped pair contributes alpha 0, which changes nothing) and leaves
-//      once its 64 pixels are opaque.
-// A staged record carries its Gaussian's form expanded about the quadrant's
-// centre and scaled to the exponent's base 2, the cutoff folded in: a pixel at
-// (u, v) from the centre evaluates q = A u^2 + B u v + C v^2 + D u + E v + F
-// with five FMAs, passes the cutoff test when q >= 0, and has alpha =
-// min(0.99, o' 2^q), o' = opacity * 2^(cutoff scaled). q differs from the
-// direct form's scaled power by float rounding only (below 2e-4 on footprints
-// from a quarter pixel to 300 pixels wide, centres up to 3.5 sigma outside the
-// quadrant).
-// No wave ever waits for another: quadrants finish as soon as their own pixels
-// do, and a quadrant with few pairs frees its slot for the next. The
-// quadrants of one tile are blocks b, b + 8, b + 16, ..., which the dispatcher
-// deals to one XCD, so their gathers of the tile's records share that XCD's L2.
+// Blend: one workgroup per 16x16 block of a tile (a 16x16 tile is one, a 32x32
+// tile four; an 8x8 tile is a block of its own), one wave per 8x8 quadrant of
+// it, one lane per pixel. The workgroup walks its tile's sorted pairs front to
+// back in rounds of a pair a lane:
+//   1. each lane stages one pair (its record gathered a round ahead, so the
+//      load is in flight while the last round is walked): it tests the pair
+//      against each quadrant's pixel-centre box with a conservative bound on
+//      the Gaussian's power (quadrantReach), puts the record into the LDS and
+//      its place into the list of every quadrant it can reach (ballot +
+//      popcount), in pair order;
+//   2. after a barrier each wave walks its quadrant's list, four records a
+//      group, and leaves once its 64 pixels are opaque. Records and lists hold
+//      two rounds, so one barrier a round is enough.
+// A tile's four quadrants share one gather and one staging of its pairs. With a
+// wave of its own for each quadrant, each gathered and tested all of them: 27M
+// cache accesses a launch against 7.5M, and half of the vector instructions,
+// on 3M splats at 1920x1080.
+// A record's Gaussian is expanded about the quadrant's centre and scaled to the
+// exponent's base 2, log2(opacity / 0.99) added: at a pixel (u, v) from the
+// centre q = A u^2 + B u v + C v^2 + D u + E v + F, the pixel is inside the
+// cutoff and above the alpha floor when q >= qmin, and alpha / 0.99 = min(1,
+// 2^q), the exponential's own output clamp. q differs from the direct form's
+// scaled power by float rounding only (below 2e-4 on footprints from a quarter
+// pixel to 300 pixels wide, centres up to 3.5 sigma outside the quadrant).
+//
+// What bounds it: the walk, by vector and matrix issue (a group of four records
+// about 250 cycles of a SIMD; the f32 matrix products and the vector FMAs do
+// not overlap), and, where one tile holds many times the others' pairs, that
+// tile's serial chain (about 480 cycles a group when a wave has a SIMD to
+// itself). Form and colour sums on FMAs with the records read from the LDS by
+// broadcast took 96 LDS cycles a group for each of the CU's four SIMDs, more
+// than the arithmetic. Blend time, that form against this one: 3M clustered
+// splats at 1920x1080 225 against 178 us, 2M splats in 64 views 5.30 against
+// 4.43 ms, 1M opaque splats at 1571x877 91 against 78 us. Broadcasting the
+// records by DPP operands instead took 198 us on the first, 4.96 ms on the
+// second.
 //
 // Per pixel it is the reference's splatBlend walk (shaders/lrt/splat/
 // splat_blend.slang:23-108, splat-only entry :110-114): skip past the cutoff,
 // alpha = min(0.99, opacity * exp(-power / 2)), skip below 1/255, accumulate
 // with the transmittance, stop below 1e-4, then linearise rgb / coverage. The
 // Gaussian's exponent runs on the hardware exp2 and the quadratic form on
-// FMAs; both move the result by a few ulps, which the image tolerances cover.
+// matrix FMAs in f32; both move the result by a few ulps, which the image
+// tolerances cover.
 //
 // The composite walk (splatBlendComposite, :116-120) is the same kernel
 // instantiated with COMPOSITE: a disc record (colour.w 1) that reaches a pixel
@@ -38,7 +49,8 @@
 // depth above 0 ends its walk at the first pair of its tile at or behind that
 // depth. That first pair may be one the quadrant's list dropped, so each staged
 // record carries the largest view z of every pair up to it (a wave max-scan at
-// staging), and the walk tests that instead of the record's own z.
+// staging, the waves and rounds before added when it is walked), and the walk
+// tests that instead of the record's own z.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -53,6 +65,8 @@ using namespace lrt::dev;
 
 constexpr uint32_t kLanes = 64;          // one wave: an 8x8 quadrant
 constexpr uint32_t kGroup = 4;           // list records walked per step
+constexpr float kAlphaMax = 0.99f;       // a splat's alpha at most (splat_blend.slang:66)
+constexpr float kLog2AlphaMax = -0.01449956969511508876f;
 constexpr float kExpScale = -0.72134752044448170368f;   // -log2(e) / 2
 constexpr float kLog2Floor = -7.99435343685885793775f;   // log2(1 / 255): alpha's floor
 
@@ -123,12 +137,35 @@ __device__ __forceinline__ void finishComposite(const FrameParams& f, uint32_t a
     }
 }
 
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;   // no pair; a task that finishes its tile's pixels itself
+
 // One pair's projected record, or an empty one (cutoff -1) past the range.
 struct Staged {
     float4 screen;   // centre.xy, view z, cutoff
     float4 conic;    // a, b, c, alpha
     float4 col;      // rgb, 0
 };
+
+// Orders a wave's own LDS writes and reads: its lanes run together, so only
+// the compiler has to keep them in order.
+__device__ __forceinline__ void waveSync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Inclusive max-scan over the wave's lanes: within rows of sixteen by row
+// shifts, then row 0 into row 1 and row 2 into row 3 (row_bcast:15), then rows
+// 0-1 into rows 2-3 (row_bcast:31); a lane with no source reads the least.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float maxWith(float v) {
+    const int least = __float_as_int(-3.4e38f);
+    return __builtin_fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(least, __float_as_int(v), CTRL, ROWS, 0xF, false)));
+}
+__device__ __forceinline__ float waveMaxScan(float v) {
+    v = maxWith<0x111, 0xF>(v);   // row_shr:1, 2, 4, 8
+    v = maxWith<0x112, 0xF>(v);
+    v = maxWith<0x114, 0xF>(v);
+    v = maxWith<0x118, 0xF>(v);
+    v = maxWith<0x142, 0xA>(v);
+    return maxWith<0x143, 0xC>(v);
+}
 
 __device__ __forceinline__ Staged gather(const float4* __restrict__ proj, uint32_t slot, uint32_t slots) {
     Staged s{make_float4(0.0f, 0.0f, 0.0f, -1.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f),
@@ -142,16 +179,28 @@ __device__ __forceinline__ Staged gather(const float4* __restrict__ proj, uint32
     return s;
 }
 
-// A quadrant's LDS list: records that reach it, in pair order, padded to a
-// multiple of kGroup with empty records (q far below 0: never pass the test).
-// One per kernel, whichever walks it runs.
-template <uint32_t LIST>
-struct BlendList {
-    float4 geom[LIST + kGroup];     // A, B, C, D of the expanded form
-    float4 conic[LIST + kGroup];    // E, F less the cutoff, o', view z
-    // rgb, then bits of the pair's place in the tile's range + 1; composite:
-    // the largest view z of the tile's pairs up to this one, kept or not
-    float4 colour[LIST + kGroup];
+// A block's LDS: the workgroup's waves each take one 8x8 quadrant of its
+// block (four waves a 16x16 block; one wave an 8x8 one), and all of them stage
+// the block's pairs, a round of a pair a lane at a time, two rounds' worth so
+// that one barrier a round is enough (a wave may stage the next round while
+// another still walks this one).
+template <uint32_t WAVES, bool COMPOSITE>
+struct BlendShared {
+    static constexpr uint32_t kRound = WAVES * kLanes;
+    // The round's records, in pair order, the conic scaled to base 2:
+    float4 at[2][kRound];       // centre.xy, A, B
+    float4 shape[2][kRound];    // C, log2(opacity / kAlphaMax), the least q that passes, 1 for a disc
+    float4 colour[2][kRound];   // rgb, view z
+    // Composite: the largest view z of the record's wave's pairs up to it, kept or not, and each wave's.
+    float reach[2][COMPOSITE ? kRound : 1];
+    float most[2][WAVES];
+    // Quadrant q's records among those source wave w staged: lanes in order, and how many.
+    uint8_t list[2][WAVES][kRound];
+    uint32_t count[2][WAVES][WAVES];
+    uint32_t done[2][WAVES];    // the wave's pixels all stopped before this round
+    // A wave's own: the least q (and the reach) of the chunk it walks, four records a vector.
+    float4 qmin[WAVES][kLanes / 4];
+    float4 chunkReach[WAVES][COMPOSITE ? kLanes / 4 : 1];
 };
 
 // A pixel's walk so far: premultiplied rgb, transmittance, depth sum, the
@@ -169,85 +218,258 @@ struct WalkState {
 // kResume starts from *state (its active lanes) and leaves the state there.
 constexpr uint32_t kFinish = 0, kPartial = 1, kResume = 2;
 
-// A tile of side 2^tileShift holds 2^quadBits 8x8 quadrants (1, 4 or 16),
-// numbered row-major inside it.
-__device__ __forceinline__ uint32_t quadBits(uint32_t tileShift) { return 2u * (tileShift - 3u); }
-
-// The first pixel of quadrant `quadrant` of tile `tile` of the frame f.
-__device__ __forceinline__ uint2 quadrantOrigin(const FrameParams& f, uint32_t tile, uint32_t quadrant) {
-    const uint32_t side = f.tileShift - 3u;
-    return make_uint2(((tile % f.tilesX) << f.tileShift) + ((quadrant & ((1u << side) - 1u)) << 3),
-                      ((tile / f.tilesX) << f.tileShift) + ((quadrant >> side) << 3));
+// A tile of side 2^tileShift holds 2^quadBits 8x8 quadrants (1, 4 or 16) and
+// 2^blockBits blocks (of four quadrants, but an 8-pixel tile's one), numbered
+// row-major inside it.
+__host__ __device__ __forceinline__ uint32_t quadBits(uint32_t tileShift) { return 2u * (tileShift - 3u); }
+__host__ __device__ __forceinline__ uint32_t blockBits(uint32_t tileShift) {
+    return tileShift <= 4u ? 0u : 2u * (tileShift - 4u);
 }
 
-// Quadrant `quadrant` of tile `tile` of the frame f, walking the pairs
+// The first pixel of part `part` of tile `tile` of the frame f, its parts
+// 2^partShift pixels square.
+__device__ __forceinline__ uint2 partOrigin(const FrameParams& f, uint32_t tile, uint32_t part, uint32_t partShift) {
+    const uint32_t side = f.tileShift - partShift;
+    return make_uint2(((tile % f.tilesX) << f.tileShift) + ((part & ((1u << side) - 1u)) << partShift),
+                      ((tile / f.tilesX) << f.tileShift) + ((part >> side) << partShift));
+}
+
+using Vec4 = float __attribute__((ext_vector_type(4)));
+
+// A pixel's walk while it runs: accum holds rgb and the depth sum over
+// kAlphaMax (the weights it sums are T alpha / kAlphaMax). The pixel walks
+// while t >= kTMin; composite: a pixel that something behind stops leaves its
+// T in tStopped and t 0. lastIn, depthIn and opaqueIn: a record's place in the
+// chunk at hand (-1: none yet).
+struct WalkLane {
+    Vec4 accum;
+    float t, tStopped;
+    float depthT;   // the depth is found once T is at most this; below 0 once found
+    int32_t lastIn, depthIn, opaqueIn;
+};
+constexpr float kTMin = 1e-4f;
+// Waves a SIMD the register allocation leaves room for: at two and more the
+// matrix results stay in the vector registers (no copies from accumulators).
+constexpr uint32_t kWavesPerSimd = 4;
+
+// The form of records 4 G .. 4 G + 3 of sixteen at the lane's own pixel.
+//
+// Both of the walk's contractions run on the matrix cores, in f32, as sixteen
+// 4x4 blocks of four lanes a block (v_mfma_f32_4x4x1, one block's lanes of A
+// given to every block). The form: rows of records times columns of pixels,
+// six products of a coefficient and the pixel's monomial; lane l < 16 of
+// `form` holds record l's A .. F, block G's four lanes are records 4 G ..
+// 4 G + 3, and q[k] lands in the lane of its pixel. The colours: rows of
+// channels times columns of pixels, one product a record, summed into the
+// lane's own accum; lane l of `colour`: channel l & 3 of record l / 4. What
+// stays on the VALU is what is no contraction: the exponential, the tests and
+// T. A matrix product costs about 14 cycles of issue, as five FMAs, and does
+// the work of four (the form) or of four with their operands' LDS reads gone
+// (the colours): the LDS, not the FMAs, is what it relieves.
+template <uint32_t G>
+__device__ __forceinline__ Vec4 formOf(const float form[6], const float mono[5]) {
+    Vec4 q = {0.0f, 0.0f, 0.0f, 0.0f};
+    q = __builtin_amdgcn_mfma_f32_4x4x1f32(form[5], 1.0f, q, 4, G, 0);
+#pragma unroll
+    for (uint32_t m = 0; m < 5; ++m) q = __builtin_amdgcn_mfma_f32_4x4x1f32(form[4 - m], mono[4 - m], q, 4, G, 0);
+    return q;
+}
+
+// One record's colour into the pixel's sums.
+template <uint32_t R>
+__device__ __forceinline__ Vec4 addColour(float colour, float weight, Vec4 accum) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(colour, weight, accum, 4, R, 0);
+}
+
+// One group of kGroup records, 4 G .. 4 G + 3 of the sixteen at hand, with form
+// q. A wave's records are one serial chain through T, and a launch cannot end
+// before its longest tile's chain, so the chain is kept short: the four
+// weights are taken as if no pixel stopped among the first three records (a
+// product and an FMA a record on the chain), and a group in which one does is
+// taken again with the test between the records. Both ways do the same
+// arithmetic for a pixel that does not stop.
+template <uint32_t DEPTH_MODE, bool COMPOSITE, bool TRACK, uint32_t G>
+__device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, float4 qmin4, float4 reach4,
+                                          float stopZ, uint64_t discs, int32_t first) {
+    constexpr uint32_t R0 = G * kGroup;
+    const float qmin[4] = {qmin4.x, qmin4.y, qmin4.z, qmin4.w};
+    bool passes[4];   // inside the cutoff and above the alpha floor
+    float alpha[4];   // over kAlphaMax
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        passes[k] = q[k] >= qmin[k];
+        // min(1, alpha / kAlphaMax): the exponential's own output clamp
+        const float scaled = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(q[k]), 0.0f, 1.0f);
+        alpha[k] = passes[k] ? scaled : 0.0f;
+    }
+    float weight[4];
+    if constexpr (COMPOSITE) {
+        // A group with a disc, or that an under-layer ends in (padding has the
+        // least reach), goes record by record.
+        const float reach[4] = {reach4.x, reach4.y, reach4.z, reach4.w};
+        const float most = fmaxS(fmaxS(reach[0], reach[1]), fmaxS(reach[2], reach[3]));
+        const bool ends = (w.t >= kTMin) & (most >= stopZ);
+        const bool anyEnds = __ballot(ends) != 0;
+        if (((discs >> R0) & 15u) != 0u || anyEnds) {
+            const auto stop = [&](bool here) {
+                w.tStopped = here ? w.t : w.tStopped;
+                w.t = here ? 0.0f : w.t;
+            };
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                if (anyEnds) stop((w.t >= kTMin) & (reach[k] >= stopZ));
+                const bool ok = (w.t >= kTMin) & passes[k];
+                weight[k] = 0.0f;
+                if (((discs >> (R0 + k)) & 1u) != 0u) {   // uniform: a disc that reaches the pixel ends its walk
+                    w.opaqueIn = ok ? first + static_cast<int32_t>(R0 + k) : w.opaqueIn;
+                    stop(ok);
+                } else {
+                    weight[k] = w.t * (ok ? alpha[k] : 0.0f);
+                    w.t = __builtin_fmaf(-kAlphaMax, weight[k], w.t);
+                    if constexpr (DEPTH_MODE == 1) {
+                        const bool at = ok & (w.t <= w.depthT);
+                        w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
+                        w.depthT = at ? -1.0f : w.depthT;
+                    }
+                }
+            }
+            w.accum = addColour<R0>(colour, weight[0], w.accum);
+            w.accum = addColour<R0 + 1>(colour, weight[1], w.accum);
+            w.accum = addColour<R0 + 2>(colour, weight[2], w.accum);
+            w.accum = addColour<R0 + 3>(colour, weight[3], w.accum);
+            return;
+        }
+    }
+    const bool walks = w.t >= kTMin;
+    float t[5];
+    t[0] = walks ? w.t : 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        weight[k] = t[k] * alpha[k];
+        t[k + 1] = __builtin_fmaf(-kAlphaMax, weight[k], t[k]);   // T (1 - alpha)
+    }
+    bool ok[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) ok[k] = walks & passes[k];
+    if (__ballot(walks & (t[3] < kTMin)) != 0) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const bool here = t[k] >= kTMin;
+            ok[k] = here & passes[k];
+            weight[k] = t[k] * (here ? alpha[k] : 0.0f);
+            t[k + 1] = __builtin_fmaf(-kAlphaMax, weight[k], t[k]);
+        }
+    }
+    w.accum = addColour<R0>(colour, weight[0], w.accum);
+    w.accum = addColour<R0 + 1>(colour, weight[1], w.accum);
+    w.accum = addColour<R0 + 2>(colour, weight[2], w.accum);
+    w.accum = addColour<R0 + 3>(colour, weight[3], w.accum);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        if constexpr (TRACK) w.lastIn = ok[k] ? first + static_cast<int32_t>(R0 + k) : w.lastIn;
+        if constexpr (DEPTH_MODE == 1) {
+            const bool at = ok[k] & (t[k + 1] <= w.depthT);
+            w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
+            w.depthT = at ? -1.0f : w.depthT;
+        }
+    }
+    w.t = walks ? t[4] : w.t;
+}
+
+// Up to sixteen records, whose forms lanes 0 .. 15 hold and whose colours
+// `colour` does (lane l: channel l & 3 of record l / 4), four a group in order,
+// while there are records and the wave has a pixel that walks; the next group's
+// form is computed while this one is blended. Returns the records walked.
+template <uint32_t DEPTH_MODE, bool COMPOSITE, bool TRACK>
+__device__ __forceinline__ uint32_t walkSixteen(WalkLane& w, uint32_t records, const float form[6], float colour,
+                                                const float mono[5], const float4* qmin, const float4* chunkReach,
+                                                float stopZ, uint64_t discs, int32_t first) {
+    uint32_t walked = 0;
+    Vec4 q = formOf<0>(form, mono);
+    const auto group = [&](auto g) -> bool {
+        constexpr uint32_t G = decltype(g)::value;
+        if (G * kGroup >= records) return false;
+        Vec4 next = q;
+        if constexpr (G + 1 < 16 / kGroup) next = formOf<G + 1>(form, mono);
+        float4 reach = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if constexpr (COMPOSITE) reach = chunkReach[G];
+        walkGroup<DEPTH_MODE, COMPOSITE, TRACK, G>(w, q, colour, qmin[G], reach, stopZ, discs, first);
+        q = next;
+        walked += kGroup;
+        return __ballot(w.t >= kTMin) != 0;
+    };
+    (void)(group(std::integral_constant<uint32_t, 0>{}) && group(std::integral_constant<uint32_t, 1>{}) &&
+           group(std::integral_constant<uint32_t, 2>{}) && group(std::integral_constant<uint32_t, 3>{}));
+    return walked;
+}
+
+// The block of WAVES quadrants whose first pixel is `origin`, walking the pairs
 // [range.x, range.y) of pairSlots (all of the tile's, or a segment of them;
 // places count from tileStart); colour and depth are the frame's images,
-// lastCount/finalT/accum its per-pixel state (each may be null).
-template <uint32_t DEPTH_MODE, uint32_t LIST, bool COMPOSITE, uint32_t MODE = kFinish, bool TRACK = true>
-__device__ __forceinline__ void blendQuadrant(BlendList<LIST>& list, const FrameParams& f, uint32_t tile,
-                                              uint32_t quadrant, uint2 range,
-                                              uint32_t tileStart, uint32_t slots,
-                                              const uint32_t* __restrict__ pairSlots,
-                                              const float4* __restrict__ proj,
-                                              const float4* __restrict__ underColour,
-                                              const float* __restrict__ underDepth, float4* __restrict__ colour,
-                                              float* __restrict__ depth, uint32_t* __restrict__ lastCount,
-                                              float* __restrict__ finalT, float4* __restrict__ accum,
-                                              WalkState* state = nullptr, float4* __restrict__ partialA = nullptr,
-                                              float2* __restrict__ partialB = nullptr,
-                                              uint32_t* __restrict__ walkSteps = nullptr,
-                                              const uint32_t* __restrict__ slotOfPair = nullptr) {
+// lastCount/finalT/accum its per-pixel state (each may be null). Every wave of
+// the workgroup calls it; a workgroup that calls it again has a barrier in
+// between (the LDS is the last call's until then).
+template <uint32_t DEPTH_MODE, uint32_t WAVES, bool COMPOSITE, uint32_t MODE = kFinish, bool TRACK = true>
+__device__ __forceinline__ void blendBlock(BlendShared<WAVES, COMPOSITE>& shared, const FrameParams& f, uint2 origin,
+                                           uint2 range, uint32_t tileStart, uint32_t slots,
+                                           const uint32_t* __restrict__ pairSlots, const float4* __restrict__ proj,
+                                           const float4* __restrict__ underColour,
+                                           const float* __restrict__ underDepth, float4* __restrict__ colour,
+                                           float* __restrict__ depth, uint32_t* __restrict__ lastCount,
+                                           float* __restrict__ finalT, float4* __restrict__ accum,
+                                           WalkState* state = nullptr, float4* __restrict__ partialA = nullptr,
+                                           float2* __restrict__ partialB = nullptr,
+                                           uint32_t* __restrict__ walkSteps = nullptr,
+                                           const uint32_t* __restrict__ slotOfPair = nullptr) {
     static_assert(!(COMPOSITE && MODE != kFinish), "a composite walk is not split");
-    // Pairs a lane stages a round: two, or one for a 64-record list.
-    constexpr uint32_t kPerLane = LIST >= 2 * kLanes ? 2u : 1u;
-    constexpr uint32_t kRound = kLanes * kPerLane;
-    static_assert(LIST % kRound == 0 && LIST >= kRound, "list length");
-    float4* const sGeom = list.geom;
-    float4* const sConic = list.conic;
-    float4* const sColour = list.colour;
-
-    const uint32_t lane = threadIdx.x;
-    const uint2 origin = quadrantOrigin(f, tile, quadrant);
-    const uint32_t x0 = origin.x, y0 = origin.y;
-    if (x0 >= f.width || y0 >= f.height) return;   // a quadrant past the frame's edge has no pixels
-    const uint32_t x1 = x0 + 8u < f.width ? x0 + 8u : f.width;
-    const uint32_t y1 = y0 + 8u < f.height ? y0 + 8u : f.height;
-    const uint32_t px = x0 + (lane & 7u);
-    const uint32_t py = y0 + (lane >> 3);
-    const bool inside = px < x1 && py < y1;
+    static_assert(WAVES == 1 || (WAVES == 4 && MODE == kFinish), "a quadrant, or the four of a 16x16 block");
+    constexpr uint32_t kRound = WAVES * kLanes;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = WAVES == 1 ? 0u : threadIdx.x >> 6;
+    // The block's quadrants: the pixel-centre box of each, empty past the frame's edge.
+    float boxLo[WAVES][2], boxHi[WAVES][2];
+    bool any[WAVES];
+#pragma unroll
+    for (uint32_t q = 0; q < WAVES; ++q) {
+        const uint32_t x0 = origin.x + (q & 1u) * 8u, y0 = origin.y + (q >> 1) * 8u;
+        any[q] = x0 < f.width && y0 < f.height;
+        boxLo[q][0] = static_cast<float>(x0) + 0.5f;
+        boxLo[q][1] = static_cast<float>(y0) + 0.5f;
+        boxHi[q][0] = static_cast<float>(x0 + 8u < f.width ? x0 + 8u : f.width) - 0.5f;
+        boxHi[q][1] = static_cast<float>(y0 + 8u < f.height ? y0 + 8u : f.height) - 0.5f;
+    }
+    const uint32_t px = origin.x + (wave & 1u) * 8u + (lane & 7u);
+    const uint32_t py = origin.y + (wave >> 1) * 8u + (lane >> 3);
+    const bool inside = px < f.width && py < f.height;
     // The pixel centre about the quadrant's centre, and that centre.
     const float pu = static_cast<float>(lane & 7u) - 3.5f;
     const float pv = static_cast<float>(lane >> 3) - 3.5f;
-    const float xm = static_cast<float>(x0) + 4.0f, ym = static_cast<float>(y0) + 4.0f;
-    const float boxLoX = static_cast<float>(x0) + 0.5f, boxLoY = static_cast<float>(y0) + 0.5f;
-    const float boxHiX = static_cast<float>(x1 - 1u) + 0.5f, boxHiY = static_cast<float>(y1 - 1u) + 0.5f;
+    const float xm = static_cast<float>(origin.x + (wave & 1u) * 8u) + 4.0f;
+    const float ym = static_cast<float>(origin.y + (wave >> 1) * 8u) + 4.0f;
     const uint64_t below = (1ull << lane) - 1ull;
 
-    // Round k's records sit in `staged` while round k + 1's are gathered.
-    // A training frame's sort carried pair indices: each pair's slot is read through it.
-    auto slotAt = [&](uint32_t at) -> uint32_t {
-        if (at >= range.y) return 0xFFFFFFFFu;
-        const uint32_t v = pairSlots[at];
-        return slotOfPair != nullptr ? slotOfPair[v] : v;
+    // A training frame's sort carried pair indices: each pair's slot is read
+    // through its index, a round ahead of its record.
+    const auto valueAt = [&](uint32_t at) -> uint32_t { return at < range.y ? pairSlots[at] : kNoSlot; };
+    const auto slotOf = [&](uint32_t v) -> uint32_t {
+        return slotOfPair != nullptr && v != kNoSlot ? slotOfPair[v] : v;
     };
-    Staged staged[kPerLane];
-#pragma unroll
-    for (uint32_t u = 0; u < kPerLane; ++u) staged[u] = gather(proj, slotAt(range.x + u * kLanes + lane), slots);
+    const uint32_t mine = range.x + threadIdx.x;
+    Staged staged = gather(proj, slotOf(valueAt(mine)), slots);
+    uint32_t slotNext = slotOf(valueAt(mine + kRound));   // the next round's slot
+    uint32_t valueNext = valueAt(mine + 2u * kRound);     // the value of the round after
 
-    float r = 0.0f, g = 0.0f, b = 0.0f, t = 1.0f, depthSum = 0.0f, depthAt = -1.0f;
+    WalkLane w{{0.0f, 0.0f, 0.0f, 0.0f}, inside ? 1.0f : 0.0f, -1.0f, 1.0f - f.depthThreshold, -1, -1, -1};
+    float depthAt = -1.0f;
     uint32_t last = 0;
-    bool active = inside;
     if constexpr (MODE == kResume) {
-        r = state->r;
-        g = state->g;
-        b = state->b;
-        t = state->t;
-        depthSum = state->depthSum;
+        w.accum = Vec4{state->r, state->g, state->b, state->depthSum} * (1.0f / kAlphaMax);
+        w.t = inside && state->active ? state->t : 0.0f;
         depthAt = state->depthAt;
+        w.depthT = depthAt < 0.0f ? w.depthT : -1.0f;
         last = state->last;
-        active = inside && state->active;
     }
+    const float mono[5] = {pu * pu, pu * pv, pv * pv, pu, pv};
     // Composite: what ends the walk from behind. A pixel with an under depth
     // above 0 stops at the first pair at or behind it (whether or not that pair
     // reaches the pixel: the reference tests the depth first), a disc that
@@ -258,142 +480,180 @@ __device__ __forceinline__ void blendQuadrant(BlendList<LIST>& list, const Frame
         if (underDepth != nullptr && inside) underZ = underDepth[at0];
     }
     const bool underHit = COMPOSITE && underZ > 0.0f;
+    const float stopZ = underHit ? underZ : __builtin_inff();   // no finite depth reaches it
     bool opaqueHit = false;
     float oR = 0.0f, oG = 0.0f, oB = 0.0f, oZ = 0.0f;
-    float zCarry = -3.4e38f;   // the largest view z of the pairs staged so far
+    float zCarry = -3.4e38f;   // the largest view z of the rounds before
     uint32_t walked = 0;       // list records walked (kGroup a step)
-    uint32_t next = range.x;   // the first pair of the round in `staged`
-    while (next < range.y) {
-        // 1-2. stage rounds into the list while a whole round still fits
-        uint32_t fill = 0;
-        while (next < range.y && fill + kRound <= LIST) {
-            Staged ahead[kPerLane];
+    bool walks = __ballot(w.t >= kTMin) != 0;
+    uint32_t buf = 0;
+    for (uint32_t next = range.x; next < range.y; next += kRound, buf ^= 1u) {
+        // 1. stage: each lane's record and which quadrants it can reach
+        const uint32_t at = next + threadIdx.x;
+        const uint32_t slot = wave * kLanes + lane;   // the record's place in the round
+        uint32_t mask = 0;
+        if (at < range.y) {
+            const Staged& s = staged;
+            const ReachConic rc = reachConic(s.conic.x, s.conic.y, s.conic.z);
 #pragma unroll
-            for (uint32_t u = 0; u < kPerLane; ++u) {
-                ahead[u] = gather(proj, slotAt(next + kRound + u * kLanes + lane), slots);
+            for (uint32_t q = 0; q < WAVES; ++q) {
+                const bool reach = quadrantReach(rc, s.screen.w, boxLo[q][0] - s.screen.x, boxLo[q][1] - s.screen.y,
+                                                 boxHi[q][0] - s.screen.x, boxHi[q][1] - s.screen.y);
+                mask |= any[q] && reach ? 1u << q : 0u;
             }
+        }
+        if constexpr (COMPOSITE) {
+            // inclusive max-scan of the wave's view z in pair order
+            const float zr = waveMaxScan(at < range.y ? staged.screen.z : -3.4e38f);
+            shared.reach[buf][slot] = zr;
+            if (lane == kLanes - 1u) shared.most[buf][wave] = zr;
+        }
+        if (mask != 0) {
+            const Staged& s = staged;
+            // q = the form plus log2(opacity / kAlphaMax): alpha / kAlphaMax = 2^q
+            // directly, and both tests (inside the cutoff, alpha >= 1/255) are
+            // q >= qmin. A disc (colour.w 1, opacity 1) has the cutoff alone.
+            const bool disc = COMPOSITE && s.col.w > 0.5f;
+            const float logOpacity = __builtin_amdgcn_logf(s.conic.w) - kLog2AlphaMax;
+            const float cut = logOpacity + kExpScale * s.screen.w;
+            shared.at[buf][slot] = make_float4(s.screen.x, s.screen.y, kExpScale * s.conic.x,
+                                               kExpScale * (s.conic.y + s.conic.y));
+            shared.shape[buf][slot] = make_float4(kExpScale * s.conic.z, logOpacity,
+                                                  disc ? cut : fmaxS(cut, kLog2Floor - kLog2AlphaMax),
+                                                  disc ? 1.0f : 0.0f);
+            shared.colour[buf][slot] = make_float4(s.col.x, s.col.y, s.col.z, s.screen.z);
+        }
 #pragma unroll
-            for (uint32_t u = 0; u < kPerLane; ++u) {
-                const Staged& s = staged[u];
-                const uint32_t at = next + u * kLanes + lane;
-                const bool keep = at < range.y &&
-                                  quadrantReach(s.conic.x, s.conic.y, s.conic.z, s.screen.w, boxLoX - s.screen.x,
-                                                boxLoY - s.screen.y, boxHiX - s.screen.x, boxHiY - s.screen.y);
-                const uint64_t vote = __ballot(keep);
-                float zReach = 0.0f;
-                if constexpr (COMPOSITE) {
-                    // inclusive max-scan of the round's view z in pair order
-                    float zr = at < range.y ? s.screen.z : -3.4e38f;
-#pragma unroll
-                    for (uint32_t d = 1; d < kLanes; d <<= 1) {
-                        const float o = __shfl_up(zr, d, 64);
-                        zr = lane >= d ? fmaxS(zr, o) : zr;
-                    }
-                    zReach = fmaxS(zr, zCarry);
-                    zCarry = shflF(zReach, kLanes - 1);
-                }
-                if (keep) {
-                    const uint32_t to = fill + static_cast<uint32_t>(__popcll(vote & below));
-                    const float ux = s.screen.x - xm, vy = s.screen.y - ym;
-                    const float fa = kExpScale * s.conic.x, fb = kExpScale * (s.conic.y + s.conic.y);
-                    const float fc = kExpScale * s.conic.z;
-                    const float scaledCut = kExpScale * s.screen.w;
-                    const float fd = -(2.0f * fa * ux + fb * vy), fe = -(2.0f * fc * vy + fb * ux);
-                    const float fbase = ux * (fa * ux + fb * vy) + fc * vy * vy;
-                    sGeom[to] = make_float4(fa, fb, fc, fd);
-                    if constexpr (COMPOSITE) {
-                        // q = the form less the cutoff; alpha = o' 2^q. A disc
-                        // (colour.w 1) is marked by o' < 0: its alpha never passes.
-                        const bool disc = s.col.w > 0.5f;
-                        const float scaledOpacity = disc ? -1.0f : s.conic.w * __builtin_amdgcn_exp2f(scaledCut);
-                        sConic[to] = make_float4(fe, fbase - scaledCut, scaledOpacity, s.screen.z);
-                    } else {
-                        // q' = the form plus log2(opacity): alpha = 2^q' directly, and
-                        // both tests (inside the cutoff, alpha >= 1/255) are q' >= qmin
-                        const float logOpacity = __builtin_amdgcn_logf(s.conic.w);
-                        const float qmin = fmaxS(logOpacity + scaledCut, kLog2Floor);
-                        sConic[to] = make_float4(fe, fbase + logOpacity, qmin, s.screen.z);
-                    }
-                    sColour[to] = make_float4(s.col.x, s.col.y, s.col.z,
-                                              COMPOSITE ? zReach : __uint_as_float(at - tileStart + 1u));
-                }
-                fill += static_cast<uint32_t>(__popcll(vote));
+        for (uint32_t q = 0; q < WAVES; ++q) {
+            const uint64_t vote = __ballot((mask >> q) & 1u);
+            if ((mask >> q) & 1u) {
+                shared.list[buf][q][wave * kLanes + static_cast<uint32_t>(__popcll(vote & below))] =
+                    static_cast<uint8_t>(lane);
             }
-#pragma unroll
-            for (uint32_t u = 0; u < kPerLane; ++u) staged[u] = ahead[u];
-            next += kRound;
+            if (lane == q) shared.count[buf][q][wave] = static_cast<uint32_t>(__popcll(vote));
         }
-        const uint32_t padded = (fill + kGroup - 1u) & ~(kGroup - 1u);
-        if (lane < padded - fill) {
-            sGeom[fill + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            sConic[fill + lane] = make_float4(0.0f, -1e30f, 0.0f, 0.0f);   // q far below any threshold: never passes
-            sColour[fill + lane] = make_float4(0.0f, 0.0f, 0.0f, COMPOSITE ? -3.4e38f : 0.0f);
-        }
+        if (lane == 0) shared.done[buf][wave] = walks ? 0u : 1u;
+        // 2. the next round's record, the slot of the one after and the value after that
+        staged = gather(proj, slotNext, slots);
+        slotNext = slotOf(valueNext);
+        valueNext = valueAt(at + 3u * kRound);
         __syncthreads();
-        // 3. walk the list: all kGroup records' reads issued together, then the
-        // pixels blend them in order
-        for (uint32_t j = 0; j < padded; j += kGroup) {
-            walked += kGroup;
-            float4 g0[kGroup], g1[kGroup], g2[kGroup];
+        if constexpr (WAVES > 1) {
+            // Written before the barrier, read after it, written again only two
+            // rounds on: every wave reads the same.
+            uint32_t stopped = 1;
 #pragma unroll
-            for (uint32_t k = 0; k < kGroup; ++k) {
-                g0[k] = sGeom[j + k];
-                g1[k] = sConic[j + k];
-                g2[k] = sColour[j + k];
-                // the place is needed only when the pair contributes; without
-                // this the compiler loads it behind a branch in the walk
-                asm volatile("" ::"v"(g2[k].w));
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kGroup; ++k) {
-                if constexpr (COMPOSITE) active = active & !(underHit & (g2[k].w >= underZ));
-                const float q = __builtin_fmaf(pu, __builtin_fmaf(g0[k].x, pu, __builtin_fmaf(g0[k].y, pv, g0[k].w)),
-                                               __builtin_fmaf(pv, __builtin_fmaf(g0[k].z, pv, g1[k].x), g1[k].y));
-                float alpha;
-                bool ok;   // bitwise, not short-circuit: no branch inside the walk
-                if constexpr (COMPOSITE) {
-                    alpha = __builtin_fminf(0.99f, g1[k].z * __builtin_amdgcn_exp2f(q));
-                    ok = active & (q >= 0.0f) & (alpha >= 1.0f / 255.0f);
-                } else {
-                    alpha = __builtin_fminf(0.99f, __builtin_amdgcn_exp2f(q));
-                    ok = active & (q >= g1[k].z);
-                }
-                const float a = ok ? alpha : 0.0f;
-                const float weight = t * a;
-                r = __builtin_fmaf(weight, g2[k].x, r);
-                g = __builtin_fmaf(weight, g2[k].y, g);
-                b = __builtin_fmaf(weight, g2[k].z, b);
-                depthSum = __builtin_fmaf(weight, g1[k].w, depthSum);
-                t = t - weight;   // T (1 - alpha)
-                if constexpr (!COMPOSITE && TRACK) last = ok ? __float_as_uint(g2[k].w) : last;
-                if constexpr (DEPTH_MODE == 1) {
-                    depthAt = (ok && depthAt < 0.0f && 1.0f - t >= f.depthThreshold) ? g1[k].w : depthAt;
-                }
-                if constexpr (COMPOSITE) {
-                    const bool hit = active & (q >= 0.0f) & (g1[k].z < 0.0f);
-                    oR = hit ? g2[k].x : oR;
-                    oG = hit ? g2[k].y : oG;
-                    oB = hit ? g2[k].z : oB;
-                    oZ = hit ? g1[k].w : oZ;
-                    opaqueHit = opaqueHit | hit;
-                    active = active & !hit;
-                }
-                active = active && !(t < 1e-4f);
-            }
-            if (__ballot(active) == 0) break;
+            for (uint32_t q = 0; q < WAVES; ++q) stopped &= shared.done[buf][q];
+            if (stopped != 0) break;
         }
-        if (__ballot(active) == 0) break;
-        __syncthreads();   // the list is refilled next
+        float before[WAVES];   // composite: the largest view z ahead of each source wave's pairs
+        if constexpr (COMPOSITE) {
+#pragma unroll
+            for (uint32_t q = 0; q < WAVES; ++q) {
+                before[q] = zCarry;
+                zCarry = fmaxS(zCarry, shared.most[buf][q]);
+            }
+        }
+        if (!walks) {
+            if constexpr (WAVES == 1) break;
+            continue;
+        }
+        // 3. walk this quadrant's records, 64 a chunk: their coefficients and
+        // colours a record a lane, for the matrix cores to hand round
+        uint32_t start[WAVES + 1];
+        start[0] = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < WAVES; ++q) {
+            start[q + 1] = start[q] + static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+                                          static_cast<int>(shared.count[buf][wave][q])));
+        }
+        const uint32_t total = start[WAVES];
+        for (uint32_t chunk = 0; chunk < total; chunk += kLanes) {
+            const uint32_t k = chunk + lane;
+            const bool real = k < total;
+            const uint32_t kk = real ? k : total - 1u;
+            uint32_t from = 0, first = 0;
+#pragma unroll
+            for (uint32_t q = 1; q < WAVES; ++q) {
+                from = kk >= start[q] ? q : from;
+                first = kk >= start[q] ? start[q] : first;
+            }
+            const uint32_t record = from * kLanes + shared.list[buf][wave][from * kLanes + (kk - first)];
+            const float4 g0 = shared.at[buf][record];
+            const float4 g1 = shared.shape[buf][record];
+            // The form about the quadrant's centre; past the list, one that passes nothing.
+            const float ux = g0.x - xm, vy = g0.y - ym;
+            const float fa = g0.z, fb = g0.w, fc = g1.x;
+            const float fd = -(2.0f * fa * ux + fb * vy), fe = -(2.0f * fc * vy + fb * ux);
+            const float fbase = ux * (fa * ux + fb * vy) + fc * vy * vy;
+            const float form[6] = {fa, fb, fc, fd, fe, real ? fbase + g1.y : -__builtin_inff()};
+            reinterpret_cast<float*>(shared.qmin[wave])[lane] = real ? g1.z : __builtin_inff();
+            uint64_t discs = 0;
+            if constexpr (COMPOSITE) {
+                discs = __ballot(real && g1.w > 0.5f);
+                float ahead = before[0];
+#pragma unroll
+                for (uint32_t q = 1; q < WAVES; ++q) ahead = from == q ? before[q] : ahead;
+                reinterpret_cast<float*>(shared.chunkReach[wave])[lane] =
+                    real ? fmaxS(ahead, shared.reach[buf][record]) : -3.4e38f;
+            }
+            waveSync();
+            const uint32_t chunkEnd = total - chunk < kLanes ? total - chunk : kLanes;
+            for (uint32_t at16 = 0; at16 < chunkEnd; at16 += 16u) {
+                float sixteen[6];
+#pragma unroll
+                for (uint32_t m = 0; m < 6; ++m) sixteen[m] = shflF(form[m], at16 + (lane & 15u));
+                const uint32_t of = shflU(record, at16 + (lane >> 2));
+                const float channel = reinterpret_cast<const float*>(&shared.colour[buf][of])[lane & 3u];
+                walked += walkSixteen<DEPTH_MODE, COMPOSITE, !COMPOSITE && TRACK>(
+                    w, chunkEnd - at16, sixteen, channel, mono, &shared.qmin[wave][at16 / 4],
+                    &shared.chunkReach[wave][COMPOSITE ? at16 / 4 : 0], stopZ, discs >> at16,
+                    static_cast<int32_t>(at16));
+                if (__ballot(w.t >= kTMin) == 0) break;
+            }
+            waveSync();
+            // the chunk's places become the records' own
+            const auto recordAt = [&](int32_t in) {
+                return static_cast<uint32_t>(__shfl(static_cast<int>(record), in < 0 ? 0 : in, 64));
+            };
+            if constexpr (!COMPOSITE && TRACK) {
+                const uint32_t of = recordAt(w.lastIn);
+                last = w.lastIn >= 0 ? next + of - tileStart + 1u : last;
+                w.lastIn = -1;
+            }
+            if constexpr (DEPTH_MODE == 1) {
+                const uint32_t of = recordAt(w.depthIn);
+                depthAt = w.depthIn >= 0 ? shared.colour[buf][of].w : depthAt;
+                w.depthIn = -1;
+            }
+            if constexpr (COMPOSITE) {
+                const uint32_t of = recordAt(w.opaqueIn);
+                if (w.opaqueIn >= 0) {
+                    const float4 o = shared.colour[buf][of];
+                    oR = o.x, oG = o.y, oB = o.z, oZ = o.w;
+                    opaqueHit = true;
+                }
+                w.opaqueIn = -1;
+            }
+            walks = __ballot(w.t >= kTMin) != 0;
+            if (!walks) break;
+        }
+        if constexpr (WAVES == 1) {
+            if (!walks) break;
+        }
     }
-    // The walk's records, counted on request (the blend's VALU work is
-    // 64 lanes x these steps).
+    const float r = kAlphaMax * w.accum[0], g = kAlphaMax * w.accum[1], b = kAlphaMax * w.accum[2];
+    const float depthSum = kAlphaMax * w.accum[3];
+    const float t = COMPOSITE && w.tStopped >= 0.0f ? w.tStopped : w.t;
+    // The walk's records, counted on request (the blend's work is 64 lanes x
+    // these steps).
     if (walkSteps != nullptr && lane == 0) atomicAdd(walkSteps, walked);
     if constexpr (MODE == kPartial) {
         partialA[lane] = make_float4(r, g, b, depthSum);
         partialB[lane] = make_float2(t, __uint_as_float(last));
         return;
     } else if constexpr (MODE == kResume) {
-        *state = WalkState{r, g, b, t, depthSum, depthAt, last, active};
+        *state = WalkState{r, g, b, t, depthSum, depthAt, last, w.t >= kTMin};
         return;
     }
     if (!inside) return;
@@ -405,73 +665,69 @@ __device__ __forceinline__ void blendQuadrant(BlendList<LIST>& list, const Frame
     }
 }
 
-template <uint32_t DEPTH_MODE, uint32_t LIST, bool COMPOSITE, bool TRACK>
-__global__ __launch_bounds__(kLanes) void blendKernel(FrameParams f, uint32_t slots, const uint32_t* __restrict__ order,
-                                                      const uint2* __restrict__ ranges,
-                                                      const uint32_t* __restrict__ pairSlots,
-                                                      const float4* __restrict__ proj,
-                                                      const float4* __restrict__ underColour,
-                                                      const float* __restrict__ underDepth,
-                                                      float4* __restrict__ colour, float* __restrict__ depth,
-                                                      uint32_t* __restrict__ lastCount,
-                                                      float* __restrict__ finalT, float4* __restrict__ accum,
-                                                      uint32_t* __restrict__ walkSteps,
-                                                      const uint32_t* __restrict__ slotOfPair) {
+// A workgroup a block: four waves a 16x16 one, one wave an 8x8 one. The blocks
+// of one 32-pixel tile are workgroups b, b + 8, b + 16, b + 24, which the
+// dispatcher deals to one XCD, so their gathers of the tile's records share
+// that XCD's L2.
+template <uint32_t DEPTH_MODE, uint32_t WAVES, bool COMPOSITE, bool TRACK>
+__global__ __launch_bounds__(WAVES* kLanes, kWavesPerSimd) void blendKernel(
+    FrameParams f, uint32_t slots, const uint32_t* __restrict__ order, const uint2* __restrict__ ranges,
+    const uint32_t* __restrict__ pairSlots, const float4* __restrict__ proj, const float4* __restrict__ underColour,
+    const float* __restrict__ underDepth, float4* __restrict__ colour, float* __restrict__ depth,
+    uint32_t* __restrict__ lastCount, float* __restrict__ finalT, float4* __restrict__ accum,
+    uint32_t* __restrict__ walkSteps, const uint32_t* __restrict__ slotOfPair) {
     const uint32_t tiles = f.tilesX * f.tilesY;
-    const uint32_t qBits = quadBits(f.tileShift);
-    const uint32_t quadrant = (blockIdx.x >> 3) & ((1u << qBits) - 1u);
-    const uint32_t place = (blockIdx.x >> (3u + qBits)) * 8u + (blockIdx.x & 7u);
+    const uint32_t bits = blockBits(f.tileShift);
+    const uint32_t part = (blockIdx.x >> 3) & ((1u << bits) - 1u);
+    const uint32_t place = (blockIdx.x >> (3u + bits)) * 8u + (blockIdx.x & 7u);
     if (place >= tiles) return;
     const uint32_t tile = order != nullptr ? order[place] : place;
     if (tile >= tiles) return;   // an order entry that is not a tile: draw nothing
-    __shared__ BlendList<LIST> list;
+    __shared__ BlendShared<WAVES, COMPOSITE> shared;
     const uint2 rg = ranges[tile];
-    blendQuadrant<DEPTH_MODE, LIST, COMPOSITE, kFinish, TRACK>(list, f, tile, quadrant, rg, rg.x, slots, pairSlots, proj,
-                                                               underColour, underDepth, colour, depth, lastCount,
-                                                               finalT, accum, nullptr, nullptr, nullptr, walkSteps,
-                                                               slotOfPair);
+    blendBlock<DEPTH_MODE, WAVES, COMPOSITE, kFinish, TRACK>(
+        shared, f, partOrigin(f, tile, part, WAVES == 1 ? 3u : 4u), rg, rg.x, slots, pairSlots, proj, underColour,
+        underDepth, colour, depth, lastCount, finalT, accum, nullptr, nullptr, nullptr, walkSteps, slotOfPair);
 }
 
-// Every quadrant of every view of a batch (2^qBits quadrants a tile). As a
-// grid (PERSISTENT false) block b is task b, the quadrants of a tile going to
-// blocks b, b + 8, b + 16, ... of one XCD; persistent, each block takes tasks
-// from a shared counter until none are left (task t: tile t >> qBits,
-// quadrant t & (2^qBits - 1)), so a block that drew a light quadrant takes the
-// next instead of leaving its slot idle.
-template <uint32_t DEPTH_MODE, uint32_t LIST, bool PERSISTENT, bool TRACK>
-__global__ __launch_bounds__(kLanes) void blendViewsKernel(const FrameParams* __restrict__ params,
-                                                           const ViewInfo* __restrict__ views, uint32_t viewCount,
-                                                           uint32_t tiles, uint32_t qBits, uint32_t tasks,
-                                                           uint32_t slots,
-                                                           const uint2* __restrict__ ranges,
-                                                           const uint32_t* __restrict__ pairSlots,
-                                                           const float4* __restrict__ proj,
-                                                           uint32_t* __restrict__ lastCount,
-                                                           float* __restrict__ finalT, float4* __restrict__ accum,
-                                                           uint32_t* __restrict__ queue,
-                                                           const uint32_t* __restrict__ slotOfPair) {
-    __shared__ BlendList<LIST> list;
-    for (uint32_t round = 0;; ++round) {
-        uint32_t task, g, quadrant;
+// Every block of every view of a batch (2^bits blocks a tile). As a grid
+// (PERSISTENT false) workgroup b is task b, the blocks of a tile going to
+// workgroups b, b + 8, b + 16, ... of one XCD; persistent, each workgroup takes
+// tasks from a shared counter until none are left (task t: tile t >> bits,
+// block t & (2^bits - 1)), so one that drew a light block takes the next
+// instead of leaving its slot idle.
+template <uint32_t DEPTH_MODE, uint32_t WAVES, bool PERSISTENT, bool TRACK>
+__global__ __launch_bounds__(WAVES* kLanes, kWavesPerSimd) void blendViewsKernel(
+    const FrameParams* __restrict__ params, const ViewInfo* __restrict__ views, uint32_t viewCount, uint32_t tiles,
+    uint32_t bits, uint32_t tasks, uint32_t slots, const uint2* __restrict__ ranges,
+    const uint32_t* __restrict__ pairSlots, const float4* __restrict__ proj, uint32_t* __restrict__ lastCount,
+    float* __restrict__ finalT, float4* __restrict__ accum, uint32_t* __restrict__ queue,
+    const uint32_t* __restrict__ slotOfPair) {
+    __shared__ BlendShared<WAVES, false> shared;
+    __shared__ uint32_t sTask;
+    while (true) {
+        uint32_t task, g, part;
         if constexpr (PERSISTENT) {
-            uint32_t taken = 0;
-            if (threadIdx.x == 0) taken = atomicAdd(queue, 1u);
-            task = static_cast<uint32_t>(__shfl(static_cast<int>(taken), 0, 64));
+            __syncthreads();   // the last task's LDS is done with
+            if (threadIdx.x == 0) sTask = atomicAdd(queue, 1u);
+            __syncthreads();
+            task = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(sTask)));
             if (task >= tasks) return;
-            g = task >> qBits;
-            quadrant = task & ((1u << qBits) - 1u);
-            if (round > 0) __syncthreads();   // the last task's LDS list is done with
+            g = task >> bits;
+            part = task & ((1u << bits) - 1u);
         } else {
             task = blockIdx.x;
-            g = (task >> (3u + qBits)) * 8u + (task & 7u);
-            quadrant = (task >> 3) & ((1u << qBits) - 1u);
+            g = (task >> (3u + bits)) * 8u + (task & 7u);
+            part = (task >> 3) & ((1u << bits) - 1u);
         }
         if (g < tiles) {
             const ViewInfo& v = views[viewOfTile(views, viewCount, g)];
+            const FrameParams& f = params[v.params];
             const uint2 rg = ranges[g];
-            blendQuadrant<DEPTH_MODE, LIST, false, kFinish, TRACK>(
-                list, params[v.params], g - v.tileBase, quadrant, rg, rg.x, slots, pairSlots, proj, nullptr, nullptr,
-                reinterpret_cast<float4*>(v.colour), v.depth, lastCount != nullptr ? lastCount + v.pixelBase : nullptr,
+            blendBlock<DEPTH_MODE, WAVES, false, kFinish, TRACK>(
+                shared, f, partOrigin(f, g - v.tileBase, part, WAVES == 1 ? 3u : 4u), rg, rg.x, slots, pairSlots,
+                proj, nullptr, nullptr, reinterpret_cast<float4*>(v.colour), v.depth,
+                lastCount != nullptr ? lastCount + v.pixelBase : nullptr,
                 finalT != nullptr ? finalT + v.pixelBase : nullptr, accum != nullptr ? accum + v.pixelBase : nullptr,
                 nullptr, nullptr, nullptr, nullptr, slotOfPair);
         }
@@ -486,7 +742,6 @@ __global__ __launch_bounds__(kLanes) void blendViewsKernel(const FrameParams* __
 // descending, wave ascending) gives each wave its first place in every bucket,
 // and each wave walks its segment again handing out places.
 constexpr uint32_t kBuckets = 33;
-constexpr uint32_t kNoSlot = 0xFFFFFFFFu;   // a task that finishes its tile's pixels itself
 constexpr uint32_t kOrderWaves = 16;
 constexpr uint32_t kOrderCached = 32768;   // tiles whose bucket the first walk leaves in LDS for the second
 
@@ -659,8 +914,8 @@ __global__ __launch_bounds__(kOrderWaves * 64) void tileOrderKernel(const uint2*
 // The tasks of a split plan: task k's quadrants are blocks b, b + 8, b + 16,
 // ... of one XCD. A task of an unsplit tile finishes its pixels; a
 // segment leaves its partial walk in its slot.
-template <uint32_t DEPTH_MODE, uint32_t LIST>
-__global__ __launch_bounds__(kLanes) void blendTasksKernel(FrameParams f, uint32_t slots, const uint4* __restrict__ tasks,
+template <uint32_t DEPTH_MODE>
+__global__ __launch_bounds__(kLanes, kWavesPerSimd) void blendTasksKernel(FrameParams f, uint32_t slots, const uint4* __restrict__ tasks,
                                                            const uint32_t* __restrict__ planCounts,
                                                            const uint2* __restrict__ ranges,
                                                            const uint32_t* __restrict__ pairSlots,
@@ -673,18 +928,19 @@ __global__ __launch_bounds__(kLanes) void blendTasksKernel(FrameParams f, uint32
     const uint32_t quadrant = (blockIdx.x >> 3) & ((1u << qBits) - 1u);
     const uint32_t task = (blockIdx.x >> (3u + qBits)) * 8u + (blockIdx.x & 7u);
     if (task >= planCounts[0]) return;
-    __shared__ BlendList<LIST> list;
+    __shared__ BlendShared<1, false> shared;
     const uint4 tk = tasks[task];
     const uint32_t tileStart = ranges[tk.x].x;
     if (tk.w == kNoSlot) {
-        blendQuadrant<DEPTH_MODE, LIST, false, kFinish>(list, f, tk.x, quadrant, make_uint2(tk.y, tk.z), tileStart, slots,
-                                                        pairSlots, proj, nullptr, nullptr, colour, depth, lastCount,
-                                                        finalT, nullptr);
+        blendBlock<DEPTH_MODE, 1, false, kFinish>(shared, f, partOrigin(f, tk.x, quadrant, 3u),
+                                                  make_uint2(tk.y, tk.z), tileStart, slots, pairSlots, proj, nullptr,
+                                                  nullptr, colour, depth, lastCount, finalT, nullptr);
     } else {
         const uint64_t at = ((static_cast<uint64_t>(tk.w) << qBits) + quadrant) * kLanes;
-        blendQuadrant<DEPTH_MODE, LIST, false, kPartial>(list, f, tk.x, quadrant, make_uint2(tk.y, tk.z), tileStart, slots,
-                                                         pairSlots, proj, nullptr, nullptr, colour, depth, lastCount,
-                                                         finalT, nullptr, nullptr, partialA + at, partialB + at);
+        blendBlock<DEPTH_MODE, 1, false, kPartial>(shared, f, partOrigin(f, tk.x, quadrant, 3u),
+                                                   make_uint2(tk.y, tk.z), tileStart, slots, pairSlots, proj, nullptr,
+                                                   nullptr, colour, depth, lastCount, finalT, nullptr, nullptr,
+                                                   partialA + at, partialB + at);
     }
 }
 
@@ -693,8 +949,8 @@ __global__ __launch_bounds__(kLanes) void blendTasksKernel(FrameParams f, uint32
 // stop inside a segment (T below 1e-4, or the threshold depth crossed) walks
 // that segment again from its true state, so it stops where the one walk
 // would; the others take the segment whole.
-template <uint32_t DEPTH_MODE, uint32_t LIST>
-__global__ __launch_bounds__(kLanes) void combineKernel(FrameParams f, uint32_t slots, const uint4* __restrict__ combine,
+template <uint32_t DEPTH_MODE>
+__global__ __launch_bounds__(kLanes, kWavesPerSimd) void combineKernel(FrameParams f, uint32_t slots, const uint4* __restrict__ combine,
                                                         const uint32_t* __restrict__ planCounts,
                                                         const uint2* __restrict__ ranges,
                                                         const uint32_t* __restrict__ pairSlots,
@@ -709,14 +965,14 @@ __global__ __launch_bounds__(kLanes) void combineKernel(FrameParams f, uint32_t 
     if (c >= planCounts[1]) return;
     const uint4 ct = combine[c];
     const uint32_t tile = ct.x, n = ct.z, lane = threadIdx.x;
-    const uint2 origin = quadrantOrigin(f, tile, quadrant);
+    const uint2 origin = partOrigin(f, tile, quadrant, 3u);
     const uint32_t x0 = origin.x, y0 = origin.y;
     if (x0 >= f.width || y0 >= f.height) return;
     const uint32_t px = x0 + (lane & 7u), py = y0 + (lane >> 3);
     const bool inside = px < f.width && py < f.height && px < x0 + 8u && py < y0 + 8u;
     const uint2 rg = ranges[tile];
     const uint32_t len = rg.y - rg.x, segLen = (len + n - 1u) / n;
-    __shared__ BlendList<LIST> list;
+    __shared__ BlendShared<1, false> shared;
     WalkState st{0.0f, 0.0f, 0.0f, 1.0f, 0.0f, -1.0f, 0u, inside};
     for (uint32_t k = 0; k < n; ++k) {
         const uint64_t at = ((static_cast<uint64_t>(ct.y + k) << qBits) + quadrant) * kLanes + lane;
@@ -741,9 +997,9 @@ __global__ __launch_bounds__(kLanes) void combineKernel(FrameParams f, uint32_t 
             const uint32_t end = begin + segLen < rg.y ? begin + segLen : rg.y;
             WalkState w = st;
             w.active = again;
-            blendQuadrant<DEPTH_MODE, LIST, false, kResume>(list, f, tile, quadrant, make_uint2(begin, end), rg.x, slots,
-                                                            pairSlots, proj, nullptr, nullptr, colour, depth,
-                                                            lastCount, finalT, nullptr, &w);
+            blendBlock<DEPTH_MODE, 1, false, kResume>(shared, f, origin, make_uint2(begin, end), rg.x, slots,
+                                                      pairSlots, proj, nullptr, nullptr, colour, depth, lastCount,
+                                                      finalT, nullptr, &w);
             if (again) st = w;
             __syncthreads();   // the walk's list is refilled by the next one
         }
@@ -754,81 +1010,76 @@ __global__ __launch_bounds__(kLanes) void combineKernel(FrameParams f, uint32_t 
 }
 
 template <uint32_t DEPTH_MODE, bool COMPOSITE>
-void launchBlend(uint32_t list, const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
+void launchBlend(const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
                  const uint32_t* pairSlots, const float4* proj, const float4* underColour, const float* underDepth,
                  float4* colour, float* depth, uint32_t* lastCount, float* finalT, float4* accum,
                  hipStream_t stream, uint32_t* walkSteps = nullptr, const uint32_t* slotOfPair = nullptr) {
-    // A block a quadrant, the grid rounded up to whole groups of eight tiles.
+    // A workgroup a block, the grid rounded up to whole groups of eight tiles.
     // The last contributor is tracked only where it is kept.
     const uint32_t tiles = f.tilesX * f.tilesY;
-    const uint32_t blocks = (tiles + 7u) / 8u * (8u << (2u * (f.tileShift - 3u)));
-    const auto go = [&](auto listLen, auto track) {
-        blendKernel<DEPTH_MODE, decltype(listLen)::value, COMPOSITE, decltype(track)::value>
-            <<<blocks, kLanes, 0, stream>>>(f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour,
-                                            depth, lastCount, finalT, accum, walkSteps, slotOfPair);
+    const uint32_t blocks = (tiles + 7u) / 8u * (8u << blockBits(f.tileShift));
+    const auto go = [&](auto waves, auto track) {
+        constexpr uint32_t W = decltype(waves)::value;
+        blendKernel<DEPTH_MODE, W, COMPOSITE, decltype(track)::value><<<blocks, W * kLanes, 0, stream>>>(
+            f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour, depth, lastCount, finalT, accum,
+            walkSteps, slotOfPair);
     };
-    using L64 = std::integral_constant<uint32_t, 64>;
-    using L128 = std::integral_constant<uint32_t, 128>;
-    using L256 = std::integral_constant<uint32_t, 256>;
-    using Keep = std::true_type;
-    using Drop = std::false_type;
-    const bool track = !COMPOSITE && lastCount != nullptr;
-    if (list <= 64) {
-        if (track) go(L64{}, Keep{}); else go(L64{}, Drop{});
-    } else if (list <= 128) {
-        if (track) go(L128{}, Keep{}); else go(L128{}, Drop{});
+    using One = std::integral_constant<uint32_t, 1>;
+    using Four = std::integral_constant<uint32_t, 4>;
+    if (!COMPOSITE && lastCount != nullptr) {
+        if (f.tileShift == 3) go(One{}, std::bool_constant<!COMPOSITE>{}); else go(Four{}, std::bool_constant<!COMPOSITE>{});
     } else {
-        if (track) go(L256{}, Keep{}); else go(L256{}, Drop{});
+        if (f.tileShift == 3) go(One{}, std::false_type{}); else go(Four{}, std::false_type{});
     }
 }
 
-template <uint32_t DEPTH_MODE, uint32_t LIST>
+template <uint32_t DEPTH_MODE>
 void launchBlendViews(bool persistent, uint32_t gridCap, const FrameParams* params, const ViewInfo* views,
                       uint32_t viewCount, uint32_t tiles, uint32_t tileShift, uint32_t slots, const uint2* ranges,
                       const uint32_t* pairSlots, const float4* proj, uint32_t* lastCount, float* finalT, float4* accum,
                       uint32_t* queue, hipStream_t stream, const uint32_t* slotOfPair) {
-    const uint32_t qBits = 2u * (tileShift - 3u);
-    const auto go = [&](auto track) {
+    const uint32_t bits = blockBits(tileShift);
+    const auto go = [&](auto waves, auto track) {
+        constexpr uint32_t W = decltype(waves)::value;
         constexpr bool T = decltype(track)::value;
         if (persistent) {
-            const uint32_t tasks = tiles << qBits;
-            const uint32_t grid = tasks < gridCap ? tasks : gridCap;
+            const uint32_t tasks = tiles << bits;
+            const uint32_t cap = gridCap / W > 0 ? gridCap / W : 1u;
+            const uint32_t grid = tasks < cap ? tasks : cap;
             fill32(queue, 0u, 1, stream);
-            blendViewsKernel<DEPTH_MODE, LIST, true, T><<<grid, kLanes, 0, stream>>>(
-                params, views, viewCount, tiles, qBits, tasks, slots, ranges, pairSlots, proj, lastCount, finalT,
+            blendViewsKernel<DEPTH_MODE, W, true, T><<<grid, W * kLanes, 0, stream>>>(
+                params, views, viewCount, tiles, bits, tasks, slots, ranges, pairSlots, proj, lastCount, finalT,
                 accum, queue, slotOfPair);
         } else {
-            const uint32_t tasks = (tiles + 7u) / 8u * (8u << qBits);
-            blendViewsKernel<DEPTH_MODE, LIST, false, T><<<tasks, kLanes, 0, stream>>>(
-                params, views, viewCount, tiles, qBits, tasks, slots, ranges, pairSlots, proj, lastCount, finalT,
+            const uint32_t tasks = (tiles + 7u) / 8u * (8u << bits);
+            blendViewsKernel<DEPTH_MODE, W, false, T><<<tasks, W * kLanes, 0, stream>>>(
+                params, views, viewCount, tiles, bits, tasks, slots, ranges, pairSlots, proj, lastCount, finalT,
                 accum, queue, slotOfPair);
         }
     };
-    if (lastCount != nullptr) go(std::true_type{}); else go(std::false_type{});
+    using One = std::integral_constant<uint32_t, 1>;
+    using Four = std::integral_constant<uint32_t, 4>;
+    if (lastCount != nullptr) {
+        if (tileShift == 3) go(One{}, std::true_type{}); else go(Four{}, std::true_type{});
+    } else {
+        if (tileShift == 3) go(One{}, std::false_type{}); else go(Four{}, std::false_type{});
+    }
 }
 
 }   // namespace
 
-void blendViews(uint32_t depthMode, uint32_t list, bool persistent, uint32_t gridCap, const FrameParams* params,
+void blendViews(uint32_t depthMode, bool persistent, uint32_t gridCap, const FrameParams* params,
                 const ViewInfo* views, uint32_t viewCount, uint32_t tiles, uint32_t tileShift, uint32_t slots,
                 const uint2* ranges,
                 const uint32_t* pairSlots, const float4* proj, uint32_t* lastCount, float* finalT, float4* accum,
                 uint32_t* queue, hipStream_t stream, const uint32_t* slotOfPair) {
     if (tiles == 0 || viewCount == 0) return;
-    const auto go = [&](auto depthMode, auto listLen) {
-        launchBlendViews<decltype(depthMode)::value, decltype(listLen)::value>(
-            persistent, gridCap, params, views, viewCount, tiles, tileShift, slots, ranges, pairSlots, proj, lastCount,
-            finalT, accum, queue, stream, slotOfPair);
-    };
-    using D0 = std::integral_constant<uint32_t, 0>;
-    using D1 = std::integral_constant<uint32_t, 1>;
-    using L64 = std::integral_constant<uint32_t, 64>;
-    using L128 = std::integral_constant<uint32_t, 128>;
-    using L256 = std::integral_constant<uint32_t, 256>;
     if (depthMode == 0) {
-        if (list <= 64) go(D0{}, L64{}); else if (list <= 128) go(D0{}, L128{}); else go(D0{}, L256{});
+        launchBlendViews<0>(persistent, gridCap, params, views, viewCount, tiles, tileShift, slots, ranges, pairSlots,
+                            proj, lastCount, finalT, accum, queue, stream, slotOfPair);
     } else {
-        if (list <= 64) go(D1{}, L64{}); else if (list <= 128) go(D1{}, L128{}); else go(D1{}, L256{});
+        launchBlendViews<1>(persistent, gridCap, params, views, viewCount, tiles, tileShift, slots, ranges, pairSlots,
+                            proj, lastCount, finalT, accum, queue, stream, slotOfPair);
     }
 }
 
@@ -837,62 +1088,57 @@ void tileOrder(const uint2* ranges, uint32_t tiles, uint32_t* order, hipStream_t
     tileOrderKernel<<<1, kOrderWaves * 64, 0, stream>>>(ranges, tiles, order, 0u, nullptr, nullptr, nullptr);
 }
 
-void blendSplit(const FrameParams& f, uint32_t list, uint32_t segmentPairs, uint32_t slots, const uint2* ranges,
+void blendSplit(const FrameParams& f, uint32_t segmentPairs, uint32_t slots, const uint2* ranges,
                 const uint32_t* pairSlots, const float4* proj, const BlendPlan& plan, float4* colour, float* depth,
                 uint32_t* lastCount, float* finalT, hipStream_t stream) {
     const uint32_t tiles = f.tilesX * f.tilesY;
     if (tiles == 0) return;
     tileOrderKernel<<<1, kOrderWaves * 64, 0, stream>>>(ranges, tiles, plan.order, segmentPairs, plan.tasks,
                                                         plan.combine, plan.counts);
-    const uint32_t qBits = 2u * (f.tileShift - 3u);
+    const uint32_t qBits = quadBits(f.tileShift);
     const uint32_t taskBlocks = (plan.taskCapacity + 7u) / 8u * (8u << qBits);
     const uint32_t combineBlocks = plan.combineCapacity << qBits;
-    const auto launch = [&](auto depthMode, auto listLen) {
-        constexpr uint32_t D = decltype(depthMode)::value, L = decltype(listLen)::value;
-        blendTasksKernel<D, L><<<taskBlocks, kLanes, 0, stream>>>(f, slots, plan.tasks, plan.counts, ranges, pairSlots,
-                                                                  proj, colour, depth, lastCount, finalT,
-                                                                  plan.partialA, plan.partialB);
+    const auto launch = [&](auto depthMode) {
+        constexpr uint32_t D = decltype(depthMode)::value;
+        blendTasksKernel<D><<<taskBlocks, kLanes, 0, stream>>>(f, slots, plan.tasks, plan.counts, ranges, pairSlots,
+                                                               proj, colour, depth, lastCount, finalT, plan.partialA,
+                                                               plan.partialB);
         if (combineBlocks > 0) {
-            combineKernel<D, L><<<combineBlocks, kLanes, 0, stream>>>(f, slots, plan.combine, plan.counts, ranges,
-                                                                      pairSlots, proj, colour, depth, lastCount,
-                                                                      finalT, plan.partialA, plan.partialB);
+            combineKernel<D><<<combineBlocks, kLanes, 0, stream>>>(f, slots, plan.combine, plan.counts, ranges,
+                                                                   pairSlots, proj, colour, depth, lastCount, finalT,
+                                                                   plan.partialA, plan.partialB);
         }
     };
-    using D0 = std::integral_constant<uint32_t, 0>;
-    using D1 = std::integral_constant<uint32_t, 1>;
-    using L64 = std::integral_constant<uint32_t, 64>;
-    using L128 = std::integral_constant<uint32_t, 128>;
-    using L256 = std::integral_constant<uint32_t, 256>;
     if (f.depthMode == 0) {
-        if (list <= 64) launch(D0{}, L64{}); else if (list <= 128) launch(D0{}, L128{}); else launch(D0{}, L256{});
+        launch(std::integral_constant<uint32_t, 0>{});
     } else {
-        if (list <= 64) launch(D1{}, L64{}); else if (list <= 128) launch(D1{}, L128{}); else launch(D1{}, L256{});
+        launch(std::integral_constant<uint32_t, 1>{});
     }
 }
 
-void blend(const FrameParams& f, uint32_t list, uint32_t slots, const uint32_t* order, const uint2* ranges,
+void blend(const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
            const uint32_t* pairSlots, const float4* proj, float4* colour, float* depth, uint32_t* lastCount,
            float* finalT, float4* accum, hipStream_t stream, uint32_t* walkSteps, const uint32_t* slotOfPair) {
     if (f.tilesX * f.tilesY == 0) return;
     if (f.depthMode == 0) {
-        launchBlend<0, false>(list, f, slots, order, ranges, pairSlots, proj, nullptr, nullptr, colour, depth,
-                              lastCount, finalT, accum, stream, walkSteps, slotOfPair);
+        launchBlend<0, false>(f, slots, order, ranges, pairSlots, proj, nullptr, nullptr, colour, depth, lastCount,
+                              finalT, accum, stream, walkSteps, slotOfPair);
     } else {
-        launchBlend<1, false>(list, f, slots, order, ranges, pairSlots, proj, nullptr, nullptr, colour, depth,
-                              lastCount, finalT, accum, stream, walkSteps, slotOfPair);
+        launchBlend<1, false>(f, slots, order, ranges, pairSlots, proj, nullptr, nullptr, colour, depth, lastCount,
+                              finalT, accum, stream, walkSteps, slotOfPair);
     }
 }
 
-void blendComposite(const FrameParams& f, uint32_t list, uint32_t slots, const uint32_t* order, const uint2* ranges,
+void blendComposite(const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
                     const uint32_t* pairSlots, const float4* proj, const float4* underColour,
                     const float* underDepth, float4* colour, float* depth, hipStream_t stream) {
     if (f.tilesX * f.tilesY == 0) return;
     if (f.depthMode == 0) {
-        launchBlend<0, true>(list, f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour, depth,
-                             nullptr, nullptr, nullptr, stream);
+        launchBlend<0, true>(f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour, depth, nullptr,
+                             nullptr, nullptr, stream);
     } else {
-        launchBlend<1, true>(list, f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour, depth,
-                             nullptr, nullptr, nullptr, stream);
+        launchBlend<1, true>(f, slots, order, ranges, pairSlots, proj, underColour, underDepth, colour, depth, nullptr,
+                             nullptr, nullptr, stream);
     }
 }
 

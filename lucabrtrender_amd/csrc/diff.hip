@@ -445,12 +445,12 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
                     screen = proj[s3];
                     conic = proj[s3 + 1];
                     col = proj[s3 + 2];
+                    const ReachConic rc = reachConic(conic.x, conic.y, conic.z);
 #pragma unroll
                     for (uint32_t q = 0; q < kWaves; ++q) {
                         if (boxHi[q][0] < 0.0f || boxHi[q][1] < 0.0f) continue;
-                        if (quadrantReach(conic.x, conic.y, conic.z, screen.w, boxLo[q][0] - screen.x,
-                                             boxLo[q][1] - screen.y, boxHi[q][0] - screen.x,
-                                             boxHi[q][1] - screen.y)) {
+                        if (quadrantReach(rc, screen.w, boxLo[q][0] - screen.x, boxLo[q][1] - screen.y,
+                                          boxHi[q][0] - screen.x, boxHi[q][1] - screen.y)) {
                             mask |= 1u << q;
                         }
                     }

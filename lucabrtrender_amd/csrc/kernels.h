@@ -201,13 +201,13 @@ void widenKeys(const uint32_t* keys, uint32_t tileShift, const uint32_t* slots, 
 // Tile indices, heaviest tile (most pairs) first, for the blend's launch order.
 void tileOrder(const uint2* ranges, uint32_t tiles, uint32_t* order, hipStream_t stream);
 // Per pixel, front to back over its tile's pairs; one wave per 8x8 quadrant,
-// whose LDS list holds `list` (64, 128 or 256) records; tiles in `order`
-// (null: index order); slots bounds the pair slots. pairSlots holds the
+// the four of a 16x16 block in one workgroup; tiles in `order` (null: index
+// order); slots bounds the pair slots. pairSlots holds the
 // sorted pairs' slots, or with slotOfPair non-null their pair indices, each
 // pair's slot then slotOfPair[index]. lastCount/finalT/accum may be null;
 // accum receives each pixel's raw rgb and depth sum before the linearisation
 // and the background.
-void blend(const FrameParams& f, uint32_t list, uint32_t slots, const uint32_t* order, const uint2* ranges,
+void blend(const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
            const uint32_t* pairSlots, const float4* proj, float4* colour, float* depth, uint32_t* lastCount,
            float* finalT, float4* accum, hipStream_t stream, uint32_t* walkSteps = nullptr,
            const uint32_t* slotOfPair = nullptr);
@@ -218,7 +218,7 @@ void blend(const FrameParams& f, uint32_t list, uint32_t slots, const uint32_t* 
 // pixel whose under depth is above 0 ends its walk at the first record at or
 // behind that depth, and the under-layer's colour (float4 a pixel) lies behind
 // what it blended. Writes colour and depth (may be null) only.
-void blendComposite(const FrameParams& f, uint32_t list, uint32_t slots, const uint32_t* order, const uint2* ranges,
+void blendComposite(const FrameParams& f, uint32_t slots, const uint32_t* order, const uint2* ranges,
                     const uint32_t* pairSlots, const float4* proj, const float4* underColour,
                     const float* underDepth, float4* colour, float* depth, hipStream_t stream);
 
@@ -240,7 +240,7 @@ struct BlendPlan {
     float2* partialB;
     uint32_t taskCapacity, combineCapacity;
 };
-void blendSplit(const FrameParams& f, uint32_t list, uint32_t segmentPairs, uint32_t slots, const uint2* ranges,
+void blendSplit(const FrameParams& f, uint32_t segmentPairs, uint32_t slots, const uint2* ranges,
                 const uint32_t* pairSlots, const float4* proj, const BlendPlan& plan, float4* colour, float* depth,
                 uint32_t* lastCount, float* finalT, hipStream_t stream);
 
@@ -250,7 +250,7 @@ void blendSplit(const FrameParams& f, uint32_t list, uint32_t segmentPairs, uint
 // cleared here). Every view's tiles are 2^tileShift pixels a side.
 // lastCount/finalT/accum (each may be null) hold the batch's pixels
 // (ViewInfo.pixelBase); accum as blend()'s.
-void blendViews(uint32_t depthMode, uint32_t list, bool persistent, uint32_t gridCap, const FrameParams* params,
+void blendViews(uint32_t depthMode, bool persistent, uint32_t gridCap, const FrameParams* params,
                 const ViewInfo* views, uint32_t viewCount, uint32_t tiles, uint32_t tileShift, uint32_t slots,
                 const uint2* ranges,
                 const uint32_t* pairSlots, const float4* proj, uint32_t* lastCount, float* finalT, float4* accum,

@@ -493,20 +493,19 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
         plan.counts = counters + 6;
         plan.partialA = partials_.as<float4>();
         plan.partialB = reinterpret_cast<float2*>(partials_.as<uint8_t>() + partialBytes);
-        kern::blendSplit(first, settings.blendBatch, seg, splatCount, ranges_.as<uint2>(), pairSlots,
+        kern::blendSplit(first, seg, splatCount, ranges_.as<uint2>(), pairSlots,
                          proj_.as<float4>(), plan, targets.colour, targets.depth, lastCountOut, finalTOut, stream_);
     } else if (composite) {
-        kern::blendComposite(first, settings.blendBatch, splatCount, order, ranges_.as<uint2>(), pairSlots,
+        kern::blendComposite(first, splatCount, order, ranges_.as<uint2>(), pairSlots,
                              proj_.as<float4>(), under != nullptr ? under->colour : nullptr,
                              under != nullptr ? under->depth : nullptr, targets.colour, targets.depth, stream_);
     } else {
-        kern::blend(first, settings.blendBatch, splatCount, order, ranges_.as<uint2>(), pairSlots,
+        kern::blend(first, splatCount, order, ranges_.as<uint2>(), pairSlots,
                     proj_.as<float4>(), targets.colour, targets.depth, lastCountOut, finalTOut,
                     training ? accum_.as<float4>() : nullptr, stream_, nullptr, slotOfPair);
     }
     lastBlendPlain_ = !split && !composite && !training;   // a training frame's accum_ is kept
     lastBlendFrame_ = first;
-    lastBlendList_ = settings.blendBatch;
     lastBlendSlots_ = splatCount;
     lastBlendOrder_ = order;
     lastBlendPairSlots_ = pairSlots;
@@ -622,7 +621,7 @@ void TileRasterizer::enqueueViews(std::span<const SplatInstance> instances, cons
     mark(7);
     // A persistent blend keeps about 24 one-wave workgroups on each CU.
     const bool keepWalk = training || settings.keepWalkState;
-    kern::blendViews(settings.depthMode, settings.blendBatch, settings.persistentBlend, computeUnits_ * 24u, params,
+    kern::blendViews(settings.depthMode, settings.persistentBlend, computeUnits_ * 24u, params,
                      views, viewCount, tiles, tileShiftOf(settings.tileSize), slots, ranges_.as<uint2>(), pairSlots,
                      proj_.as<float4>(),
                      keepWalk ? lastCount_.as<uint32_t>() : nullptr, keepWalk ? finalT_.as<float>() : nullptr,
@@ -824,7 +823,7 @@ Status TileRasterizer::runViews(std::span<const View> views, std::span<const Spl
             // address: any change of either needs a new capture.
             std::string key = std::to_string(viewCount) + "/" + std::to_string(splatsPerView) + "/" +
                               std::to_string(tiles) + "/" + std::to_string(pairCapacity_) + "/" +
-                              std::to_string(settings.blendBatch) + "/" + std::to_string(settings.persistentBlend) +
+                              std::to_string(settings.persistentBlend) +
                               "/" + std::to_string(settings.keepWalkState) + "/" + std::to_string(training) + "/" +
                               std::to_string(settings.depthMode) + "/" + std::to_string(settings.tileSize) + "/" +
                               std::to_string(settings.radixBits) + "/" +
@@ -998,13 +997,11 @@ Status TileRasterizer::autotuneViews(std::span<const View> views, std::span<cons
                                      RenderSettings& settings, float* ms) {
     RenderSettings best = settings;
     double bestMs = -1.0;
-    for (const uint32_t tile : {8u, 16u, 32u})
-    for (const uint32_t list : {64u, 128u, 256u}) {
+    for (const uint32_t tile : {8u, 16u, 32u}) {
         for (const bool persistent : {false, true}) {
             for (const bool graph : {false, true}) {
                 RenderSettings trial = settings;
                 trial.tileSize = tile;
-                trial.blendBatch = list;
                 trial.persistentBlend = persistent;
                 trial.useGraph = graph;
                 Status s = renderViews(views, instances, trial, nullptr);   // sizes buffers, captures
@@ -1327,7 +1324,7 @@ Status TileRasterizer::debugCopy(int which, void* host, size_t bytes, size_t* ne
         if (!(s = accum_.reserve(std::max<uint64_t>(pixels, 1) * 16, "walk.colour")).ok()) return s;
         if (!(s = walkSteps_.reserve(4, "walk.steps")).ok()) return s;
         kern::fill32(walkSteps_.as<uint32_t>(), 0u, 1, stream_);
-        kern::blend(lastBlendFrame_, lastBlendList_, lastBlendSlots_, lastBlendOrder_, ranges_.as<uint2>(),
+        kern::blend(lastBlendFrame_, lastBlendSlots_, lastBlendOrder_, ranges_.as<uint2>(),
                     lastBlendPairSlots_, proj_.as<float4>(), accum_.as<float4>(), nullptr, nullptr, nullptr, nullptr,
                     stream_, walkSteps_.as<uint32_t>());
         src = walkSteps_.get();

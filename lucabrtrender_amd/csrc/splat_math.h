@@ -150,27 +150,40 @@ __device__ __forceinline__ float minPowerOverBox(float a, float b, float c, floa
 
 // Can the Gaussian (power a x^2 + 2 b x y + c y^2 about its centre) reach
 // cutoff at some point of the box [lox, hix] x [loy, hiy] (coordinates about
-// the centre)? The power is convex, so its minimum over the box is 0 when the
-// centre is inside and otherwise lies on an edge, at the clamped minimiser of
-// the edge's 1-D quadratic. The answer may be yes for a box that no pixel
+// the centre, at most 8 on a side)? The power is convex, so over a box that
+// does not hold the centre its minimum lies on an edge that faces the centre:
+// x = the box's nearest x, or y = its nearest y, each at the clamped minimiser
+// of the edge's 1-D quadratic (a box that holds the centre has the centre for
+// nearest point, power 0). The answer may be yes for a box that no pixel
 // reaches, never no for one that a pixel reaches: the slack bounds the float
 // rounding of this evaluation and of the per-pixel one, both below a few ulps
 // of (a + 2|b| + c) * r2 with r2 the largest squared coordinate in the box,
 // ten times over; the edge minimisers use the hardware reciprocal, whose error
 // moves the value only to second order. A degenerate form is always kept.
-__device__ __forceinline__ bool quadrantReach(float a, float b, float c, float cutoff, float lox, float loy,
-                                              float hix, float hiy) {
-    const bool centreInside = lox <= 0.0f && hix >= 0.0f && loy <= 0.0f && hiy >= 0.0f;
-    const bool degenerate = !(a > 1e-12f && c > 1e-12f);
-    const float ra = __builtin_amdgcn_rcpf(a), rc = __builtin_amdgcn_rcpf(c);
-    const auto form = [&](float x, float y) { return __builtin_fmaf(a * x, x, __builtin_fmaf(2.0f * b * x, y, c * y * y)); };
-    float best = form(lox, fminS(fmaxS(-b * lox * rc, loy), hiy));
-    best = fminS(best, form(hix, fminS(fmaxS(-b * hix * rc, loy), hiy)));
-    best = fminS(best, form(fminS(fmaxS(-b * loy * ra, lox), hix), loy));
-    best = fminS(best, form(fminS(fmaxS(-b * hiy * ra, lox), hix), hiy));
-    const float r2 = fmaxS(fmaxS(lox * lox, hix * hix), fmaxS(loy * loy, hiy * hiy));
-    const float slack = 4e-6f * (a + 2.0f * __builtin_fabsf(b) + c) * r2 + 1e-5f * cutoff + 1e-6f;
-    return centreInside || degenerate || best <= cutoff + slack;
+// What depends on the form alone is taken once for several boxes (ReachConic).
+struct ReachConic {
+    float a, b2, c;      // the form, b doubled
+    float yOfX, xOfY;    // the edge minimisers' slopes, -b / c and -b / a
+    float size;          // a + 2|b| + c, times the slack's factor
+    bool degenerate;
+};
+
+__device__ __forceinline__ ReachConic reachConic(float a, float b, float c) {
+    const float b2 = b + b;
+    return ReachConic{a, b2, c, -b * __builtin_amdgcn_rcpf(c), -b * __builtin_amdgcn_rcpf(a),
+                      4e-6f * (a + __builtin_fabsf(b2) + c), !(a > 1e-12f && c > 1e-12f)};
+}
+
+__device__ __forceinline__ bool quadrantReach(const ReachConic& k, float cutoff, float lox, float loy, float hix,
+                                              float hiy) {
+    const float nx = __builtin_amdgcn_fmed3f(0.0f, lox, hix), ny = __builtin_amdgcn_fmed3f(0.0f, loy, hiy);
+    const float y = __builtin_amdgcn_fmed3f(k.yOfX * nx, loy, hiy);
+    const float x = __builtin_amdgcn_fmed3f(k.xOfY * ny, lox, hix);
+    const float onX = __builtin_fmaf(k.a * nx, nx, y * __builtin_fmaf(k.b2, nx, k.c * y));
+    const float onY = __builtin_fmaf(k.a * x, x, ny * __builtin_fmaf(k.b2, x, k.c * ny));
+    const float r = __builtin_fmaxf(__builtin_fabsf(nx), __builtin_fabsf(ny)) + 8.0f;   // no coordinate is further
+    const float slack = __builtin_fmaf(k.size * r, r, __builtin_fmaf(1e-5f, cutoff, 1e-6f));
+    return k.degenerate | (__builtin_fminf(onX, onY) <= cutoff + slack);
 }
 
 // Does tile (tx, ty), 1 << tileShift pixels square, hold a pixel centre inside

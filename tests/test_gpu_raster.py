@@ -417,3 +417,36 @@ def test_a_frame_of_one_pair_draws_it(rast, tile):
     H.assert_bit_exact(gpu, ora)
     assert ora["colour"].max() > 0.1
     np.testing.assert_allclose(gpu["colour"], ora["colour"], rtol=0, atol=2e-5)
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+@pytest.mark.parametrize("count", [1, 3, 15, 17, 63, 65, 255, 257, 769])
+@pytest.mark.parametrize("opacity,depth_mode", [(0.02, 0), (0.6, 0), (0.6, 1)])
+def test_lists_of_every_length_blend_as_the_oracle(rast, count, tile, opacity, depth_mode):
+    """The ends of the blend's groups of four records, sixteens, chunks of 64 and
+    rounds of a pair a lane, on a frame whose last blocks have pixels past both
+    edges; faint splats (no pixel stops) and strong ones (pixels stop at every
+    place of a group). Colours and depths are sums of at most `count` 32-bit
+    terms whose exponents are off by a few ulps of |q| <= 16 (2e-6 of a weight):
+    2e-5 of their size, and a pixel whose pair lies at its cutoff, its floor or
+    its last place may differ by that pair (1/255 of a weight at the floor)."""
+    rng = np.random.default_rng(count)
+    fields = np.zeros((count, 14), np.float32)
+    fields[:, 0] = rng.uniform(-0.35, 0.35, count)
+    fields[:, 1] = rng.uniform(-0.25, 0.25, count)
+    fields[:, 2] = rng.uniform(-1.0, 1.0, count)
+    fields[:, 3] = opacity
+    fields[:, 4:7] = rng.uniform(-4.0, -1.5, (count, 3))
+    fields[:, 7:11] = rng.normal(0.0, 1.0, (count, 4))
+    fields[:, 11:14] = rng.uniform(0.0, 1.0, (count, 3))
+    scene = scenes.pack_splats(fields, 0)
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=60.0)
+    s = raster.RenderSettings(width=37, height=27, tile_size=tile, depth_mode=depth_mode)
+    inst = [(scene, np.eye(4), raster.SplatEdit())]
+    gpu = H.run_gpu(cam, s, inst, rast)
+    ora = H.run_oracle(cam, s, inst)
+    H.assert_bit_exact(gpu, ora)
+    for name, scale in (("colour", 1.0), ("depth", 5.0)):
+        d = np.abs(gpu[name].astype(np.float64) - ora[name])
+        assert np.quantile(d, 0.97) <= 2e-5 * scale, (name, np.quantile(d, 0.97))
+        assert d.max() <= (1.0 if (name, depth_mode) == ("depth", 1) else scale / 255.0 * 2.0), (name, d.max())
