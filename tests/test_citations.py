@@ -96,7 +96,7 @@ def test_every_header_citation_is_registered():
     assert len(_citations()) >= 40
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="the reference sources are not present here")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "modules")), reason="the reference sources are not present here")
 def test_every_header_citation_names_its_symbol():
     wrong = []
     for header, number, cite, first, last in _citations():
