@@ -46,6 +46,21 @@ def sort_pass_bytes(pairs, passes, key_bits):
     return pairs * 24 * passes
 
 
+def pass_count(bits):
+    """A sort's passes over `bits` key bits: digits of 8, or of 9 where that saves one."""
+    return min(-(-bits // 8), -(-bits // 9)) if bits else 0
+
+
+def depth_first_bytes(pairs, visible, tiles, key_bits):
+    """(histogram bytes, pass bytes) of a frame that sorts its drawn splats by
+    depth first (u32 keys and slots: 8 bytes read for the counts' offsets and
+    histogram, 16 a pass) and its pairs by tile (u16 tiles and u32 slots, 12
+    bytes a pass)."""
+    tile_bits = bits_for(tiles)
+    return (2 * pairs + 4 * visible,
+            pairs * 12 * pass_count(tile_bits) + visible * (8 + 16 * pass_count(key_bits - tile_bits)))
+
+
 def bits_for(values):
     """The bits a key needs to tell `values` values apart (at least one)."""
     return max(1, (max(values, 1) - 1).bit_length())
@@ -552,6 +567,9 @@ def sort_stress_leg(torch, raster, scenes, _abi, reps):
     defined, defined_passes = defined_sort_bytes(pairs, tiles)
     pass_bytes = sort_pass_bytes(pairs, passes, st.key_bits)
     moved = pairs * 8 + pass_bytes   # the histogram reads every key once
+    if st.depth_sort_ms > 0.0:
+        hist_bytes, pass_bytes = depth_first_bytes(pairs, visible, tiles, st.key_bits)
+        moved = hist_bytes + pass_bytes
     # The sort at each digit width the library offers (the default above).
     by_radix = {}
     for radix in (8, 9, 10):

@@ -161,15 +161,18 @@ typedef struct {
     float* depth;
 } lrt_render_targets;
 
-/* render::FrameStats (TileRasterizer.h:120-126). depth_sort_ms is 0: one
- * 64-bit (tile, depth) sort replaces the reference's depth sort + tile sort
- * and is reported as tile_sort_ms. total_ms is the call's wall clock, as the
+/* render::FrameStats (TileRasterizer.h:120-126). One 64-bit (tile, depth) sort
+ * replaces the reference's depth sort + tile sort and is reported as
+ * tile_sort_ms, depth_sort_ms then 0; a frame of many pairs a splat sorts its
+ * drawn splats by depth first (depth_sort_ms, with time_stages) and its pairs
+ * by tile. total_ms is the call's wall clock, as the
  * reference's; the stage figures (with time_stages) are GPU time from HIP
  * events, counts_ms including the pair-count readback's wait. key_bits and
  * sort_passes (no counterpart in the reference) describe the frame's sort: its
  * virtual key is the tile id over the depth key (bits(view z) >> 7) less the
  * frame's least drawn one, in bitsFor(tiles) + bitsFor(depth-key range) bits,
- * eight a pass (a batch of views, which reads no counts back before its sort,
+ * eight a pass, or nine where that saves one; depth first, the depth field's
+ * passes and the tile field's (a batch of views, which reads no counts back before its sort,
  * bounds the depth keys by its views' least near and greatest far plane). */
 typedef struct {
     uint32_t splats, visible, pairs;

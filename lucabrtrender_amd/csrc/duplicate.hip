@@ -14,6 +14,10 @@
 // pair's own index in this slot-major order (and its slot goes to pairSlot):
 // after the sort each pair then knows where its splat's run of pairs lies, so
 // per-pair gradients written there sum per splat over contiguous runs.
+//
+// A frame of many pairs a slot duplicates its drawn slots in depth order
+// instead (duplicateOrdered): the keys are then the tiles alone, u16 where the
+// frame has no more than 65,536, and one stable sort by tile is enough.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -27,15 +31,15 @@ using namespace lrt::dev;
 constexpr uint32_t kBlock = 256;
 
 // Writes pair `at` of slot s, or counts it as past the capacity.
-template <bool EMIT_INDEX>
-__device__ __forceinline__ void emitPair(uint32_t at, uint64_t key, uint32_t s, uint64_t* __restrict__ keys,
+template <bool EMIT_INDEX, typename Key>
+__device__ __forceinline__ void emitPair(uint32_t at, uint32_t index, Key key, uint32_t s, Key* __restrict__ keys,
                                          uint32_t* __restrict__ values, uint32_t* __restrict__ pairSlot,
                                          uint32_t capacity, uint32_t* __restrict__ overflow) {
     if (at < capacity) {
         keys[at] = key;
         if constexpr (EMIT_INDEX) {
-            values[at] = at;
-            pairSlot[at] = s;
+            values[at] = index;
+            if constexpr (sizeof(Key) == 8) pairSlot[index] = s;   // (else fillPairSlots', in slot order)
         } else {
             values[at] = s;
         }
@@ -56,21 +60,26 @@ __device__ __forceinline__ void emitPair(uint32_t at, uint64_t key, uint32_t s, 
 // differ across lanes and travel with each candidate. With depthRange
 // non-null, a slot whose depth key (bits(z) >> 7) lies outside
 // [depthRange[0], depthRange[1]] is counted in *outOfRange.
-template <bool EMIT_INDEX, bool PER_VIEW>
-__device__ __forceinline__ void duplicateWave(uint32_t s, uint32_t expected, uint32_t width, uint32_t height,
+// `first` is the place of the slot's first pair. Key u64: the keys as above. A
+// narrower Key: the tile alone, for slots that come in depth order (not
+// consecutive), with EMIT_INDEX each with the slot-order index of its first
+// pair (`firstIndex`).
+template <bool EMIT_INDEX, bool PER_VIEW, typename Key>
+__device__ __forceinline__ void duplicateWave(uint32_t s, uint32_t expected, uint32_t first, uint32_t firstIndex,
+                                              uint32_t width, uint32_t height,
                                               uint32_t tilesX, uint32_t tileShift, uint32_t tileBase,
                                               const float4* __restrict__ proj,
-                                              const uint2* __restrict__ rects, const uint32_t* __restrict__ offsets,
-                                              uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
+                                              const uint2* __restrict__ rects,
+                                              Key* __restrict__ keys, uint32_t* __restrict__ values,
                                               uint32_t* __restrict__ pairSlot, uint32_t capacity,
                                               uint32_t* __restrict__ overflow,
                                               const uint32_t* __restrict__ depthRange,
                                               uint32_t* __restrict__ outOfRange) {
     const uint32_t lane = __lane_id();
-    uint32_t first = 0, x0 = 0, y0 = 0, w = 1, area = 0;
+    constexpr bool kOrdered = sizeof(Key) < 8;
+    uint32_t x0 = 0, y0 = 0, w = 1, area = 0;
     float4 screen = make_float4(0.0f, 0.0f, 0.0f, 0.0f), conic = screen;
     if (expected != 0) {
-        first = offsets[s];
         screen = proj[static_cast<uint64_t>(s) * 3];
         conic = proj[static_cast<uint64_t>(s) * 3 + 1];
         const uint2 rc = rects[s];
@@ -86,7 +95,7 @@ __device__ __forceinline__ void duplicateWave(uint32_t s, uint32_t expected, uin
     const WaveTiles wt = waveTiles(area);
     const bool exact = wt.total >= (1u << 20);
     const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t slotOfLane0 = s - lane;   // the wave's slots are consecutive
+    const uint32_t slotOfLane0 = s - lane;   // in slot order the wave's slots are consecutive
     uint32_t written = 0;                    // this lane's slot's pairs so far
     for (uint32_t base = 0; base < wt.total; base += 64) {
         const uint32_t cand = base + lane;
@@ -102,7 +111,13 @@ __device__ __forceinline__ void duplicateWave(uint32_t s, uint32_t expected, uin
             oBase = shflU(tileBase, o);
         }
         const uint32_t oFirst = shflU(first, o), oExpected = shflU(expected, o), oWritten = shflU(written, o);
-        const uint32_t oDepth = shflU(depthBits, o);
+        uint32_t oDepth = 0, oSlot = slotOfLane0 + o, oIndex = oFirst;
+        if constexpr (kOrdered) {
+            oSlot = shflU(s, o);
+            if constexpr (EMIT_INDEX) oIndex = shflU(firstIndex, o);
+        } else {
+            oDepth = shflU(depthBits, o);
+        }
         bool hit = false;
         uint32_t tx = 0, ty = 0;
         if (cand < wt.total) {
@@ -119,8 +134,15 @@ __device__ __forceinline__ void duplicateWave(uint32_t s, uint32_t expected, uin
             const uint64_t sameRunBelow = below & ~((1ull << runLo) - 1ull);
             const uint32_t place = oWritten + static_cast<uint32_t>(__popcll(vote & sameRunBelow));
             if (place < oExpected) {
-                const uint64_t key = (static_cast<uint64_t>(oBase + ty * oTilesX + tx) << 32) | oDepth;
-                emitPair<EMIT_INDEX>(oFirst + place, key, slotOfLane0 + o, keys, values, pairSlot, capacity, overflow);
+                const uint32_t tile = oBase + ty * oTilesX + tx;
+                Key key;
+                if constexpr (kOrdered) {
+                    key = static_cast<Key>(tile);
+                } else {
+                    key = (static_cast<uint64_t>(tile) << 32) | oDepth;
+                }
+                emitPair<EMIT_INDEX>(oFirst + place, oIndex + place, key, oSlot, keys, values, pairSlot, capacity,
+                                     overflow);
             }
         }
         written += static_cast<uint32_t>(__popcll(vote & runMask(wt.start, wt.area, base)));
@@ -141,8 +163,48 @@ __global__ __launch_bounds__(kBlock) void duplicateKernel(FrameParams f, uint32_
                                                           uint32_t* __restrict__ outOfRange) {
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
     const uint32_t expected = s < slots ? touched[s] : 0u;   // every lane stays for the wave's walk
-    duplicateWave<EMIT_INDEX, false>(s, expected, f.width, f.height, f.tilesX, f.tileShift, 0u, proj, rects, offsets,
-                                     keys, values, pairSlot, capacity, overflow, depthRange, outOfRange);
+    duplicateWave<EMIT_INDEX, false>(s, expected, expected != 0 ? offsets[s] : 0u, 0u, f.width, f.height, f.tilesX,
+                                     f.tileShift, 0u, proj, rects, keys, values, pairSlot, capacity, overflow,
+                                     depthRange, outOfRange);
+}
+
+// pairSlot[i] = s for every pair i of slot s in slot order: a wave's 64 slots'
+// pairs are one range, written 64 a round, each place's slot found among the
+// lanes' ends (the depth-ordered duplication would write each slot's few words
+// to a place of their own).
+__global__ __launch_bounds__(kBlock) void fillPairSlotsKernel(uint32_t slots, const uint32_t* __restrict__ touched,
+                                                              const uint32_t* __restrict__ offsets,
+                                                              uint32_t* __restrict__ pairSlot, uint32_t capacity) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t lane = __lane_id();
+    const WaveTiles wt = waveTiles(s < slots ? touched[s] : 0u);
+    if (wt.total == 0) return;   // uniform across the wave
+    const uint32_t first = offsets[s - lane];   // lane 0's slot: every later lane's pairs follow
+    for (uint32_t base = 0; base < wt.total; base += 64) {
+        const uint32_t o = ownerOf(wt.incl, base + lane);
+        const uint32_t at = first + base + lane;
+        if (base + lane < wt.total && at < capacity) pairSlot[at] = s - lane + o;
+    }
+}
+
+// The drawn slots in depth order: thread j takes order[j].
+template <bool EMIT_INDEX, typename Key>
+__global__ __launch_bounds__(kBlock) void duplicateOrderedKernel(
+    FrameParams f, uint32_t slots, uint32_t count, const uint32_t* __restrict__ order, const float4* __restrict__ proj,
+    const uint2* __restrict__ rects, const uint32_t* __restrict__ touched, const uint32_t* __restrict__ offsets,
+    const uint32_t* __restrict__ slotOffsets, Key* __restrict__ keys, uint32_t* __restrict__ values,
+    uint32_t capacity, uint32_t* __restrict__ overflow,
+    const uint32_t* __restrict__ depthRange, uint32_t* __restrict__ outOfRange) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t s = j < count ? order[j] : slots;
+    uint32_t expected = 0, first = 0, firstIndex = 0;
+    if (s < slots) {
+        expected = touched[s];
+        first = offsets[j];
+        if constexpr (EMIT_INDEX) firstIndex = slotOffsets[s];
+    }
+    duplicateWave<EMIT_INDEX, false>(s, expected, first, firstIndex, f.width, f.height, f.tilesX, f.tileShift, 0u, proj,
+                                     rects, keys, values, nullptr, capacity, overflow, depthRange, outOfRange);
 }
 
 // A batch of views: slot s belongs to view s / splatsPerView.
@@ -170,8 +232,9 @@ __global__ __launch_bounds__(kBlock) void duplicateViewsKernel(const ViewInfo* _
         tileBase = v.tileBase;
         if (outOfRange != nullptr) depthRange = &v.depthLo;   // depthLo, depthHi
     }
-    duplicateWave<EMIT_INDEX, true>(s, expected, width, height, tilesX, tileShift, tileBase, proj, rects, offsets, keys,
-                                    values, pairSlot, capacity, overflow, depthRange, outOfRange);
+    duplicateWave<EMIT_INDEX, true>(s, expected, expected != 0 ? offsets[s] : 0u,
+                                    expected != 0 ? offsets[s] : 0u, width, height, tilesX, tileShift, tileBase, proj,
+                                    rects, keys, values, pairSlot, capacity, overflow, depthRange, outOfRange);
 }
 
 }   // namespace
@@ -190,6 +253,34 @@ void duplicate(const FrameParams& f, uint32_t slots, const float4* proj, const u
                                                               nullptr, capacity, overflow, depthRange, outOfRange);
     }
 }
+
+template <typename Key>
+void duplicateOrdered(const FrameParams& f, uint32_t slots, uint32_t count, const uint32_t* order, const float4* proj,
+                      const uint2* rects, const uint32_t* touched, const uint32_t* offsets,
+                      const uint32_t* slotOffsets, Key* keys, uint32_t* values, uint32_t* pairSlot, uint32_t capacity,
+                      uint32_t* overflow, hipStream_t stream, const uint32_t* depthRange, uint32_t* outOfRange) {
+    if (count == 0) return;
+    const uint32_t blocks = (count + kBlock - 1) / kBlock;
+    if (pairSlot != nullptr) {
+        fillPairSlotsKernel<<<(slots + kBlock - 1) / kBlock, kBlock, 0, stream>>>(slots, touched, slotOffsets,
+                                                                                 pairSlot, capacity);
+        duplicateOrderedKernel<true, Key><<<blocks, kBlock, 0, stream>>>(f, slots, count, order, proj, rects, touched,
+                                                                        offsets, slotOffsets, keys, values, capacity,
+                                                                        overflow, depthRange, outOfRange);
+    } else {
+        duplicateOrderedKernel<false, Key><<<blocks, kBlock, 0, stream>>>(f, slots, count, order, proj, rects, touched,
+                                                                         offsets, nullptr, keys, values, capacity,
+                                                                         overflow, depthRange, outOfRange);
+    }
+}
+template void duplicateOrdered<uint16_t>(const FrameParams&, uint32_t, uint32_t, const uint32_t*, const float4*,
+                                         const uint2*, const uint32_t*, const uint32_t*, const uint32_t*, uint16_t*,
+                                         uint32_t*, uint32_t*, uint32_t, uint32_t*, hipStream_t, const uint32_t*,
+                                         uint32_t*);
+template void duplicateOrdered<uint32_t>(const FrameParams&, uint32_t, uint32_t, const uint32_t*, const float4*,
+                                         const uint2*, const uint32_t*, const uint32_t*, const uint32_t*, uint32_t*,
+                                         uint32_t*, uint32_t*, uint32_t, uint32_t*, hipStream_t, const uint32_t*,
+                                         uint32_t*);
 
 void duplicateViews(const ViewInfo* views, uint32_t splatsPerView, uint32_t tileShift, uint32_t slots,
                     const float4* proj,

@@ -32,9 +32,19 @@ inline uint64_t scanStatusWords(uint32_t n) { return uint64_t{scanPartitions(n)}
 void scanExclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint64_t* status, uint32_t* total,
                    uint32_t* nonzero, uint32_t* error, hipStream_t stream, const uint32_t* depthBlocks = nullptr,
                    uint32_t depthEntries = 0, uint32_t* depthRange = nullptr, uint32_t* alsoZero = nullptr,
-                   uint32_t alsoZeroWords = 0, bool zeroed = false);
+                   uint32_t alsoZeroWords = 0, bool zeroed = false, const uint32_t* index = nullptr);
+// (With index non-null element i is in[index[i]]; with nonzero null the
+// non-zero inputs are not counted and no depth range is folded.)
 // The u32 words of `status` a scan of n elements needs zeroed before it runs.
 inline uint32_t scanZeroWords(uint32_t n) { return scanPartitions(n) * 2; }
+
+// The drawn slots of a frame in slot order: keys[i] their depth keys less
+// depthMin, slots[i] the slots, for every slot with touched > 0. To run after
+// scanExclusive over touched[0, n) with the same status (whose counts of
+// non-zero inputs it turns into places), and then clears the first zeroWords
+// u32 words of status for a scan of the drawn slots.
+void compactDrawn(const uint32_t* touched, const float4* proj, uint32_t n, uint32_t depthMin, uint64_t* status,
+                  uint32_t* keys, uint32_t* slots, uint32_t zeroWords, hipStream_t stream);
 
 // Words a launch zeroes on the side (either span may be empty): a later
 // launch's look-back words and counters, cleared by one that runs anyway.
@@ -83,6 +93,16 @@ void duplicate(const FrameParams& f, uint32_t slots, const float4* proj, const u
                const uint32_t* touched, const uint32_t* offsets, uint64_t* keys, uint32_t* values,
                uint32_t* pairSlot, uint32_t capacity, uint32_t* overflow, hipStream_t stream,
                const uint32_t* depthRange = nullptr, uint32_t* outOfRange = nullptr);
+// The same in the order of `order` (count drawn slots, in depth order): order[j]'s
+// pairs go to offsets[j].., their keys the tile alone. With pairSlot non-null
+// the values are the pairs' indices in slot order, slotOffsets[slot].., and
+// pairSlot[index] the slot.
+template <typename Key>
+void duplicateOrdered(const FrameParams& f, uint32_t slots, uint32_t count, const uint32_t* order, const float4* proj,
+                      const uint2* rects, const uint32_t* touched, const uint32_t* offsets,
+                      const uint32_t* slotOffsets, Key* keys, uint32_t* values, uint32_t* pairSlot, uint32_t capacity,
+                      uint32_t* overflow, hipStream_t stream, const uint32_t* depthRange = nullptr,
+                      uint32_t* outOfRange = nullptr);
 // A batch of views (device ViewInfo array): slot s is view s / splatsPerView's,
 // its keys carry the view's tileBase; pairSlot as duplicate()'s. With
 // outOfRange non-null, a drawn slot whose depth key lies outside its view's
@@ -100,6 +120,8 @@ enum class KeyMode : uint32_t {
     TileDepth = 1,    // (key >> 32) << depthBits | ((key & 0x7FFFFFFF) >> 7) - depthMin:
                       // tile id over the top 24 bits of a positive float depth, less
                       // the frame's least; keyBits = tileBits + depthBits
+    Word32 = 2,       // a u32 key's low keyBits bits (sortWords)
+    Word16 = 3,       // a u16 key's (sortWords)
 };
 
 // TileDepth's depth field: the frame's depth keys lie in [depthMin, depthMin +
@@ -160,6 +182,13 @@ bool sortPairs(uint64_t* keys, uint32_t* values, uint64_t* keysAlt, uint32_t* va
                TileDepthLayout depth = {}, uint32_t* alsoZero = nullptr, uint64_t alsoZeroWords = 0,
                uint32_t radixBits = 0);
 
+// The same sort of u32 or u16 keys (bits 0 .. keyBits of them), their values
+// beside them; the workspace as sortPairs' for keyBits.
+template <typename Key>
+bool sortWords(Key* keys, uint32_t* values, Key* keysAlt, uint32_t* valuesAlt, uint32_t n, uint32_t keyBits,
+               const SortWorkspace& ws, hipStream_t stream, hipEvent_t afterHistogram = nullptr,
+               uint32_t* alsoZero = nullptr, uint64_t alsoZeroWords = 0, uint32_t radixBits = 0);
+
 // ---- load: raw splat records into packed splats --------------------------------
 // The decode's view of an io::SplatEncoding: field offsets in floats, modes
 // numbered as the encoding numbers them, the rest basis functions kept and the
@@ -192,8 +221,14 @@ void tileRanges(const uint64_t* keys, uint32_t pairs, uint32_t tiles, uint2* ran
 // The same over a narrowed sort's u32 keys: the tile is key >> tileShift.
 void tileRangesNarrow(const uint32_t* keys, uint32_t tileShift, uint32_t pairs, uint32_t tiles, uint2* ranges,
                       hipStream_t stream, const uint32_t* nDevice = nullptr, bool zeroed = false);
+// The same over u16 keys that are the tiles.
+void tileRangesWords(const uint16_t* keys, uint32_t pairs, uint32_t tiles, uint2* ranges, hipStream_t stream,
+                     bool zeroed = false);
 // u64 keys tile << 32 | bits(view z) rebuilt from a narrowed sort's u32 keys
-// and the pairs' slots (the view z read from each slot's record), for readback.
+// (or u16 tiles) and the pairs' slots (the view z read from each slot's
+// record), for readback.
+void widenKeys(const uint16_t* keys, const uint32_t* slots, const float4* proj, uint32_t pairs, uint64_t* out,
+               hipStream_t stream);
 void widenKeys(const uint32_t* keys, uint32_t tileShift, const uint32_t* slots, const float4* proj, uint32_t pairs,
                uint64_t* out, hipStream_t stream);
 

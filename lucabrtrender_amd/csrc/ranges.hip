@@ -24,9 +24,10 @@ __device__ __forceinline__ uint32_t fromLane(uint32_t v, uint32_t missing) {
 // key shifted right by tileShift.
 __device__ __forceinline__ uint32_t tileOf(uint64_t key, uint32_t) { return static_cast<uint32_t>(key >> 32); }
 __device__ __forceinline__ uint32_t tileOf(uint32_t key, uint32_t tileShift) { return key >> tileShift; }
+__device__ __forceinline__ uint32_t tileOf(uint16_t key, uint32_t) { return key; }
 
 // Thread g takes pairs [4g, 4g + 4) with 16-byte loads (two of u64 keys, one
-// of u32); the tile before its first pair and after its last come from the
+// of u32; one 8-byte load of u16); the tile before its first pair and after its last come from the
 // neighbouring lanes (DPP wave shifts), the wave's two end lanes loading
 // theirs. Keys must be 16-byte aligned (the rasteriser's sort buffers are).
 template <typename Key>
@@ -48,6 +49,12 @@ __global__ __launch_bounds__(kBlock) void rangesKernel(const Key* __restrict__ k
             t[1] = a.w;
             t[2] = b.y;
             t[3] = b.w;
+        } else if constexpr (sizeof(Key) == 2) {
+            const uint2 a = *reinterpret_cast<const uint2*>(keys + i0);
+            t[0] = a.x & 0xFFFFu;
+            t[1] = a.x >> 16;
+            t[2] = a.y & 0xFFFFu;
+            t[3] = a.y >> 16;
         } else {
             const uint4 a = *reinterpret_cast<const uint4*>(keys + i0);
             t[0] = a.x >> tileShift;
@@ -74,13 +81,14 @@ __global__ __launch_bounds__(kBlock) void rangesKernel(const Key* __restrict__ k
     }
 }
 
-__global__ __launch_bounds__(kBlock) void widenKeysKernel(const uint32_t* __restrict__ keys, uint32_t tileShift,
+template <typename Key>
+__global__ __launch_bounds__(kBlock) void widenKeysKernel(const Key* __restrict__ keys, uint32_t tileShift,
                                                           const uint32_t* __restrict__ slots,
                                                           const float4* __restrict__ proj, uint32_t pairs,
                                                           uint64_t* __restrict__ out) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= pairs) return;
-    const uint64_t tile = keys[i] >> tileShift;
+    const uint64_t tile = tileOf(keys[i], tileShift);
     const float z = proj[static_cast<uint64_t>(slots[i]) * 3].z;
     out[i] = tile << 32 | __float_as_uint(z);
 }
@@ -112,7 +120,18 @@ void tileRangesNarrow(const uint32_t* keys, uint32_t tileShift, uint32_t pairs, 
 void widenKeys(const uint32_t* keys, uint32_t tileShift, const uint32_t* slots, const float4* proj, uint32_t pairs,
                uint64_t* out, hipStream_t stream) {
     if (pairs == 0) return;
-    widenKeysKernel<<<(pairs + kBlock - 1) / kBlock, kBlock, 0, stream>>>(keys, tileShift, slots, proj, pairs, out);
+    widenKeysKernel<uint32_t><<<(pairs + kBlock - 1) / kBlock, kBlock, 0, stream>>>(keys, tileShift, slots, proj, pairs, out);
+}
+
+void widenKeys(const uint16_t* keys, const uint32_t* slots, const float4* proj, uint32_t pairs, uint64_t* out,
+               hipStream_t stream) {
+    if (pairs == 0) return;
+    widenKeysKernel<uint16_t><<<(pairs + kBlock - 1) / kBlock, kBlock, 0, stream>>>(keys, 0u, slots, proj, pairs, out);
+}
+
+void tileRangesWords(const uint16_t* keys, uint32_t pairs, uint32_t tiles, uint2* ranges, hipStream_t stream,
+                     bool zeroed) {
+    launchRanges(keys, 0u, pairs, tiles, ranges, stream, nullptr, zeroed);
 }
 
 }   // namespace lrt::kern

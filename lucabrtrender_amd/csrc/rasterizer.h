@@ -273,6 +273,13 @@ private:
     // (the composite blend when `composite`, over `under` when non-null).
     // scanZeroed: the projection already cleared the scan's look-back words
     // and the counters.
+    // A frame's pairs binned depth first (finishFrame): the drawn slots sorted by
+    // depth, duplicated in that order, the pairs sorted by tile, the ranges.
+    // Returns whether the sorted pairs are in the second pair of buffers.
+    template <typename Workspace>
+    bool binDepthFirst(const FrameParams& first, uint32_t slots, uint32_t drawn, uint32_t pairs,
+                       const kern::TileDepthLayout& layout, const RenderSettings& settings, bool training,
+                       const Workspace& workspace);
     Status finishFrame(const FrameParams& first, uint32_t splatCount, const RenderSettings& settings,
                        RenderTargets& targets, FrameStats* stats, bool training, bool composite = false,
                        const RenderTargets* under = nullptr, bool scanZeroed = false);
@@ -311,7 +318,7 @@ private:
     // of the frame's drawn slots, [10] drawn slots outside that range.
     DeviceBuffer counters_;
     uint32_t* hostCounters_ = nullptr;   // pinned
-    hipEvent_t events_[9] = {};
+    hipEvent_t events_[11] = {};
     hipEvent_t countsCopied_ = nullptr;   // the pair-count readback has landed (no timing)
     // GPU milliseconds of the last timed render: project, scan, duplicate, sort
     // histogram, sort passes, ranges (with the heaviest-first ordering), blend, their sum.
@@ -323,7 +330,9 @@ private:
     bool lastWalkDropped_ = false;   // the last frame kept no per-pixel walk state
     uint64_t lastPixels_ = 0;
     int lastSorted_ = 0;   // which of keys_/values_ hold the sorted pairs
-    bool lastNarrow_ = false;       // the sorted keys are u32 (kern::sortNarrows)
+    bool lastNarrow_ = false;       // the sorted keys are u32 (kern::sortNarrows) or
+    bool lastTiles16_ = false;      // u16 tiles
+    bool depthFirst_ = false;       // the last frame's counts asked for the depth sort first
     uint32_t lastTileShift_ = 0;    // their tile is key >> lastTileShift_
     bool lastSlotsSorted_ = false;  // the sorted values are pair indices (their slots: pairSlot_)
     // The last plain (one view, splats only, not split) blend's launch, for

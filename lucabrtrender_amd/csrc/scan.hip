@@ -60,7 +60,7 @@ __global__ __launch_bounds__(kBlock) void scanKernel(const uint32_t* __restrict_
                                                      uint32_t n, uint64_t* __restrict__ status,
                                                      uint32_t* __restrict__ total,
                                                      uint32_t* __restrict__ nonzeroParts, uint32_t* __restrict__ error,
-                                                     bool vectorised) {
+                                                     bool vectorised, const uint32_t* __restrict__ index) {
     __shared__ uint32_t sWave[kBlock / 64];
     __shared__ uint32_t sNonzero[kBlock / 64];
     __shared__ uint32_t sPrefix;
@@ -71,7 +71,13 @@ __global__ __launch_bounds__(kBlock) void scanKernel(const uint32_t* __restrict_
     const uint64_t first = static_cast<uint64_t>(part) * kPart + static_cast<uint64_t>(tid) * kItems;
 
     uint32_t v[kItems];
-    if (vectorised && first + kItems <= n) {
+    if (index != nullptr) {
+        uint32_t at[kItems];
+#pragma unroll
+        for (uint32_t j = 0; j < kItems; ++j) at[j] = first + j < n ? index[first + j] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kItems; ++j) v[j] = first + j < n ? in[at[j]] : 0u;
+    } else if (vectorised && first + kItems <= n) {
         const uint4* src = reinterpret_cast<const uint4*>(in + first);
 #pragma unroll
         for (uint32_t q = 0; q < kItems / 4; ++q) {
@@ -234,7 +240,82 @@ __global__ __launch_bounds__(1024) void sumPartsKernel(const uint32_t* __restric
     }
 }
 
+// One workgroup: the partitions' non-zero counts turned into exclusive sums.
+__global__ __launch_bounds__(1024) void placePartsKernel(uint32_t* __restrict__ parts, uint32_t count) {
+    __shared__ uint32_t sWave[1024 / 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < count; base += 1024) {
+        const uint32_t i = base + threadIdx.x;
+        const uint32_t x = i < count ? parts[i] : 0u;
+        const uint32_t inclusive = waveInclusiveScan(x, lane);
+        if (lane == 63) sWave[wave] = inclusive;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < 1024 / 64; ++w) {
+            before += w < wave ? sWave[w] : 0u;
+            all += sWave[w];
+        }
+        if (i < count) parts[i] = carry + before + inclusive - x;
+        carry += all;
+        __syncthreads();   // the waves' sums are read
+    }
+}
+
+// A workgroup a scan partition: its drawn slots in order, from the place
+// placePartsKernel gave it. Round j of a thread is slot j * kBlock + tid of the
+// partition, so loads and stores are coalesced; a slot's place is its round's
+// and wave's (counts in LDS) plus its rank among the wave's drawn lanes.
+__global__ __launch_bounds__(kBlock) void compactDrawnKernel(const uint32_t* __restrict__ touched,
+                                                             const float4* __restrict__ proj, uint32_t n,
+                                                             uint32_t depthMin, const uint32_t* __restrict__ parts,
+                                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ slots,
+                                                             uint32_t* __restrict__ clear, uint32_t clearWords) {
+    __shared__ uint32_t sCount[kItems * (kBlock / 64)];
+    for (uint32_t w = blockIdx.x * kBlock + threadIdx.x; w < clearWords; w += gridDim.x * kBlock) clear[w] = 0u;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * kPart + threadIdx.x;
+    uint64_t votes[kItems];
+    uint32_t t[kItems];
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j) t[j] = first + j * kBlock < n ? touched[first + j * kBlock] : 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j) {
+        votes[j] = __ballot(t[j] != 0u);
+        if (lane == 0) sCount[j * (kBlock / 64) + wave] = static_cast<uint32_t>(__popcll(votes[j]));
+    }
+    __syncthreads();
+    if (wave == 0) {
+        static_assert(kItems * (kBlock / 64) == 64, "one wave scans the counts");
+        const uint32_t x = sCount[lane];
+        sCount[lane] = waveInclusiveScan(x, lane) - x;
+    }
+    __syncthreads();
+    const uint32_t base = parts[blockIdx.x];
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j) {
+        if (t[j] != 0u) {
+            const uint64_t slot = first + j * kBlock;
+            const uint32_t to = base + sCount[j * (kBlock / 64) + wave] +
+                                static_cast<uint32_t>(__popcll(votes[j] & ((1ull << lane) - 1ull)));
+            keys[to] = ((__float_as_uint(proj[slot * 3].z) & 0x7FFFFFFFu) >> 7) - depthMin;
+            slots[to] = static_cast<uint32_t>(slot);
+        }
+    }
+}
+
 }   // namespace
+
+void compactDrawn(const uint32_t* touched, const float4* proj, uint32_t n, uint32_t depthMin, uint64_t* status,
+                  uint32_t* keys, uint32_t* slots, uint32_t zeroWords, hipStream_t stream) {
+    const uint32_t parts = scanPartitions(n);
+    if (parts == 0) return;
+    uint32_t* nonzeroParts = reinterpret_cast<uint32_t*>(status + parts);
+    placePartsKernel<<<1, 1024, 0, stream>>>(nonzeroParts, parts);
+    compactDrawnKernel<<<parts, kBlock, 0, stream>>>(touched, proj, n, depthMin, nonzeroParts, keys, slots,
+                                                     reinterpret_cast<uint32_t*>(status), zeroWords);
+}
 
 void fill32(uint32_t* dst, uint32_t value, uint64_t count, hipStream_t stream) {
     if (count == 0) return;
@@ -292,7 +373,7 @@ hipError_t scanExclusiveStatic(const uint32_t* in, uint32_t* out, uint32_t n, ui
 void scanExclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint64_t* status, uint32_t* total,
                    uint32_t* nonzero, uint32_t* error, hipStream_t stream, const uint32_t* depthBlocks,
                    uint32_t depthEntries, uint32_t* depthRange, uint32_t* alsoZero, uint32_t alsoZeroWords,
-                   bool zeroed) {
+                   bool zeroed, const uint32_t* index) {
     const uint32_t parts = scanPartitions(n);
     if (const uint64_t words = static_cast<uint64_t>(parts) * 2 + alsoZeroWords; words > 0 && !zeroed) {
         // (an empty scan with nothing else to clear launches nothing: a grid of 0 is an error)
@@ -302,7 +383,7 @@ void scanExclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint64_t* stat
     }
     if (n == 0) {
         fill32(total, 0u, 1, stream);
-        fill32(nonzero, 0u, 1, stream);
+        if (nonzero != nullptr) fill32(nonzero, 0u, 1, stream);
         if (depthRange != nullptr) {
             fill32(depthRange, 0xFFFFFFFFu, 1, stream);
             fill32(depthRange + 1, 0u, 1, stream);
@@ -313,7 +394,8 @@ void scanExclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint64_t* stat
     uint32_t* nonzeroParts = reinterpret_cast<uint32_t*>(status + parts);
     // 16-byte loads and stores only where both arrays allow them.
     const bool vectorised = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && (reinterpret_cast<uintptr_t>(out) % 16 == 0);
-    scanKernel<<<parts, kBlock, 0, stream>>>(in, out, n, status, total, nonzeroParts, error, vectorised);
+    scanKernel<<<parts, kBlock, 0, stream>>>(in, out, n, status, total, nonzeroParts, error, vectorised, index);
+    if (nonzero == nullptr) return;
     sumPartsKernel<<<1, 1024, 0, stream>>>(nonzeroParts, parts, nonzero,
                                            reinterpret_cast<const uint2*>(depthBlocks), depthEntries, depthRange);
 }

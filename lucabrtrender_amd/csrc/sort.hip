@@ -93,12 +93,17 @@ __device__ __forceinline__ uint64_t tileDepthKey(uint64_t key, uint32_t depthMin
     return ((key >> 32) << depthBits) | depth;
 }
 
+// The type of the keys a mode sorts.
 template <KeyMode MODE>
-__device__ __forceinline__ uint64_t sortKey(uint64_t key, uint32_t bitLo, uint64_t mask, TileDepthLayout depth) {
+using KeyOf = std::conditional_t<MODE == KeyMode::Word32, uint32_t,
+                                 std::conditional_t<MODE == KeyMode::Word16, uint16_t, uint64_t>>;
+
+template <KeyMode MODE>
+__device__ __forceinline__ uint64_t sortKey(KeyOf<MODE> key, uint32_t bitLo, uint64_t mask, TileDepthLayout depth) {
     if constexpr (MODE == KeyMode::TileDepth) {
         return tileDepthKey(key, depth.depthMin, depth.depthBits) & mask;
     } else {
-        return (key >> bitLo) & mask;
+        return (static_cast<uint64_t>(key) >> bitLo) & mask;
     }
 }
 
@@ -111,7 +116,7 @@ __device__ __forceinline__ uint64_t sortKey(uint64_t key, uint32_t bitLo, uint64
 // costs two LDS atomics whatever its length, and no lane searches for the
 // run's end.
 template <KeyMode MODE>
-__global__ __launch_bounds__(kHistBlock) void histogramKernel(const uint64_t* __restrict__ keys, uint32_t cap,
+__global__ __launch_bounds__(kHistBlock) void histogramKernel(const KeyOf<MODE>* __restrict__ keys, uint32_t cap,
                                                               const uint32_t* __restrict__ nDevice, uint32_t bitLo,
                                                               uint64_t mask, TileDepthLayout depth, HistPlan plan,
                                                               uint32_t* __restrict__ hist,
@@ -242,10 +247,11 @@ __global__ __launch_bounds__(1024) void digitOffsetsKernel(const uint32_t* __res
 //   TileNarrow:   u64 in (the duplication's keys), u32 out: the virtual key
 //                 shifted right by `narrow` (its low `narrow` bits are this
 //                 pass's, consumed once it is done); the digit as TileDepth64's.
-//   Narrow32:     u32 in and out (TileNarrow's output); the digit is bits
-//                 [shift, +width) of the stored key.
+//   Narrow32:     u32 in and out (TileNarrow's output, or Word32 keys); the
+//                 digit is bits [shift, +width) of the stored key.
+//   Plain16:      u16 in and out, the same.
 // `mask` holds the digit's width in ones.
-enum class PassKind : uint32_t { Plain64, TileDepth64, TileNarrow, Narrow32 };
+enum class PassKind : uint32_t { Plain64, TileDepth64, TileNarrow, Narrow32, Plain16 };
 
 struct PassDigit {
     uint32_t shift;
@@ -256,8 +262,9 @@ struct PassDigit {
 
 template <PassKind K>
 struct PassKeys {
-    using In = std::conditional_t<K == PassKind::Narrow32, uint32_t, uint64_t>;
-    using Out = std::conditional_t<K == PassKind::TileNarrow || K == PassKind::Narrow32, uint32_t, uint64_t>;
+    using Wide = std::conditional_t<K == PassKind::Plain16, uint16_t, uint64_t>;
+    using In = std::conditional_t<K == PassKind::Narrow32, uint32_t, Wide>;
+    using Out = std::conditional_t<K == PassKind::TileNarrow || K == PassKind::Narrow32, uint32_t, Wide>;
 };
 
 // The digit of an input key and the key as the pass writes it.
@@ -563,7 +570,7 @@ void launchPass(uint32_t tableBits, uint32_t parts, hipStream_t stream, const vo
 }
 
 template <KeyMode MODE>
-void launchPasses(uint64_t* keys, uint32_t* values, uint64_t* keysAlt, uint32_t* valuesAlt, uint32_t n,
+void launchPasses(KeyOf<MODE>* keys, uint32_t* values, KeyOf<MODE>* keysAlt, uint32_t* valuesAlt, uint32_t n,
                   const uint32_t* nDevice, uint32_t bitLo, uint32_t keyBits, const SortPlan& plan,
                   TileDepthLayout depth, const SortWorkspace& ws, hipStream_t stream, hipEvent_t afterHistogram,
                   uint32_t* alsoZero, uint64_t alsoZeroWords) {
@@ -597,7 +604,13 @@ void launchPasses(uint64_t* keys, uint32_t* values, uint64_t* keysAlt, uint32_t*
         const uint32_t* offsets = ws.offsets + plan.bins[p];
         uint32_t* status = ws.status + uint64_t{parts} * plan.bins[p];
         const uint32_t tb = hp.tableBits[p];
-        if constexpr (MODE == KeyMode::Plain) {
+        if constexpr (MODE == KeyMode::Word32) {
+            launchPass<PassKind::Narrow32>(tb, parts, stream, kin, vin, kout, vout, n, nDevice, pd, offsets, status,
+                                           ws.error);
+        } else if constexpr (MODE == KeyMode::Word16) {
+            launchPass<PassKind::Plain16>(tb, parts, stream, kin, vin, kout, vout, n, nDevice, pd, offsets, status,
+                                          ws.error);
+        } else if constexpr (MODE == KeyMode::Plain) {
             pd.shift = bitLo + plan.shift[p];
             launchPass<PassKind::Plain64>(tb, parts, stream, kin, vin, kout, vout, n, nDevice, pd, offsets, status,
                                           ws.error);
@@ -690,5 +703,25 @@ bool sortPairs(uint64_t* keys, uint32_t* values, uint64_t* keysAlt, uint32_t* va
     }
     return (plan.passes & 1u) != 0u;
 }
+
+template <typename Key>
+bool sortWords(Key* keys, uint32_t* values, Key* keysAlt, uint32_t* valuesAlt, uint32_t n, uint32_t keyBits,
+               const SortWorkspace& ws, hipStream_t stream, hipEvent_t afterHistogram, uint32_t* alsoZero,
+               uint64_t alsoZeroWords, uint32_t radixBits) {
+    if (n < 2 || keyBits == 0) {
+        if (alsoZero != nullptr) fill32(alsoZero, 0u, alsoZeroWords, stream);
+        if (afterHistogram != nullptr) (void)hipEventRecord(afterHistogram, stream);
+        return false;
+    }
+    constexpr KeyMode kMode = sizeof(Key) == 2 ? KeyMode::Word16 : KeyMode::Word32;
+    const SortPlan plan = sortPlan(keyBits, radixBits);
+    launchPasses<kMode>(keys, values, keysAlt, valuesAlt, n, nullptr, 0, keyBits, plan, {}, ws, stream, afterHistogram,
+                        alsoZero, alsoZeroWords);
+    return (plan.passes & 1u) != 0u;
+}
+template bool sortWords<uint32_t>(uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t, uint32_t, const SortWorkspace&,
+                                  hipStream_t, hipEvent_t, uint32_t*, uint64_t, uint32_t);
+template bool sortWords<uint16_t>(uint16_t*, uint32_t*, uint16_t*, uint32_t*, uint32_t, uint32_t, const SortWorkspace&,
+                                  hipStream_t, hipEvent_t, uint32_t*, uint64_t, uint32_t);
 
 }   // namespace lrt::kern

@@ -311,7 +311,7 @@ class FrameStats:
     blend_ms: float = 0.0
     total_ms: float = 0.0
     key_bits: int = 0       # the sort's virtual key: tile bits + the frame's depth-key range bits
-    sort_passes: int = 0    # eight key bits a pass
+    sort_passes: int = 0    # its passes (depth first: the depth field's and the tile field's)
 
 
 class RenderTargets:

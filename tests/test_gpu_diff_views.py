@@ -202,3 +202,37 @@ def test_a_batch_backward_needs_a_batch():
     with pytest.raises(LrtError) as err:
         rast.backward_views(gcols, grads)                  # the batch backward after a single frame
     assert err.value.code == 3
+
+
+def test_a_frame_binned_depth_first_has_the_batch_of_ones_gradients():
+    """A training frame past the pair count where the slots are sorted by depth
+    first, against a batch of that one view (which sorts its pairs once): the
+    image and every gradient bit for bit."""
+    import torch
+
+    from lucabrtrender_amd import autograd, raster, scenes
+    count, width, height = 50_011, 1920, 1080
+    p = scenes.diff_params(count, seed=5, degree=1, log_scale=(-2.7, 0.3))
+    cam = raster.Camera.looking_at((0.0, 0.0, 0.0), (0.0, 0.0, -1.0))
+    cam.lens = raster.Lens(focal=30.0)
+    settings = raster.RenderSettings(width=width, height=height)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    grad = torch.randn((height, width, 4), generator=g, device="cuda")
+    names = ("means", "log_scales", "quats", "opacity_logits", "sh")
+
+    def leaves():
+        return [torch.from_numpy(p[k]).cuda().requires_grad_() for k in names]
+
+    rast = raster.TileRasterizer()
+    a, b = leaves(), leaves()
+    for _ in range(2):
+        one = autograd.rasterize(*a, rast, cam, settings)
+        got = torch.autograd.grad(one, a, grad)
+    st = rast.render_diff(cam, raster.DiffSplats(*[t.detach() for t in a]), settings,
+                          raster.RenderTargets(width, height))
+    assert st.pairs > 6_000_000 + 4 * st.visible, st
+    (batch,) = autograd.rasterize_views(*b, raster.TileRasterizer(), [cam], [(width, height)], settings)
+    want = torch.autograd.grad(batch, b, grad)
+    assert torch.equal(one, batch)
+    for name, x, y in zip(names, got, want):
+        assert torch.equal(x, y), name

@@ -450,3 +450,57 @@ def test_lists_of_every_length_blend_as_the_oracle(rast, count, tile, opacity, d
         d = np.abs(gpu[name].astype(np.float64) - ora[name])
         assert np.quantile(d, 0.97) <= 2e-5 * scale, (name, np.quantile(d, 0.97))
         assert d.max() <= (1.0 if (name, depth_mode) == ("depth", 1) else scale / 255.0 * 2.0), (name, d.max())
+
+
+def _broad_splats(count, seed, log_scale):
+    """Splats wide enough to reach hundreds of tiles each, their depths spread
+    with some equal (ties that the slot order breaks)."""
+    rng = np.random.default_rng(seed)
+    fields = np.zeros((count, 14), np.float32)
+    fields[:, :2] = rng.uniform(-1.2, 1.2, (count, 2))
+    fields[:, 2] = np.round(rng.uniform(-1.0, 1.0, count) * 300.0) / 300.0
+    fields[:, 3] = rng.uniform(0.02, 0.9, count)
+    fields[:, 4:7] = rng.normal(log_scale, 0.3, (count, 3))
+    fields[:, 7:11] = rng.normal(0.0, 1.0, (count, 4))
+    fields[:, 11:14] = rng.uniform(0.0, 1.0, (count, 3))
+    return scenes.pack_splats(fields, 0)
+
+
+@pytest.mark.parametrize("size,tile,count,log_scale,discs", [((1920, 1080), 16, 60_011, -2.7, 0),
+                                                            ((1923, 1077), 32, 250_001, -2.7, 0),
+                                                            ((3840, 2160), 8, 2_003, -2.4, 0),
+                                                            ((1920, 1080), 16, 60_011, -2.7, 3_000)])
+def test_frames_of_many_pairs_a_splat_bin_as_the_oracle(size, tile, count, log_scale, discs):
+    """Past the pair count where the slots are sorted by depth first and the pairs
+    by tile alone: u16 tiles, u32 tiles (more than 65,536), discs among the
+    splats. Pairs, ranges and images are the one sort's; the first frame, the
+    same again (whose duplication waits for the counts) and one of few pairs
+    after it (whose duplication does not)."""
+    rast = raster.TileRasterizer()
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=30.0)
+    s = raster.RenderSettings(width=size[0], height=size[1], tile_size=tile)
+    inst = [(_broad_splats(count, 3, log_scale), np.eye(4), raster.SplatEdit())]
+    points = []
+    if discs:
+        pos, col = F.random_points(discs, 5)
+        points = [(pos, col, np.eye(4), raster.PointStyle(size=0.05))]
+        ora = H.run_oracle_composite(cam, s, inst, points)
+    else:
+        ora = H.run_oracle(cam, s, inst)
+    assert ora["pairs"] > 6_000_000 + 1.25 * ora["visible"]
+    for _ in range(2):
+        if discs:
+            gpu = H.run_gpu_composite(cam, s, inst, points, rast=rast)
+        else:
+            gpu = H.run_gpu(cam, s, inst, rast)
+        assert gpu["stats"].pairs == ora["pairs"] and gpu["stats"].key_bits == H.expected_key_bits(ora)
+        depth_bits = gpu["stats"].key_bits - H.bits_for(len(ora["ranges"]))
+        assert gpu["stats"].sort_passes == (H.expected_passes(depth_bits)
+                                            + H.expected_passes(H.bits_for(len(ora["ranges"]))))
+        H.assert_bit_exact(dict(gpu, stats=None), ora)
+        d = np.abs(gpu["colour"].astype(np.float64) - ora["colour"])
+        assert np.quantile(d, 0.99) <= 1e-3 and d.max() <= 1e-2   # the image targets of every frame test
+    few = raster.RenderSettings(width=250, height=190, tile_size=tile)
+    small = [(_broad_splats(500, 4, -3.5), np.eye(4), raster.SplatEdit())]
+    for _ in range(2):
+        H.assert_bit_exact(H.run_gpu(cam, few, small, rast), H.run_oracle(cam, few, small))
