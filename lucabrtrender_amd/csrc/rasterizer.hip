@@ -1156,9 +1156,10 @@ Status TileRasterizer::backward(const float4* gradColour, const kern::DiffGrads&
     }
     Status s = check(hipSetDevice(device_), "hipSetDevice");
     if (!s.ok()) return s;
-    if (!(s = pairGrad_.reserve(uint64_t{std::max(pairCapacity_, 1u)} * kern::kPairGradBytes, "pair.grad")).ok()) return s;
+    if (!(s = pairGrad_.reserve(kern::pairGradBytes(std::max(pairCapacity_, 1u)), "pair.grad")).ok()) return s;
     const kern::PairGrads pairGrads = kern::pairGradsIn(pairGrad_.get(), std::max(pairCapacity_, 1u));
     if (millis != nullptr) (void)hipEventRecord(events_[0], stream_);
+    kern::fill32(pairGrads.live, 0u, kern::pairLiveWords(lastPairs_), stream_);
     // One view's tiles in raster order: neighbouring tiles share splats in L2,
     // and on a 1M-splat 720p frame that beat heaviest-first by about 10%.
     kern::blendBackward(diffFrame_, lastSplats_, ranges_.as<uint2>(), pairSlot_.as<uint32_t>(),
@@ -1196,7 +1197,7 @@ Status TileRasterizer::backwardViews(std::span<const float4* const> gradColours,
     }
     Status s = check(hipSetDevice(device_), "hipSetDevice");
     if (!s.ok()) return s;
-    if (!(s = pairGrad_.reserve(uint64_t{std::max(pairCapacity_, 1u)} * kern::kPairGradBytes, "pair.grad")).ok()) return s;
+    if (!(s = pairGrad_.reserve(kern::pairGradBytes(std::max(pairCapacity_, 1u)), "pair.grad")).ok()) return s;
     const kern::PairGrads pairGrads = kern::pairGradsIn(pairGrad_.get(), std::max(pairCapacity_, 1u));
     if (diffViews_ > gradPtrCapacity_) {
         if (hostGradPtrs_ != nullptr) (void)hipHostFree(hostGradPtrs_);
@@ -1216,6 +1217,7 @@ Status TileRasterizer::backwardViews(std::span<const float4* const> gradColours,
         return s;
     const auto* params = viewParams_.as<FrameParams>();
     if (millis != nullptr) (void)hipEventRecord(events_[0], stream_);
+    kern::fill32(pairGrads.live, 0u, kern::pairLiveWords(lastPairs_), stream_);
     // The batch's tiles heaviest first: a view of few, long tiles (a small view
     // close to the cloud) would otherwise finish alone at the end.
     kern::tileOrder(ranges_.as<uint2>(), lastTiles_, tileOrder_.as<uint32_t>(), stream_);

@@ -19,7 +19,7 @@ import pytest
 import torch
 
 import oracle_lib as O
-from lucabrtrender_amd import raster, scenes
+from lucabrtrender_amd import _abi, raster, scenes
 from lucabrtrender_amd.autograd import rasterize
 from lucabrtrender_amd._abi import LrtError
 from oracle import diff_oracle as D
@@ -97,6 +97,36 @@ def test_forward_and_gradients_against_the_fp64_oracle(rast, case):
         rel = np.linalg.norm(a - b) / np.linalg.norm(b)
         print(f"  {name:15s} relative error vs FP64 autodiff {rel:.2e}")
         assert rel < 1e-2, (name, rel)
+
+
+@pytest.mark.parametrize("log_scale,runs", [(-4.5, (1, 8)), (-2.2, (9, 64)), (0.0, (65, 165))])
+def test_runs_of_every_length_sum_to_the_fp64_oracles_gradients(rast, log_scale, runs):
+    """Splats over few tiles, over tens, and over more than 64 (a run of pairs a
+    splat: one lane's, or a row of lanes'), nearly opaque, so that splats, and
+    tiles of a splat, that nothing sees lie between those that are seen. The
+    bound is that of the frames above; a second backward gives the same bits
+    (no record is left of the first), and a splat that no pixel saw has none."""
+    n, width, height = 200, 240, 176
+    p = scenes.diff_params(n, 31, degree=3, log_scale=(log_scale, 0.4))
+    p["opacity_logits"] = np.ascontiguousarray(p["opacity_logits"] + np.float32(5.0))
+    s = raster.RenderSettings(width=width, height=height)
+    g = np.random.default_rng(7).normal(0.0, 1.0, (height, width, 4))
+    _, grads = _gpu_grads(rast, p, s, g)
+    touched = rast.debug(_abi.DEBUG_TOUCHED)[:n]
+    assert ((touched >= runs[0]) & (touched <= runs[1])).any(), np.unique(touched)
+    frame = _oracle_frame(s, n, 15)
+    ref = D.gradients(frame, p, g)
+    for name in GROUPS:
+        a, b = grads[name].astype(np.float64).reshape(-1), ref[name].reshape(-1)
+        rel = np.linalg.norm(a - b) / np.linalg.norm(b)
+        print(f"  runs {runs} {name:15s} relative error vs FP64 autodiff {rel:.2e}", flush=True)
+        assert rel < 1e-2, (name, rel)
+        assert not grads[name][touched == 0].any()
+    again = {k: torch.full_like(torch.from_numpy(v), 7.0).cuda() for k, v in grads.items()}
+    rast.backward(torch.from_numpy(np.ascontiguousarray(g, dtype=np.float32)).cuda(), again)
+    torch.cuda.synchronize()
+    for name in GROUPS:
+        np.testing.assert_array_equal(again[name].cpu().numpy().view(np.uint32), grads[name].view(np.uint32))
 
 
 def test_gradients_against_fp64_central_differences(rast):
