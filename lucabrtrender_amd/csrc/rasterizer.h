@@ -196,7 +196,7 @@ public:
     // its size). stats: the batch's totals.
     Status renderViews(std::span<const View> views, std::span<const SplatInstance> instances,
                        const RenderSettings& settings, FrameStats* stats);
-    // Times the batch under each launch choice (list length 128/256, grid or
+    // Times the batch under each launch choice (grid or
     // persistent blend, graph replay or not; the best of three runs each) and
     // leaves the fastest in `settings`; *ms gets its time.
     Status autotuneViews(std::span<const View> views, std::span<const SplatInstance> instances,
