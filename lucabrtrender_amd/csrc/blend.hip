@@ -16,10 +16,10 @@
 // cache accesses a launch against 7.5M, and half of the vector instructions,
 // on 3M splats at 1920x1080.
 // A record's Gaussian is expanded about the quadrant's centre and scaled to the
-// exponent's base 2, log2(opacity / 0.99) added: at a pixel (u, v) from the
+// exponent's base 2, log2(opacity) added: at a pixel (u, v) from the
 // centre q = A u^2 + B u v + C v^2 + D u + E v + F, the pixel is inside the
-// cutoff and above the alpha floor when q >= qmin, and alpha / 0.99 = min(1,
-// 2^q), the exponential's own output clamp. q differs from the direct form's
+// cutoff and above the alpha floor when q >= the record's bound, and alpha =
+// min(0.99, 2^q). q differs from the direct form's
 // scaled power by float rounding only (below 2e-4 on footprints from a quarter
 // pixel to 300 pixels wide, centres up to 3.5 sigma outside the quadrant).
 //
@@ -66,7 +66,6 @@ using namespace lrt::dev;
 constexpr uint32_t kLanes = 64;          // one wave: an 8x8 quadrant
 constexpr uint32_t kGroup = 4;           // list records walked per step
 constexpr float kAlphaMax = 0.99f;       // a splat's alpha at most (splat_blend.slang:66)
-constexpr float kLog2AlphaMax = -0.01449956969511508876f;
 constexpr float kExpScale = -0.72134752044448170368f;   // -log2(e) / 2
 constexpr float kLog2Floor = -7.99435343685885793775f;   // log2(1 / 255): alpha's floor
 
@@ -189,7 +188,7 @@ struct BlendShared {
     static constexpr uint32_t kRound = WAVES * kLanes;
     // The round's records, in pair order, the conic scaled to base 2:
     float4 at[2][kRound];       // centre.xy, A, B
-    float4 shape[2][kRound];    // C, log2(opacity / kAlphaMax), the least q that passes, 1 for a disc
+    float4 shape[2][kRound];    // C, what F adds to the form at the centre, the test's bound, 0
     float4 colour[2][kRound];   // rgb, view z
     // Composite: the largest view z of the record's wave's pairs up to it, kept or not, and each wave's.
     float reach[2][COMPOSITE ? kRound : 1];
@@ -198,8 +197,9 @@ struct BlendShared {
     uint8_t list[2][WAVES][kRound];
     uint32_t count[2][WAVES][WAVES];
     uint32_t done[2][WAVES];    // the wave's pixels all stopped before this round
-    // A wave's own: the least q (and the reach) of the chunk it walks, four records a vector.
-    float4 qmin[WAVES][kLanes / 4];
+    // A wave's own: of the chunk it walks, four records a vector, D, E, F, the
+    // test's bound (and the reach).
+    float4 chunk[WAVES][4][kLanes / 4];
     float4 chunkReach[WAVES][COMPOSITE ? kLanes / 4 : 1];
 };
 
@@ -236,15 +236,14 @@ __device__ __forceinline__ uint2 partOrigin(const FrameParams& f, uint32_t tile,
 
 using Vec4 = float __attribute__((ext_vector_type(4)));
 
-// A pixel's walk while it runs: accum holds rgb and the depth sum over
-// kAlphaMax (the weights it sums are T alpha / kAlphaMax). The pixel walks
-// while t >= kTMin; composite: a pixel that something behind stops leaves its
-// T in tStopped and t 0. lastIn, depthIn and opaqueIn: a record's place in the
-// chunk at hand (-1: none yet).
+// A pixel's walk while it runs: accum holds rgb and the depth sum. The pixel
+// walks while t >= kTMin; composite: a pixel that something behind stops leaves
+// its T in tStopped and t 0. lastIn, depthIn and opaqueIn: a record's place in
+// the chunk at hand (-1: none yet).
 struct WalkLane {
     Vec4 accum;
     float t, tStopped;
-    float depthT;   // the depth is found once T is at most this; below 0 once found
+    float depthAt;   // the depth is found once 1 - T is at least this; infinite once found
     int32_t lastIn, depthIn, opaqueIn;
 };
 constexpr float kTMin = 1e-4f;
@@ -252,26 +251,39 @@ constexpr float kTMin = 1e-4f;
 // matrix results stay in the vector registers (no copies from accumulators).
 constexpr uint32_t kWavesPerSimd = 4;
 
-// The form of records 4 G .. 4 G + 3 of sixteen at the lane's own pixel.
+// The form of records 4 G .. 4 G + 3 of sixteen at the lane's own pixel:
+// q = u (A u + (B v + D)) + (v (C v + E) + F), each step a fused multiply-add.
 //
-// Both of the walk's contractions run on the matrix cores, in f32, as sixteen
-// 4x4 blocks of four lanes a block (v_mfma_f32_4x4x1, one block's lanes of A
-// given to every block). The form: rows of records times columns of pixels,
-// six products of a coefficient and the pixel's monomial; lane l < 16 of
-// `form` holds record l's A .. F, block G's four lanes are records 4 G ..
-// 4 G + 3, and q[k] lands in the lane of its pixel. The colours: rows of
-// channels times columns of pixels, one product a record, summed into the
-// lane's own accum; lane l of `colour`: channel l & 3 of record l / 4. What
-// stays on the VALU is what is no contraction: the exponential, the tests and
-// T. A matrix product costs about 14 cycles of issue, as five FMAs, and does
-// the work of four (the form) or of four with their operands' LDS reads gone
-// (the colours): the LDS, not the FMAs, is what it relieves.
+// The walk's contractions run on the matrix cores, in f32, as sixteen 4x4
+// blocks of four lanes a block (v_mfma_f32_4x4x1, one block's lanes of A given
+// to every block): a product and a sum rounded once, bit for bit the fused
+// multiply-add. The form's three products of a coefficient and the pixel's u or
+// v: rows of records times columns of pixels; lane l < 16 of `form` holds record
+// l's A, B and C, block G's four lanes are records 4 G .. 4 G + 3, q[k] lands in
+// the lane of its pixel, and D, E and F (four records' a vector, one LDS read
+// each) start the sums. The two outer steps multiply by a sum of the pixel's
+// own and stay on the VALU. The colours: rows of channels times columns of
+// pixels, one product a record, summed into the lane's own accum; lane l of
+// `colour`: channel l & 3 of record l / 4. What stays on the VALU besides is
+// what is no contraction: the exponential, the tests and T.
+//
+// Every step rounds as the walk of one record after the other on FMAs does, so
+// a pair at its cutoff or at the alpha floor falls on the same side. (The six
+// terms as one sum of six products, all on the matrix cores, rounds otherwise:
+// about one pixel-pair in ten million fell the other way, a whole contribution
+// each. Frames took 1 to 2 % less time with it.)
 template <uint32_t G>
-__device__ __forceinline__ Vec4 formOf(const float form[6], const float mono[5]) {
-    Vec4 q = {0.0f, 0.0f, 0.0f, 0.0f};
-    q = __builtin_amdgcn_mfma_f32_4x4x1f32(form[5], 1.0f, q, 4, G, 0);
+__device__ __forceinline__ Vec4 formOf(const float form[3], float u, float v, const float4 (*chunk)[kLanes / 4],
+                                       uint32_t at) {
+    const float4 d = chunk[0][at + G], e = chunk[1][at + G], f = chunk[2][at + G];
+    Vec4 x = {d.x, d.y, d.z, d.w}, y = {e.x, e.y, e.z, e.w};
+    x = __builtin_amdgcn_mfma_f32_4x4x1f32(form[1], v, x, 4, G, 0);
+    y = __builtin_amdgcn_mfma_f32_4x4x1f32(form[2], v, y, 4, G, 0);
+    x = __builtin_amdgcn_mfma_f32_4x4x1f32(form[0], u, x, 4, G, 0);
+    const float f4[4] = {f.x, f.y, f.z, f.w};
+    Vec4 q;
 #pragma unroll
-    for (uint32_t m = 0; m < 5; ++m) q = __builtin_amdgcn_mfma_f32_4x4x1f32(form[4 - m], mono[4 - m], q, 4, G, 0);
+    for (uint32_t k = 0; k < 4; ++k) q[k] = __builtin_fmaf(u, x[k], __builtin_fmaf(v, y[k], f4[k]));
     return q;
 }
 
@@ -285,30 +297,37 @@ __device__ __forceinline__ Vec4 addColour(float colour, float weight, Vec4 accum
 // q. A wave's records are one serial chain through T, and a launch cannot end
 // before its longest tile's chain, so the chain is kept short: the four
 // weights are taken as if no pixel stopped among the first three records (a
-// product and an FMA a record on the chain), and a group in which one does is
+// product and a difference a record on the chain), and a group in which one does is
 // taken again with the test between the records. Both ways do the same
 // arithmetic for a pixel that does not stop.
 template <uint32_t DEPTH_MODE, bool COMPOSITE, bool TRACK, uint32_t G>
-__device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, float4 qmin4, float4 reach4,
+__device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, float4 bound4, float4 reach4,
                                           float stopZ, uint64_t discs, int32_t first) {
     constexpr uint32_t R0 = G * kGroup;
-    const float qmin[4] = {qmin4.x, qmin4.y, qmin4.z, qmin4.w};
+    const float bound[4] = {bound4.x, bound4.y, bound4.z, bound4.w};
     bool passes[4];   // inside the cutoff and above the alpha floor
-    float alpha[4];   // over kAlphaMax
+    bool inside[4];   // composite: inside the cutoff
+    float alpha[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        passes[k] = q[k] >= qmin[k];
-        // min(1, alpha / kAlphaMax): the exponential's own output clamp
-        const float scaled = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(q[k]), 0.0f, 1.0f);
-        alpha[k] = passes[k] ? scaled : 0.0f;
+        const float power2 = __builtin_amdgcn_exp2f(q[k]);
+        if constexpr (COMPOSITE) {
+            const float a = __builtin_fminf(kAlphaMax, bound[k] * power2);
+            inside[k] = q[k] >= 0.0f;
+            passes[k] = inside[k] & (a >= 1.0f / 255.0f);
+            alpha[k] = passes[k] ? a : 0.0f;
+        } else {
+            passes[k] = q[k] >= bound[k];
+            alpha[k] = passes[k] ? __builtin_fminf(kAlphaMax, power2) : 0.0f;
+        }
     }
     float weight[4];
     if constexpr (COMPOSITE) {
-        // A group with a disc, or that an under-layer ends in (padding has the
-        // least reach), goes record by record.
+        // A group with a disc, or that an under-layer ends in, goes record by
+        // record. The reach grows along the list (padding has the last one's),
+        // so a group's last says whether one of it ends a pixel's walk.
         const float reach[4] = {reach4.x, reach4.y, reach4.z, reach4.w};
-        const float most = fmaxS(fmaxS(reach[0], reach[1]), fmaxS(reach[2], reach[3]));
-        const bool ends = (w.t >= kTMin) & (most >= stopZ);
+        const bool ends = (w.t >= kTMin) & (reach[3] >= stopZ);
         const bool anyEnds = __ballot(ends) != 0;
         if (((discs >> R0) & 15u) != 0u || anyEnds) {
             const auto stop = [&](bool here) {
@@ -318,18 +337,19 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
 #pragma unroll
             for (uint32_t k = 0; k < 4; ++k) {
                 if (anyEnds) stop((w.t >= kTMin) & (reach[k] >= stopZ));
-                const bool ok = (w.t >= kTMin) & passes[k];
                 weight[k] = 0.0f;
                 if (((discs >> (R0 + k)) & 1u) != 0u) {   // uniform: a disc that reaches the pixel ends its walk
-                    w.opaqueIn = ok ? first + static_cast<int32_t>(R0 + k) : w.opaqueIn;
-                    stop(ok);
+                    const bool hit = (w.t >= kTMin) & inside[k];
+                    w.opaqueIn = hit ? first + static_cast<int32_t>(R0 + k) : w.opaqueIn;
+                    stop(hit);
                 } else {
+                    const bool ok = (w.t >= kTMin) & passes[k];
                     weight[k] = w.t * (ok ? alpha[k] : 0.0f);
-                    w.t = __builtin_fmaf(-kAlphaMax, weight[k], w.t);
+                    w.t = w.t - weight[k];
                     if constexpr (DEPTH_MODE == 1) {
-                        const bool at = ok & (w.t <= w.depthT);
+                        const bool at = ok & (1.0f - w.t >= w.depthAt);
                         w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
-                        w.depthT = at ? -1.0f : w.depthT;
+                        w.depthAt = at ? __builtin_inff() : w.depthAt;
                     }
                 }
             }
@@ -346,7 +366,7 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
         weight[k] = t[k] * alpha[k];
-        t[k + 1] = __builtin_fmaf(-kAlphaMax, weight[k], t[k]);   // T (1 - alpha)
+        t[k + 1] = t[k] - weight[k];   // T (1 - alpha)
     }
     bool ok[4];
 #pragma unroll
@@ -357,7 +377,7 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
             const bool here = t[k] >= kTMin;
             ok[k] = here & passes[k];
             weight[k] = t[k] * (here ? alpha[k] : 0.0f);
-            t[k + 1] = __builtin_fmaf(-kAlphaMax, weight[k], t[k]);
+            t[k + 1] = t[k] - weight[k];
         }
     }
     w.accum = addColour<R0>(colour, weight[0], w.accum);
@@ -368,32 +388,33 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
     for (uint32_t k = 0; k < 4; ++k) {
         if constexpr (TRACK) w.lastIn = ok[k] ? first + static_cast<int32_t>(R0 + k) : w.lastIn;
         if constexpr (DEPTH_MODE == 1) {
-            const bool at = ok[k] & (t[k + 1] <= w.depthT);
+            const bool at = ok[k] & (1.0f - t[k + 1] >= w.depthAt);
             w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
-            w.depthT = at ? -1.0f : w.depthT;
+            w.depthAt = at ? __builtin_inff() : w.depthAt;
         }
     }
     w.t = walks ? t[4] : w.t;
 }
 
-// Up to sixteen records, whose forms lanes 0 .. 15 hold and whose colours
+// Up to sixteen records, whose A, B and C lanes 0 .. 15 hold and whose colours
 // `colour` does (lane l: channel l & 3 of record l / 4), four a group in order,
 // while there are records and the wave has a pixel that walks; the next group's
 // form is computed while this one is blended. Returns the records walked.
 template <uint32_t DEPTH_MODE, bool COMPOSITE, bool TRACK>
-__device__ __forceinline__ uint32_t walkSixteen(WalkLane& w, uint32_t records, const float form[6], float colour,
-                                                const float mono[5], const float4* qmin, const float4* chunkReach,
-                                                float stopZ, uint64_t discs, int32_t first) {
+__device__ __forceinline__ uint32_t walkSixteen(WalkLane& w, uint32_t records, const float form[3], float colour,
+                                                float u, float v, const float4 (*chunk)[kLanes / 4], uint32_t at,
+                                                const float4* chunkReach, float stopZ, uint64_t discs,
+                                                int32_t first) {
     uint32_t walked = 0;
-    Vec4 q = formOf<0>(form, mono);
+    Vec4 q = formOf<0>(form, u, v, chunk, at);
     const auto group = [&](auto g) -> bool {
         constexpr uint32_t G = decltype(g)::value;
         if (G * kGroup >= records) return false;
         Vec4 next = q;
-        if constexpr (G + 1 < 16 / kGroup) next = formOf<G + 1>(form, mono);
+        if constexpr (G + 1 < 16 / kGroup) next = formOf<G + 1>(form, u, v, chunk, at);
         float4 reach = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if constexpr (COMPOSITE) reach = chunkReach[G];
-        walkGroup<DEPTH_MODE, COMPOSITE, TRACK, G>(w, q, colour, qmin[G], reach, stopZ, discs, first);
+        walkGroup<DEPTH_MODE, COMPOSITE, TRACK, G>(w, q, colour, chunk[3][at + G], reach, stopZ, discs, first);
         q = next;
         walked += kGroup;
         return __ballot(w.t >= kTMin) != 0;
@@ -459,17 +480,16 @@ __device__ __forceinline__ void blendBlock(BlendShared<WAVES, COMPOSITE>& shared
     uint32_t slotNext = slotOf(valueAt(mine + kRound));   // the next round's slot
     uint32_t valueNext = valueAt(mine + 2u * kRound);     // the value of the round after
 
-    WalkLane w{{0.0f, 0.0f, 0.0f, 0.0f}, inside ? 1.0f : 0.0f, -1.0f, 1.0f - f.depthThreshold, -1, -1, -1};
+    WalkLane w{{0.0f, 0.0f, 0.0f, 0.0f}, inside ? 1.0f : 0.0f, -1.0f, f.depthThreshold, -1, -1, -1};
     float depthAt = -1.0f;
     uint32_t last = 0;
     if constexpr (MODE == kResume) {
-        w.accum = Vec4{state->r, state->g, state->b, state->depthSum} * (1.0f / kAlphaMax);
+        w.accum = Vec4{state->r, state->g, state->b, state->depthSum};
         w.t = inside && state->active ? state->t : 0.0f;
         depthAt = state->depthAt;
-        w.depthT = depthAt < 0.0f ? w.depthT : -1.0f;
+        w.depthAt = depthAt < 0.0f ? w.depthAt : __builtin_inff();
         last = state->last;
     }
-    const float mono[5] = {pu * pu, pu * pv, pv * pv, pu, pv};
     // Composite: what ends the walk from behind. A pixel with an under depth
     // above 0 stops at the first pair at or behind it (whether or not that pair
     // reaches the pixel: the reference tests the depth first), a disc that
@@ -510,17 +530,22 @@ __device__ __forceinline__ void blendBlock(BlendShared<WAVES, COMPOSITE>& shared
         }
         if (mask != 0) {
             const Staged& s = staged;
-            // q = the form plus log2(opacity / kAlphaMax): alpha / kAlphaMax = 2^q
-            // directly, and both tests (inside the cutoff, alpha >= 1/255) are
-            // q >= qmin. A disc (colour.w 1, opacity 1) has the cutoff alone.
-            const bool disc = COMPOSITE && s.col.w > 0.5f;
-            const float logOpacity = __builtin_amdgcn_logf(s.conic.w) - kLog2AlphaMax;
-            const float cut = logOpacity + kExpScale * s.screen.w;
+            const float scaledCut = kExpScale * s.screen.w;
+            float base, bound;
+            if constexpr (COMPOSITE) {
+                // q = the form less the cutoff; alpha = o' 2^q, the bound o'. A
+                // disc (colour.w 1) is marked by o' < 0: its alpha never passes.
+                base = -scaledCut;
+                bound = s.col.w > 0.5f ? -1.0f : s.conic.w * __builtin_amdgcn_exp2f(scaledCut);
+            } else {
+                // q = the form plus log2(opacity): alpha = 2^q directly, and both
+                // tests (inside the cutoff, alpha >= 1/255) are q >= the bound
+                base = __builtin_amdgcn_logf(s.conic.w);
+                bound = fmaxS(base + scaledCut, kLog2Floor);
+            }
             shared.at[buf][slot] = make_float4(s.screen.x, s.screen.y, kExpScale * s.conic.x,
                                                kExpScale * (s.conic.y + s.conic.y));
-            shared.shape[buf][slot] = make_float4(kExpScale * s.conic.z, logOpacity,
-                                                  disc ? cut : fmaxS(cut, kLog2Floor - kLog2AlphaMax),
-                                                  disc ? 1.0f : 0.0f);
+            shared.shape[buf][slot] = make_float4(kExpScale * s.conic.z, base, bound, 0.0f);
             shared.colour[buf][slot] = make_float4(s.col.x, s.col.y, s.col.z, s.screen.z);
         }
 #pragma unroll
@@ -586,27 +611,30 @@ __device__ __forceinline__ void blendBlock(BlendShared<WAVES, COMPOSITE>& shared
             const float fa = g0.z, fb = g0.w, fc = g1.x;
             const float fd = -(2.0f * fa * ux + fb * vy), fe = -(2.0f * fc * vy + fb * ux);
             const float fbase = ux * (fa * ux + fb * vy) + fc * vy * vy;
-            const float form[6] = {fa, fb, fc, fd, fe, real ? fbase + g1.y : -__builtin_inff()};
-            reinterpret_cast<float*>(shared.qmin[wave])[lane] = real ? g1.z : __builtin_inff();
+            const float form[3] = {fa, fb, fc};
+            reinterpret_cast<float*>(shared.chunk[wave][0])[lane] = fd;
+            reinterpret_cast<float*>(shared.chunk[wave][1])[lane] = fe;
+            reinterpret_cast<float*>(shared.chunk[wave][2])[lane] = real ? fbase + g1.y : -__builtin_inff();
+            reinterpret_cast<float*>(shared.chunk[wave][3])[lane] =
+                real ? g1.z : (COMPOSITE ? 0.0f : __builtin_inff());
             uint64_t discs = 0;
             if constexpr (COMPOSITE) {
-                discs = __ballot(real && g1.w > 0.5f);
+                discs = __ballot(real && g1.z < 0.0f);
                 float ahead = before[0];
 #pragma unroll
                 for (uint32_t q = 1; q < WAVES; ++q) ahead = from == q ? before[q] : ahead;
-                reinterpret_cast<float*>(shared.chunkReach[wave])[lane] =
-                    real ? fmaxS(ahead, shared.reach[buf][record]) : -3.4e38f;
+                reinterpret_cast<float*>(shared.chunkReach[wave])[lane] = fmaxS(ahead, shared.reach[buf][record]);
             }
             waveSync();
             const uint32_t chunkEnd = total - chunk < kLanes ? total - chunk : kLanes;
             for (uint32_t at16 = 0; at16 < chunkEnd; at16 += 16u) {
-                float sixteen[6];
+                float sixteen[3];
 #pragma unroll
-                for (uint32_t m = 0; m < 6; ++m) sixteen[m] = shflF(form[m], at16 + (lane & 15u));
+                for (uint32_t m = 0; m < 3; ++m) sixteen[m] = shflF(form[m], at16 + (lane & 15u));
                 const uint32_t of = shflU(record, at16 + (lane >> 2));
                 const float channel = reinterpret_cast<const float*>(&shared.colour[buf][of])[lane & 3u];
                 walked += walkSixteen<DEPTH_MODE, COMPOSITE, !COMPOSITE && TRACK>(
-                    w, chunkEnd - at16, sixteen, channel, mono, &shared.qmin[wave][at16 / 4],
+                    w, chunkEnd - at16, sixteen, channel, pu, pv, shared.chunk[wave], at16 / 4,
                     &shared.chunkReach[wave][COMPOSITE ? at16 / 4 : 0], stopZ, discs >> at16,
                     static_cast<int32_t>(at16));
                 if (__ballot(w.t >= kTMin) == 0) break;
@@ -642,8 +670,7 @@ __device__ __forceinline__ void blendBlock(BlendShared<WAVES, COMPOSITE>& shared
             if (!walks) break;
         }
     }
-    const float r = kAlphaMax * w.accum[0], g = kAlphaMax * w.accum[1], b = kAlphaMax * w.accum[2];
-    const float depthSum = kAlphaMax * w.accum[3];
+    const float r = w.accum[0], g = w.accum[1], b = w.accum[2], depthSum = w.accum[3];
     const float t = COMPOSITE && w.tStopped >= 0.0f ? w.tStopped : w.t;
     // The walk's records, counted on request (the blend's work is 64 lanes x
     // these steps).

@@ -452,6 +452,66 @@ def test_lists_of_every_length_blend_as_the_oracle(rast, count, tile, opacity, d
         assert d.max() <= (1.0 if (name, depth_mode) == ("depth", 1) else scale / 255.0 * 2.0), (name, d.max())
 
 
+def _fma(a, b, c):
+    """float32 fused multiply-add (the product is exact in float64; a second
+    rounding at a midpoint is a 2^-29 chance a step)."""
+    return (np.asarray(a, np.float64) * np.asarray(b, np.float64) + np.asarray(c, np.float64)).astype(np.float32)
+
+
+def test_pairs_at_their_bound_fall_as_the_nested_form_says(rast):
+    """Which pixels a pair is drawn on, in float32 and step by step as the walk
+    takes it: q = u (A u + (B v + D)) + (v (C v + E) + F) about the quadrant's
+    centre, drawn where q >= the bound. Another order of the same sum takes about
+    one such decision in ten million otherwise (it is asserted that these splats
+    hold one at least); each is worth 1/255 of a pixel's transmittance. The
+    opacity is a power of two, so its logarithm is exact on both sides; what is
+    left is the product of a few hundred float32 factors, 6e-8 each."""
+    count, width, height = 6000, 384, 288
+    rng = np.random.default_rng(1)
+    fields = np.zeros((count, 14), np.float32)
+    fields[:, 0] = rng.uniform(-1.0, 1.0, count)
+    fields[:, 1] = rng.uniform(-0.8, 0.8, count)
+    fields[:, 2] = rng.uniform(-1.0, 1.0, count)
+    fields[:, 3] = 2.0 ** -6
+    fields[:, 4:7] = rng.normal(-3.0, 2.0, (count, 3))
+    fields[:, 7:11] = rng.normal(0.0, 1.0, (count, 4))
+    fields[:, 11:14] = 0.5
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=50.0)
+    s = raster.RenderSettings(width=width, height=height, antialias=False)
+    inst = [(scenes.pack_splats(fields, 0), np.eye(4), raster.SplatEdit())]
+    gpu = H.run_gpu(cam, s, inst, rast)
+    ora = H.run_oracle(cam, s, inst)
+    H.assert_bit_exact(gpu, ora)
+
+    f = np.float32
+    scale, floor = f(-0.72134752044448170368), f(-7.99435343685885793775)
+    tiles_x = (width + 15) // 16
+    y, x = np.mgrid[0:16, 0:16]
+    u, v = ((x & 7) - 3.5).astype(f), ((y & 7) - 3.5).astype(f)
+    t = np.ones((tiles_x * 16, (height + 15) // 16 * 16)).T.copy()
+    otherwise = 0
+    for i in range(0, len(ora["pair_splats"]), 4096):
+        tile = ora["pair_tiles"][i:i + 4096].astype(np.int64)
+        r = ora["proj"][ora["pair_splats"][i:i + 4096]][:, :, None, None]
+        px, py = (tile % tiles_x * 16)[:, None, None] + x, (tile // tiles_x * 16)[:, None, None] + y
+        cx, cy, cutoff, opacity = r[:, 0], r[:, 1], r[:, 3], r[:, 7]
+        a, b, c = scale * r[:, 4], scale * (r[:, 5] + r[:, 5]), scale * r[:, 6]
+        ux, vy = cx - ((px & ~7) + 4).astype(f), cy - ((py & ~7) + 4).astype(f)
+        d, e = -(f(2) * a * ux + b * vy), -(f(2) * c * vy + b * ux)
+        log = np.log2(opacity).astype(f)
+        at = ux * (a * ux + b * vy) + c * vy * vy + log
+        bound = np.maximum(log + scale * cutoff, floor)
+        q = _fma(u, _fma(a, u, _fma(b, v, d)), _fma(v, _fma(c, v, e), at))
+        drawn = (q >= bound) & (px < width) & (py < height)
+        flat = _fma(a, u * u, _fma(b, u * v, _fma(c, v * v, _fma(d, u, _fma(e, v, at)))))
+        otherwise += int((((flat >= bound) != drawn) & (px < width) & (py < height)).sum())
+        np.multiply.at(t, (py, px), np.where(drawn, 1.0 - np.exp2(q.astype(np.float64)), 1.0))
+    assert otherwise > 0
+    t = t[:height, :width]
+    assert t.min() > 2e-4   # no pixel's walk ends early
+    np.testing.assert_allclose(gpu["final_t"], t, rtol=2e-4)
+
+
 def _broad_splats(count, seed, log_scale):
     """Splats wide enough to reach hundreds of tiles each, their depths spread
     with some equal (ties that the slot order breaks)."""
