@@ -10,11 +10,12 @@
 // and its raw accumulated rgb. The backward walks each tile's pairs back to
 // front from there, recovering T before each contributor as T / (1 - alpha).
 //
-// Gradients reach the splats without atomics. The duplication gave each pair
-// its index in the slot-major pair order as its sort value; a tile's four
+// Gradients reach the splats without atomic adds. The duplication gave each
+// pair its index in the slot-major pair order as its sort value; a tile's four
 // quadrant waves reduce each pair's per-pixel gradients across their lanes
-// (DPP), the workgroup adds the four quadrants in LDS and writes one record per
-// pair at that index; each splat then sums its own contiguous run of records.
+// (lane swaps and DPP), the workgroup adds the four quadrants in LDS and writes
+// a record at that index, and sets the pair's bit (an atomic or), for a pair
+// that a pixel saw; each splat then sums the records of its own contiguous run.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -253,6 +254,77 @@ __global__ __launch_bounds__(kBlock) void gatherSlotsKernel(const uint32_t* __re
 
 // ---- blend backward ---------------------------------------------------------
 
+// DPP lane moves for the wave sum; lanes outside row_mask read 0.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dppMove(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+
+// The same move leaving the rows outside row_mask undefined (one instruction
+// fewer than reading 0 there): for steps whose other rows no later step reads.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dppMoveRows(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+
+// Sum over the 64 lanes, landing in lane 63 (the other lanes hold partial or
+// undefined values): pairs, quads, half rows and rows by quad_perm and the row
+// mirrors, then row 0 into row 1 and row 2 into row 3 (row_bcast:15), then
+// rows 0-1 into rows 2-3 (row_bcast:31). Lane 63 reads only rows the earlier
+// steps wrote. Every lane must be active.
+__device__ __forceinline__ float rowSum(float v) {
+    v += dppMove<0xB1, 0xF>(v);       // quad_perm [1, 0, 3, 2]
+    v += dppMove<0x4E, 0xF>(v);       // quad_perm [2, 3, 0, 1]
+    v += dppMove<0x141, 0xF>(v);      // row_half_mirror
+    v += dppMove<0x140, 0xF>(v);      // row_mirror
+    return v;                         // every lane holds its row's sum
+}
+
+__device__ __forceinline__ float waveSum(float v) {
+    v = rowSum(v);
+    v += dppMoveRows<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v += dppMoveRows<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// Two terms' halves (lanes 0-31 and 32-63) summed at once: permlane32_swap
+// leaves a's low half and b's low half in one register and both high halves in
+// the other, so one add gives a's half sums in lanes 0-31 and b's in 32-63.
+__device__ __forceinline__ float halvesOfTwo(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// The same for rows: permlane16_swap leaves rows 0 and 2 of a and of b in one
+// register and rows 1 and 3 in the other, so one add gives row pairs summed:
+// rows 0-3 of the result hold a's rows 0+1, b's rows 0+1, a's rows 2+3 and
+// b's rows 2+3.
+__device__ __forceinline__ float rowsOfTwo(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// A record's nine terms, each summed over the wave's 64 lanes, stored to
+// out[0..8] by the lanes that end with them. Terms 0-7 go in pairs through
+// halvesOfTwo, then the pairs' results in pairs through rowsOfTwo, which
+// leaves four terms a register, one a row (rows 0-3: terms 0, 2, 1, 3 of the
+// four), for the in-row steps; term 8 takes the whole-wave sum. 26
+// instructions where nine whole-wave sums take 54. Every lane must be active.
+__device__ __forceinline__ void waveSum9(const float v[9], float* out) {
+    const float w0 = halvesOfTwo(v[0], v[1]), w1 = halvesOfTwo(v[2], v[3]);
+    const float w2 = halvesOfTwo(v[4], v[5]), w3 = halvesOfTwo(v[6], v[7]);
+    const float x0 = rowSum(rowsOfTwo(w0, w1)), x1 = rowSum(rowsOfTwo(w2, w3));
+    const float s8 = waveSum(v[8]);
+    const uint32_t lane = __lane_id();
+    if ((lane & 15u) == 0u) {
+        const uint32_t row = lane >> 4;
+        const uint32_t at = ((row & 1u) << 1) | (row >> 1);
+        out[at] = x0;
+        out[4 + at] = x1;
+    }
+    if (lane == 63) out[8] = s8;
+}
+
 // sRGB decode and its derivative, for the blend's linearisation
 // (reference color.slang:7-10).
 __device__ __forceinline__ void srgbToLinearGrad(float x, float& value, float& slope) {
@@ -269,63 +341,33 @@ __device__ __forceinline__ void srgbToLinearGrad(float x, float& value, float& s
 
 constexpr uint32_t kWaves = 4;
 constexpr uint32_t kBatch = 64;    // pairs a step, one a lane of each wave
-constexpr uint32_t kSums = 9;      // a pair's sums over a quadrant's pixels
-constexpr uint32_t kRows = 8;      // records whose sums are taken together
-constexpr uint32_t kRowPitch = 68; // a row of 64 pixels, padded so that sixteen rows' vectors spread over the banks
-
-using Vec4 = float __attribute__((ext_vector_type(4)));
 
 // Orders a wave's own LDS writes and reads: its lanes run together, so only
 // the compiler has to keep them in order.
 __device__ __forceinline__ void waveSync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
-// A pair's nine sums over a quadrant's 64 pixels are products of two numbers a
-// pixel and terms that are the same for every record: P = dL/d(power) times
-// 1, u, v, u^2, u v, v^2 (the pixel about the quadrant's centre), and W = T
-// alpha times dL/d(rgb). For eight records they are one matrix product, rows
-// (8 of P, 8 of W) times 64 pixels by 64 pixels times columns (6 + 3), which
-// runs on the matrix cores in f32 (16 of v_mfma_f32_16x16x4): the rows are
-// written to the LDS a pixel a lane and read back a row a lane. Lane l of
-// sumTerms' result holds column l & 15 at pixels 16 (l >> 4) + 0 .. 15.
-//
-// What bounds the backward: vector and matrix issue in the walk, and how many
-// waves are there to hide its chains. Sums by cross-lane adds took 26
-// instructions a record after eight products, six of them swaps at twice an
-// add's cost; staging a 16x16 tile's pairs for four waves took three barriers a
-// batch and 32 KB. Now a wave stages its own quadrant's records (29 KB, five
-// workgroups a CU), two barriers a batch. Blend backward, that against this: 1M
-// splats at 1280x720 262 against 230 us, 24 views of 1M splats 3.85 against
-// 3.12 ms, 30k splats at 489x363 140 against 106 us. The matrix sums with the
-// tile staged together (43 KB, three workgroups a CU): 259 us, 3.75 ms, 104 us.
-// The forward's form by matrix products and one test a record instead of the
-// direct form and three took 188 us, 2.62 ms and 77 us, but where the form's
-// rounding moves a pair over the alpha floor the gradient moves with it: an
-// error against 64 bits up to 1.5 times this one's on some scenes.
-__device__ __forceinline__ void sumTerms(const float dR[3], float* rows, float terms[16]) {
-    const uint32_t lane = threadIdx.x & 63u, column = lane & 15u, first = (lane >> 4) * 16u;
-#pragma unroll
-    for (uint32_t ch = 0; ch < 3; ++ch) rows[ch * kRowPitch + lane] = dR[ch];
-    waveSync();
-    const bool colour = column >= 6u && column < kSums;
-    const float* row = rows + (colour ? column - 6u : 0u) * kRowPitch + first;
-#pragma unroll
-    for (uint32_t s = 0; s < 16; ++s) {
-        const uint32_t px = first + s;
-        const float u = static_cast<float>(px & 7u) - 3.5f, v = static_cast<float>(px >> 3) - 3.5f;
-        float t = column == 0u ? 1.0f : 0.0f;
-        t = column == 1u ? u : t;
-        t = column == 2u ? v : t;
-        t = column == 3u ? u * u : t;
-        t = column == 4u ? u * v : t;
-        t = column == 5u ? v * v : t;
-        terms[s] = colour ? row[s] : t;
-    }
-    waveSync();   // the rows are the records' next
-}
-
 // One tile of frame f (its pairs [range.x, range.y) of the sorted order): the
 // workgroup's four waves take its four quadrants. accum, lastCount, finalT and
 // gradColour are the frame's own per-pixel arrays.
+//
+// What bounds it: vector issue in the walk (a record's products and its 26
+// instructions of cross-lane sums) and, on a small frame, the longest tile's
+// chain through T. Each wave stages its own quadrant's records (12 KB a
+// workgroup, 64 registers: eight waves a SIMD) with the gathers three batches
+// ahead; the tile's pairs staged together for four waves took three barriers a
+// batch and 32 KB. Blend backward, that against this: 1M splats at 1280x720
+// 262 against 222 us, 24 views of 1M splats 3.85 against 2.95 ms, 30k splats at
+// 489x363 140 against 133 us.
+//
+// A pixel's terms are its own until they are summed, zero for a pair that it
+// did not see, and a footprint's moments are taken about its own centre. The
+// nine sums as one f32 matrix product, P = dL/d(power) and W = T alpha of eight
+// records against the monomials of the quadrant's pixels and dL/d(rgb), took
+// 230 us, 3.14 ms and 106 us, but 0 times a pixel's infinite dL/d(rgb) reached
+// every splat of the quadrant, and moments about the quadrant's centre lost
+// half of the digits' margin of footprints under a pixel. Two pairs' sums
+// interleaved (232 us, 3.15 ms, 130 us) and the next record read ahead (237 us,
+// 3.32 ms, 132 us) cost the registers of a wave a SIMD.
 __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t tile, uint2 range, uint32_t slots,
                                                   const uint32_t* __restrict__ pairSlot,
                                                   const uint32_t* __restrict__ pairIndex,
@@ -339,7 +381,6 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
     // a, 2 b; c, alpha, cutoff; rgb, bits of the pair's place in the tile's range.
     // A record's nine sums replace it.
     __shared__ __align__(16) float sRecords[kWaves][kBatch][12];
-    __shared__ __align__(16) float sRows[kWaves][2 * kRows * kRowPitch];
     __shared__ uint64_t sReach[kWaves];   // the batch's pairs that reach each quadrant
     __shared__ uint32_t sMaxLast;
 
@@ -387,18 +428,16 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
             }
         }
     }
-    float terms[16];
-    sumTerms(dR, sRows[wave], terms);
     if (tid == 0) sMaxLast = 0;
     __syncthreads();
     if (last > 0) atomicMax(&sMaxLast, last);
     __syncthreads();
     // A last contributor lies inside its tile's range; the bound keeps the walk there.
     const uint32_t maxLast = sMaxLast < range.y - range.x ? sMaxLast : range.y - range.x;
-    // t: T before the walk's current pair; behind: sum over the channels of dR
-    // times the colour accumulated behind it (the only use of that colour), and
-    // what lies behind every pair, dL/dT times the final T.
-    float t = tFinal, behind = dT * tFinal;
+    // t: T before the walk's current pair; behindDot: sum over the channels of
+    // dR times the colour accumulated behind it (the only use of that colour).
+    float t = tFinal, behindDot = 0.0f;
+    const float dTFinal = dT * tFinal;
     const uint64_t below = (1ull << lane) - 1ull;
     // A batch's records are gathers of three loads one after the other (the
     // pair's index, its slot, the record), so they are loaded ahead: the walk of
@@ -431,12 +470,11 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
                                          loY - screen.y, hiX - screen.x, hiY - screen.y);
         const uint64_t vote = __ballot(reach);
         const uint32_t count = static_cast<uint32_t>(__popcll(vote));
-        const float ca = conic.x, cb2 = conic.y + conic.y, cc = conic.z, opacity = conic.w;
-        const float centreX = screen.x, centreY = screen.y;
+        const float ca = conic.x, cb2 = conic.y + conic.y, cc = conic.z;
         if (reach) {
             auto* record = reinterpret_cast<float4*>(sRecords[wave][__popcll(vote & below)]);
-            record[0] = make_float4(centreX, centreY, ca, cb2);
-            record[1] = make_float4(cc, opacity, screen.w, 0.0f);
+            record[0] = make_float4(screen.x, screen.y, ca, cb2);
+            record[1] = make_float4(cc, conic.w, screen.w, 0.0f);
             record[2] = make_float4(col.x, col.y, col.z, __uint_as_float(maxLast - 1u - done - lane));
         }
         if (lane == 0) sReach[wave] = vote;
@@ -448,101 +486,76 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
         index0 = index1;
         index1 = index2;
         index2 = indexAt(done + 3u * kBatch + lane);
-        // 2. this quadrant's pixels, pair by pair, back to front, the sums of
-        // kRows records at a time
-        float* const rows = sRows[wave];
-        for (uint32_t j0 = 0; j0 < count; j0 += kRows) {
-#pragma unroll
-            for (uint32_t r = 0; r < kRows; ++r) {
-                const uint32_t j = j0 + r;
-                const auto* record = reinterpret_cast<const float4*>(sRecords[wave][j < count ? j : count - 1u]);
-                const float4 g0 = record[0], g1 = record[1], g2 = record[2];
-                const uint32_t place = __float_as_uint(g2.w);
-                const float dx = pxf - g0.x;
-                const float dy = pyf - g0.y;
-                const float power = __builtin_fmaf(dx, __builtin_fmaf(g0.z, dx, g0.w * dy), (g1.x * dy) * dy);
-                const float raw = g1.y * __builtin_amdgcn_exp2f(kExpScale * power);
-                const float alpha = __builtin_fminf(0.99f, raw);
-                // (past the list's end the last record again, which nothing passes)
-                const bool ok = (j < count) & (place < last) & (power <= g1.z) & (alpha >= 1.0f / 255.0f);
+        // 2. this quadrant's pixels, pair by pair, back to front
+        for (uint32_t j = 0; j < count; ++j) {
+            float* const sums = sRecords[wave][j];
+            const auto* record = reinterpret_cast<const float4*>(sums);
+            const float4 g0 = record[0], g1 = record[1], g2 = record[2];
+            const uint32_t place = __float_as_uint(g2.w);
+            const float dx = pxf - g0.x;
+            const float dy = pyf - g0.y;
+            const float power = __builtin_fmaf(dx, __builtin_fmaf(g0.z, dx, g0.w * dy), (g1.x * dy) * dy);
+            const float gauss = __builtin_amdgcn_exp2f(kExpScale * power);
+            const float raw = g1.y * gauss;
+            const float alpha = __builtin_fminf(0.99f, raw);
+            const bool ok = (place < last) & (power <= g1.z) & (alpha >= 1.0f / 255.0f);
+            float v[9] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            if (ok) {
                 const float inv = __builtin_amdgcn_rcpf(1.0f - alpha);
                 const float tBefore = t * inv;
                 // sum_ch dR (T_before c - behind / (1 - alpha)) - dT tFinal / (1 - alpha)
                 const float dotColour = __builtin_fmaf(dR[2], g2.z, __builtin_fmaf(dR[1], g2.y, dR[0] * g2.x));
-                const float dAlpha = __builtin_fmaf(tBefore, dotColour, -(behind * inv));
-                const float weight = ok ? tBefore * alpha : 0.0f;
-                behind = __builtin_fmaf(weight, dotColour, behind);
-                t = ok ? tBefore : t;
-                // alpha = opacity exp(-power / 2); none of it through the clamp
-                const float dPower = (ok & (raw < 0.99f)) ? -0.5f * alpha * dAlpha : 0.0f;
-                rows[r * kRowPitch + lane] = dPower;
-                rows[(kRows + r) * kRowPitch + lane] = weight;
-            }
-            waveSync();
-            const float4* row = reinterpret_cast<const float4*>(rows + (lane & 15u) * kRowPitch + (lane >> 4) * 16u);
-            Vec4 sums = {0.0f, 0.0f, 0.0f, 0.0f};
+                const float dAlpha = __builtin_fmaf(tBefore, dotColour, -(behindDot + dTFinal) * inv);
+                const float weight = tBefore * alpha;
 #pragma unroll
-            for (uint32_t c = 0; c < 4; ++c) {
-                const float4 v = row[c];
-                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, terms[4 * c], sums, 0, 0, 0);
-                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, terms[4 * c + 1], sums, 0, 0, 0);
-                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, terms[4 * c + 2], sums, 0, 0, 0);
-                sums = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, terms[4 * c + 3], sums, 0, 0, 0);
+                for (int ch = 0; ch < 3; ++ch) v[6 + ch] = dR[ch] * weight;
+                behindDot = __builtin_fmaf(weight, dotColour, behindDot);
+                t = tBefore;
+                if (raw < 0.99f) {
+                    // alpha = opacity * exp(-power / 2). The power's gradient is
+                    // summed as moments over the pixels (dPower dx, dPower dy,
+                    // dPower dx^2, dPower dx dy, dPower dy^2); the pair's conic
+                    // turns them into its centre and conic terms once the
+                    // quadrants are added.
+                    const float dPower = -0.5f * alpha * dAlpha;
+                    v[5] = dAlpha * gauss;
+                    v[0] = dPower * dx;
+                    v[1] = dPower * dy;
+                    v[2] = v[0] * dx;
+                    v[3] = v[0] * dy;
+                    v[4] = v[1] * dy;
+                }
             }
-            // Lane l holds rows 4 (l >> 4) + 0 .. 3 at column l & 15: P's six
-            // columns in the first two groups of lanes, W's three in the others.
-            const uint32_t column = lane & 15u, group = lane >> 4;
-            const bool mine = group < 2u ? column < 6u : column >= 6u && column < kSums;
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-                const uint32_t j = j0 + (group & 1u) * 4u + i;
-                if (mine && j < count) sRecords[wave][j][column] = sums[i];
+            if (__ballot(ok) != 0) {
+                waveSum9(v, sums);
+            } else if (lane < 9) {
+                sums[lane] = 0.0f;
             }
-            waveSync();   // the rows are read: the next records' may be written
         }
         __syncthreads();
         // 3. the four quadrants' sums, one record per pair (the waves in turn)
         if (wave == ((done / kBatch) & 3u)) {
-            // (in 64 bits: a long splat's conic gradient is what is left of large
-            // moments, and the shift must not cost it digits)
-            double s0 = 0.0, sx = 0.0, sy = 0.0, sxx = 0.0, sxy = 0.0, syy = 0.0;
-            float rgb[3] = {0.0f, 0.0f, 0.0f};
+            float sum[9] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (uint32_t q = 0; q < kWaves; ++q) {
                 const uint64_t m = sReach[q];
                 if ((m >> lane) & 1u) {
                     const float* p = sRecords[q][__popcll(m & below)];
-                    // The moments about the quadrant's centre to those about the
-                    // pair's: du = u - cx, dv = v - cy.
-                    const double cx = double{centreX} - static_cast<double>(tileX * kTile + (q & 1u) * 8u + 4u);
-                    const double cy = double{centreY} - static_cast<double>(tileY * kTile + (q >> 1) * 8u + 4u);
-                    const double m0 = p[0], m1 = p[1], m2 = p[2];
-                    const double mx = m1 - cx * m0, my = m2 - cy * m0;
-                    s0 += m0;
-                    sx += mx;
-                    sy += my;
-                    sxx += double{p[3]} - cx * (m1 + mx);
-                    sxy += double{p[4]} - cy * m1 - cx * my;
-                    syy += double{p[5]} - cy * (m2 + my);
 #pragma unroll
-                    for (int ch = 0; ch < 3; ++ch) rgb[ch] += p[6 + ch];
+                    for (int k = 0; k < 9; ++k) sum[k] += p[k];
                 }
             }
             // The moments to d(centre) = -(2a Sx + 2b Sy, 2b Sx + 2c Sy) and
-            // d(conic) = (Sxx, 2 Sxy, Syy); d(alpha) = sum of dL/d(alpha at the
-            // pixel) exp(-power / 2) = -2 S / alpha.
-            const double ca2 = 2.0 * double{ca}, cc2 = 2.0 * double{cc};
-            const float4 a = make_float4(static_cast<float>(-(ca2 * sx + double{cb2} * sy)),
-                                         static_cast<float>(-(double{cb2} * sx + cc2 * sy)), static_cast<float>(sxx),
-                                         static_cast<float>(2.0 * sxy));
-            const float4 b = make_float4(static_cast<float>(syy),
-                                         s0 != 0.0 ? -2.0f * static_cast<float>(s0) / opacity : 0.0f, rgb[0], rgb[1]);
+            // d(conic) = (Sxx, 2 Sxy, Syy).
+            const float4 a = make_float4(-(2.0f * ca * sum[0] + cb2 * sum[1]), -(cb2 * sum[0] + 2.0f * cc * sum[1]),
+                                         sum[2], 2.0f * sum[3]);
+            const float4 b = make_float4(sum[4], sum[5], sum[6], sum[7]);
             const bool live = a.x != 0.0f || a.y != 0.0f || a.z != 0.0f || a.w != 0.0f || b.x != 0.0f || b.y != 0.0f ||
-                             b.z != 0.0f || b.w != 0.0f || rgb[2] != 0.0f;
+                             b.z != 0.0f || b.w != 0.0f || sum[8] != 0.0f;
             if (live) {
                 pairGrad.ab[2 * uint64_t{index}] = a;
                 pairGrad.ab[2 * uint64_t{index} + 1] = b;
-                pairGrad.c[index] = rgb[2];
+                pairGrad.c[index] = sum[8];
                 atomicOr(&pairGrad.live[index >> 5], 1u << (index & 31u));
             }
         }
@@ -550,7 +563,7 @@ __device__ __forceinline__ void blendBackwardTile(const FrameParams& f, uint32_t
     }
 }
 
-__global__ __launch_bounds__(kBlock, 4) void blendBackwardKernel(FrameParams f, uint32_t slots,
+__global__ __launch_bounds__(kBlock, 8) void blendBackwardKernel(FrameParams f, uint32_t slots,
                                                               const uint2* __restrict__ ranges,
                                                               const uint32_t* __restrict__ pairSlot,
                                                               const uint32_t* __restrict__ pairIndex,
@@ -571,7 +584,7 @@ __global__ __launch_bounds__(kBlock, 4) void blendBackwardKernel(FrameParams f, 
 // Every tile of a batch of views: workgroup g takes batch tile g, in its view's
 // frame and per-pixel arrays (ViewInfo.pixelBase), with that view's colour
 // gradient.
-__global__ __launch_bounds__(kBlock, 4) void blendBackwardViewsKernel(const FrameParams* __restrict__ params,
+__global__ __launch_bounds__(kBlock, 8) void blendBackwardViewsKernel(const FrameParams* __restrict__ params,
                                                                    const ViewInfo* __restrict__ views,
                                                                    uint32_t viewCount, uint32_t slots,
                                                                    const uint2* __restrict__ ranges,

@@ -129,6 +129,59 @@ def test_runs_of_every_length_sum_to_the_fp64_oracles_gradients(rast, log_scale,
         np.testing.assert_array_equal(again[name].cpu().numpy().view(np.uint32), grads[name].view(np.uint32))
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_a_non_finite_gradient_stays_with_the_splats_its_pixel_saw(rast, bad):
+    """Two splats apart in one 8x8 quadrant of pixels. A gradient that is not a
+    number at a pixel neither covers changes nothing; at the first one's centre
+    it takes that splat's gradients and leaves the second's bit for bit."""
+    focal = W / (2.0 * np.tan(np.radians(30.0)))
+    at = np.array([[65.5, 49.5], [70.5, 54.5]])
+    p = scenes.diff_params(2, 3, degree=1, log_scale=(-6.0, 0.0))
+    p["means"] = np.stack([(at[:, 0] - W / 2) * 4.0 / focal, (at[:, 1] - HGT / 2) * 4.0 / focal,
+                           np.full(2, -4.0)], 1).astype(np.float32)
+    p["opacity_logits"] = np.ones(2, np.float32)
+    s = raster.RenderSettings(width=W, height=HGT, antialias=False)
+    g = np.random.default_rng(9).normal(0.0, 1.0, (HGT, W, 4))
+    image, _ = _gpu_grads(rast, p, s, g)
+    covered = image[48:56, 64:72, 3] > 0.0
+    assert covered[1, 1] and covered[6, 6] and not covered[0, 7] and covered.sum() < 32
+    for (y, x), lost in (((48, 71), 0), ((49, 65), 1)):
+        for channel in range(3):
+            g0, g1 = g.copy(), g.copy()
+            g0[y, x] = 0.0
+            g1[y, x] = 0.0
+            g1[y, x, channel] = bad
+            _, clean = _gpu_grads(rast, p, s, g0)
+            _, got = _gpu_grads(rast, p, s, g1)
+            for name in GROUPS:
+                np.testing.assert_array_equal(got[name][lost:].view(np.uint32), clean[name][lost:].view(np.uint32))
+                assert np.isfinite(clean[name]).all()
+            if lost:
+                assert not np.isfinite(got["sh"][0]).all() and not np.isfinite(got["means"][0]).all()
+
+
+def test_small_footprints_keep_float32_gradients(rast):
+    """Splats under a pixel wide: the second moments of a footprint are sums about
+    its own centre, so a splat's scale gradients are right to a few float32
+    roundings (15 of them, 6e-8 each, at the median, and 40 at nine in ten; taken
+    about the quadrant's centre and moved, they were off by twice that)."""
+    n = 400
+    p = scenes.diff_params(n, 1, degree=0, log_scale=(-6.0, 0.3))
+    p["opacity_logits"] = np.ones(n, np.float32)
+    s = raster.RenderSettings(width=W, height=HGT, linearise=False, antialias=False)
+    y, x = np.mgrid[0:HGT, 0:W]
+    g = np.zeros((HGT, W, 4))
+    g[..., :3] = (1.0 + 0.3 * np.sin(x * 0.05) * np.cos(y * 0.04))[..., None]
+    _, grads = _gpu_grads(rast, p, s, g)
+    ref = D.gradients(_oracle_frame(s, n, 0), p, g)
+    a, b = grads["log_scales"].astype(np.float64), ref["log_scales"].reshape(n, 3)
+    size = np.linalg.norm(b, axis=1)
+    off = np.linalg.norm(a - b, axis=1)[size > 0] / size[size > 0]
+    print(f"  log_scales, a splat's relative error vs FP64: median {np.median(off):.1e}, "
+          f"nine in ten below {np.quantile(off, 0.9):.1e}", flush=True)
+    assert np.median(off) < 9e-7 and np.quantile(off, 0.9) < 2.4e-6
+
+
 def test_gradients_against_fp64_central_differences(rast):
     """The 8 largest gradient components of each group against FP64 central
     differences of the C brute force. The forward is piecewise smooth: a pixel
