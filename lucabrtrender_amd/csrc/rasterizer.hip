@@ -605,9 +605,11 @@ bool TileRasterizer::binDepthFirst(const FrameParams& first, uint32_t slots, uin
     };
     // The drawn slots and their depth keys, sorted so that they end in the second
     // pair of pair buffers (drawn <= pairs <= capacity; the duplication below
-    // fills the first), the offsets of their pairs behind the keys there.
+    // fills the first), the offsets of their pairs behind the keys there. One
+    // slot alone is sorted as it is: no pass moves it.
     mark(9);
-    const int from = kern::sortPasses(layout.depthBits, settings.radixBits) % 2 == 0 ? 1 : 0;
+    const uint32_t passes = drawn < 2 ? 0u : kern::sortPasses(layout.depthBits, settings.radixBits);
+    const int from = passes % 2 == 0 ? 1 : 0;
     uint32_t* depthKeys[2] = {keys_[0].as<uint32_t>(), keys_[1].as<uint32_t>()};
     uint32_t* slotsOf[2] = {values_[0].as<uint32_t>(), values_[1].as<uint32_t>()};
     kern::compactDrawn(touched_.as<uint32_t>(), proj_.as<float4>(), slots, layout.depthMin,

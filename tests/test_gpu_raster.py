@@ -564,3 +564,37 @@ def test_frames_of_many_pairs_a_splat_bin_as_the_oracle(size, tile, count, log_s
     small = [(_broad_splats(500, 4, -3.5), np.eye(4), raster.SplatEdit())]
     for _ in range(2):
         H.assert_bit_exact(H.run_gpu(cam, few, small, rast), H.run_oracle(cam, few, small))
+
+
+def test_one_splat_over_millions_of_tiles_draws_as_at_larger_tiles():
+    """A single drawn splat past the pair count where slots are sorted by depth
+    first: there is nothing to sort, and its pairs are its own. 6.25M 8-pixel
+    tiles against the same frame in 16-pixel tiles, whose 1.6M pairs take the
+    one sort: bit for bit, with another splat's frame drawn before."""
+    import torch
+    side = 20_000
+    fields = np.zeros((3, 14), np.float32)
+    fields[:, 3] = 0.6
+    fields[:, 4:7] = (3.0, 2.5, 2.0)
+    fields[:, 10] = 1.0
+    fields[:, 11:14] = (0.9, 0.5, 0.2)
+    fields[1:, :3] = ((0.3, 0.2, 0.5), (0.0, 0.0, 9.0))   # the last behind the camera
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=30.0)
+    rast = raster.TileRasterizer()
+
+    def draw(rows, tile):
+        scene = scenes.pack_splats(np.ascontiguousarray(fields[rows]), 0).to_device()
+        targets = raster.RenderTargets(side, side)
+        st = rast.render(cam, [raster.SplatInstance(scene)],
+                         raster.RenderSettings(width=side, height=side, tile_size=tile), targets)
+        torch.cuda.synchronize()
+        return st, targets
+
+    draw([1, 0], 8)
+    st, one = draw([2, 0], 8)
+    assert st.visible == 1 and st.pairs == (side // 8) ** 2
+    st, want = draw([2, 0], 16)
+    assert st.visible == 1 and st.pairs == (side // 16) ** 2
+    assert float(want.colour[::999, ::999].min()) > 0.0
+    assert torch.equal(one.colour.view(torch.int32), want.colour.view(torch.int32))
+    assert torch.equal(one.depth.view(torch.int32), want.depth.view(torch.int32))
