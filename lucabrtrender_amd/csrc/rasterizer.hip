@@ -429,8 +429,8 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
     const auto countsDone = std::chrono::steady_clock::now();
     const uint32_t pairs = splatCount > 0 ? hostCounters_[0] : 0u;
     const uint32_t visible = splatCount > 0 ? hostCounters_[1] : 0u;
-    if (hostCounters_[5] != 0) {
-        return abandon(Status::error(ErrorCode::InternalError, "the scan's look-back gave up"));
+    if (hostCounters_[kScanGaveUp] != 0) {
+        return abandon(Status::error(ErrorCode::InternalError, kScanGaveUpMessage));
     }
     if (pairs > kMaxPairs) {
         return abandon(Status::error(ErrorCode::Unsupported, "more than 2^30 - 1 (tile, splat) pairs in one frame"));
@@ -548,11 +548,7 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
         return s;
     if (!(s = check(hipStreamSynchronize(stream_), "frame")).ok()) return s;
     if (!(s = check(hipGetLastError(), "frame")).ok()) return s;
-    if (hostCounters_[2] != 0) return Status::error(ErrorCode::InternalError, "the duplication overran its pairs");
-    if (hostCounters_[10] != 0) {
-        return Status::error(ErrorCode::InternalError, "a drawn splat's depth key fell outside the frame's range");
-    }
-    if (hostCounters_[4] != 0) return Status::error(ErrorCode::InternalError, "the sort's look-back gave up");
+    if (!(s = binningStatus(hostCounters_, "a drawn splat's depth key fell outside the frame's range")).ok()) return s;
     const auto wallEnd = std::chrono::steady_clock::now();
 
     lastSplats_ = splatCount;
@@ -983,19 +979,16 @@ Status TileRasterizer::runViews(std::span<const View> views, std::span<const Spl
         }
         if (!(s = check(hipStreamSynchronize(stream_), "batch")).ok()) return s;
         if (!(s = check(hipGetLastError(), "batch")).ok()) return s;
-        if (hostCounters_[5] != 0) return Status::error(ErrorCode::InternalError, "the scan's look-back gave up");
+        if (hostCounters_[kScanGaveUp] != 0) return Status::error(ErrorCode::InternalError, kScanGaveUpMessage);
         const uint32_t pairs = hostCounters_[0];
         if (pairs > kMaxPairs) {
             return Status::error(ErrorCode::Unsupported, "more than 2^30 - 1 (tile, splat) pairs in one batch");
         }
-        if (hostCounters_[2] == 0) break;
+        if (hostCounters_[kPairsDropped] == 0) break;
         if (attempt == 1) return Status::error(ErrorCode::InternalError, "the duplication overran its pairs");
         if (!(s = reservePairs(pairs, keyBits, training, settings.radixBits)).ok()) return s;
     }
-    if (hostCounters_[10] != 0) {
-        return Status::error(ErrorCode::InternalError, "a drawn splat's depth key fell outside the batch's planes");
-    }
-    if (hostCounters_[4] != 0) return Status::error(ErrorCode::InternalError, "the sort's look-back gave up");
+    if (!(s = binningStatus(hostCounters_, "a drawn splat's depth key fell outside the batch's planes")).ok()) return s;
     const auto wallEnd = std::chrono::steady_clock::now();
     if (settings.timeStages && !settings.useGraph) {
         static constexpr int kFrom[7] = {0, 1, 3, 4, 5, 6, 7};
@@ -1090,7 +1083,7 @@ Status TileRasterizer::referenceRender(const Projection& projection, std::span<c
         return s;
     if (!(s = check(hipStreamSynchronize(stream_), "reference")).ok()) return s;
     if (!(s = check(hipGetLastError(), "reference")).ok()) return s;
-    if (hostCounters_[4] != 0) return Status::error(ErrorCode::InternalError, "the sort's look-back gave up");
+    if (hostCounters_[kSortGaveUp] != 0) return Status::error(ErrorCode::InternalError, "the sort's look-back gave up");
     return {};
 }
 
@@ -1335,7 +1328,7 @@ Status TileRasterizer::decodeCloud(const io::RawSplats& raw, uint32_t maxDegree,
         (void)hipEventRecord(events_[2], stream_);
         (void)hipMemcpyAsync(hostCounters_, counters, 32, hipMemcpyDeviceToHost, stream_);
         if (!(s = check(hipStreamSynchronize(stream_), "decode splats")).ok()) return s;
-        if (hostCounters_[5] != 0) return Status::error(ErrorCode::InternalError, "the scan's look-back gave up");
+        if (hostCounters_[kScanGaveUp] != 0) return Status::error(ErrorCode::InternalError, kScanGaveUpMessage);
         written += hostCounters_[0];
         float ms = 0.0F;
         if (hipEventElapsedTime(&ms, events_[0], events_[1]) == hipSuccess) uploadMs += ms;

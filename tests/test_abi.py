@@ -143,3 +143,35 @@ def test_every_ctypes_mirror_has_the_header_s_layout(tmp_path):
     subprocess.run([gcc, "-std=c11", "-I", include, str(src), "-o", str(exe)], check=True)
     got = [int(v) for v in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
     assert got == expected
+
+
+def test_every_failure_word_of_a_frame_s_counters_fails_it(tmp_path):
+    """The check that ends a frame and a batch (status.h, host code alone): each
+    word that a kernel flags a failure in is an error, the scan's among them (a
+    frame that sorts by depth first scans again after the host has read the
+    counts), and the words that are counts are none."""
+    import shutil
+    import subprocess
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no C++ compiler")
+    src = tmp_path / "counters.cpp"
+    src.write_text("""#include <cstdio>
+#include "status.h"
+int main() {
+    for (int k = -1; k < 12; ++k) {
+        uint32_t counters[12] = {};
+        if (k >= 0) counters[k] = 1;
+        const lrt::Status s = lrt::binningStatus(counters, "outside");
+        std::printf("%d %s\\n", static_cast<int>(s.code), s.message.c_str());
+    }
+}
+""")
+    exe = tmp_path / "counters"
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([gxx, "-std=c++20", "-I", os.path.join(root, "lucabrtrender_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines()
+    failures = {k - 1: line.split(" ", 1)[1] for k, line in enumerate(out) if line.split()[0] != "0"}
+    assert set(failures) == {2, 4, 5, 10}
+    assert "scan" in failures[5] and "sort" in failures[4] and failures[10] == "outside"
