@@ -273,6 +273,19 @@ private:
     // (the composite blend when `composite`, over `under` when non-null).
     // scanZeroed: the projection already cleared the scan's look-back words
     // and the counters.
+    // Whether the last frame of a shape (tiles, splats to a power of two, training
+    // or not) asked for the depth sort first: decides whether the next one's
+    // duplication is queued before its counts are known, and nothing of what it
+    // draws. The last eight shapes: a program that draws a large and a small
+    // view in turn keeps each one's.
+    struct BinHint {
+        uint64_t shape = 0;
+        bool depthFirst = false;
+    };
+    BinHint& binHint(uint32_t tiles, uint32_t splatCount, bool training);
+    std::array<BinHint, 8> binHints_{};
+    uint32_t nextBinHint_ = 0;
+
     // A frame's pairs binned depth first (finishFrame): the drawn slots sorted by
     // depth, duplicated in that order, the pairs sorted by tile, the ranges.
     // Returns whether the sorted pairs are in the second pair of buffers.
@@ -332,7 +345,6 @@ private:
     int lastSorted_ = 0;   // which of keys_/values_ hold the sorted pairs
     bool lastNarrow_ = false;       // the sorted keys are u32 (kern::sortNarrows) or
     bool lastTiles16_ = false;      // u16 tiles
-    bool depthFirst_ = false;       // the last frame's counts asked for the depth sort first
     uint32_t lastTileShift_ = 0;    // their tile is key >> lastTileShift_
     bool lastSlotsSorted_ = false;  // the sorted values are pair indices (their slots: pairSlot_)
     // The last plain (one view, splats only, not split) blend's launch, for

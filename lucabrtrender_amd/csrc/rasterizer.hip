@@ -45,9 +45,12 @@ constexpr uint32_t kMaxPairs = (1u << 30) - 1;
 // against depth first: 500k slots and 4.6M pairs 217 and 215; 1M and 9.3M 352
 // and 305 (training 343 and 337); 1M and 16.5M 592 and 432; 3M and 49M 1656 and
 // 1080; 1.2M and 3.6M 258 and 309; 6M and 694M 23.3 ms and 13.1 ms.
-bool depthFirst(uint32_t pairs, uint32_t drawn, bool training) {
+// A frame whose pairs are already duplicated in slot order (`duplicated`) has
+// 7.5 us a million pairs less to gain: that duplication is done, and done again.
+bool depthFirst(uint32_t pairs, uint32_t drawn, bool training, bool duplicated) {
     const uint64_t quarterSlots = training ? 16u : 5u;
-    return 4ull * pairs > 24'000'000ull + quarterSlots * drawn;
+    return duplicated ? 3ull * pairs > 30'000'000ull + 2u * quarterSlots * drawn
+                      : 4ull * pairs > 24'000'000ull + quarterSlots * drawn;
 }
 
 }   // namespace
@@ -415,9 +418,10 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
                         counters + 8, counters + 10);
         mark(4);
     };
-    // (Not after a frame that sorted by depth first: its successor most likely
-    // does, and this duplication would be done for nothing.)
-    const bool early = pairCapacity_ > 0 && !depthFirst_ &&
+    // (Not where the last frame of this shape sorted by depth first: this one
+    // most likely does, and the duplication would be done for nothing.)
+    BinHint& hint = binHint(tiles, splatCount, training);
+    const bool early = pairCapacity_ > 0 && !hint.depthFirst &&
                        (!training || pairSlot_.bytes() >= uint64_t{pairCapacity_} * 4);
     if (early) duplicateInto();
     // A frame given up here leaves nothing of its own running on the stream.
@@ -448,9 +452,9 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
     }
     const uint32_t keyBits = bitsFor(tiles) + layout.depthBits;
     stats.keyBits = keyBits;
-    depthFirst_ = depthFirst(pairs, visible, training);
+    hint.depthFirst = depthFirst(pairs, visible, training, false);
     const bool fits = early && pairs <= pairCapacity_;
-    const bool ordered = depthFirst_ && !fits;
+    const bool ordered = depthFirst(pairs, visible, training, fits);
     if (!fits) {
         // The early run must be done before its buffers may be replaced.
         if (early && !(s = check(hipStreamSynchronize(stream_), "duplicate")).ok()) return s;
@@ -587,6 +591,15 @@ Status TileRasterizer::finishFrame(const FrameParams& first, uint32_t splatCount
     }
     if (statsOut != nullptr) *statsOut = stats;
     return {};
+}
+
+TileRasterizer::BinHint& TileRasterizer::binHint(uint32_t tiles, uint32_t splatCount, bool training) {
+    const uint64_t shape = uint64_t{tiles} << 8 | std::bit_width(splatCount) << 1 | (training ? 1u : 0u);
+    for (BinHint& h : binHints_)
+        if (h.shape == shape) return h;
+    BinHint& h = binHints_[nextBinHint_++ % binHints_.size()];
+    h = BinHint{shape, false};
+    return h;
 }
 
 template <typename Workspace>

@@ -566,6 +566,33 @@ def test_frames_of_many_pairs_a_splat_bin_as_the_oracle(size, tile, count, log_s
         H.assert_bit_exact(H.run_gpu(cam, few, small, rast), H.run_oracle(cam, few, small))
 
 
+def test_a_large_and_a_small_view_in_turn_keep_their_own_order():
+    """Two views on one rasteriser, one of many pairs a splat: from its second
+    frame on the large one sorts by depth first, whatever was drawn in between,
+    and the small one never does; the images are the same either way."""
+    import dataclasses
+
+    import torch
+    rast = raster.TileRasterizer()
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=30.0)
+    large = raster.RenderSettings(width=1920, height=1080, time_stages=True)
+    small = dataclasses.replace(large, width=250, height=190)
+    broad, few = _broad_splats(60_011, 3, -2.7).to_device(), _broad_splats(500, 4, -3.5).to_device()
+    images = []
+    for turn in range(3):
+        for s, cloud, settings in (("small", few, small), ("large", broad, large)):
+            targets = raster.RenderTargets(settings.width, settings.height)
+            st = rast.render(cam, [raster.SplatInstance(cloud)], settings, targets)
+            torch.cuda.synchronize()
+            if s == "small":
+                assert st.depth_sort_ms == 0.0
+                continue
+            assert st.pairs > 6_000_000 + 1.25 * st.visible
+            assert turn == 0 or st.depth_sort_ms > 0.0, turn
+            images.append(targets.colour.view(torch.int32))
+    assert torch.equal(images[0], images[1]) and torch.equal(images[0], images[2])
+
+
 def test_one_splat_over_millions_of_tiles_draws_as_at_larger_tiles():
     """A single drawn splat past the pair count where slots are sorted by depth
     first: there is nothing to sort, and its pairs are its own. 6.25M 8-pixel
