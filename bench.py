@@ -127,7 +127,8 @@ WALK_FLOPS = 5 * 2 + 1 + 1 + 1 + 4 * 2 + 1
 
 def roofline_of(kernel, stages, passes):
     """The dominant kernel against the ceiling that bounds it: the blend against
-    MI355X's FP32 VALU peak (its walk is VALU-bound; achieved = walk steps x 64
+    MI355X's FP32 peak, the same for its vector units and its matrix cores (its
+    walk issues on both; achieved = walk steps x 64
     pixels x WALK_FLOPS / the launch's time), any other kernel against HBM
     (achieved = algorithmic bytes / time). traffic: the kernel's measured HBM
     bytes a launch (rocprofv3 counters, the committed traffic summary)."""
@@ -135,7 +136,7 @@ def roofline_of(kernel, stages, passes):
     traffic = measured_traffic_bytes(kernel, passes)
     if kernel == "blend":
         achieved = st["TFLOP/s"]
-        return {"kernel": kernel, "bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+        return {"kernel": kernel, "bound": "fp32", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / FP32_PEAK_TFLOPS, 4), "traffic": traffic,
                 "walk_steps": st["walk_steps"], "flops_per_step": 64 * WALK_FLOPS,
                 "hbm": {"algorithmic_bytes": st["bytes"], "GB/s": st["GB/s"], "frac": st["hbm_frac"]}}
@@ -405,8 +406,8 @@ def _batch_against_sequence(torch, raster, rast, views, inst, settings, reps):
             "sequence_ms": round(seq_s * 1e3, 3), "views_per_s_single": round(n / seq_s, 1),
             "speedup": round(seq_s / batch_s, 3),
             "stage_ms_eager": {name: round(float(acc[k] / reps), 3) for k, name in enumerate(STAGES)},
-            "tuned": {"blend_batch": tuned.blend_batch, "persistent_blend": tuned.persistent_blend,
-                      "use_graph": tuned.use_graph, "tile_size": tuned.tile_size}}
+            "tuned": {"persistent_blend": tuned.persistent_blend, "use_graph": tuned.use_graph,
+                      "tile_size": tuned.tile_size, "radix_bits": tuned.radix_bits}}
 
 
 def views_leg(torch, raster, scenes, reps):
@@ -563,7 +564,9 @@ def sort_stress_leg(torch, raster, scenes, _abi, reps):
     sort_ms = float(ms[3] + ms[4])
     # The metric's algorithmic bytes (64-bit keys with the full 24-bit depth key
     # every pass), and the bytes this sort moves (keys u32 after the first pass,
-    # the depth field narrowed to the drawn keys' span).
+    # the depth field narrowed to the drawn keys' span). The metric's bytes over
+    # the time are a share of the memory's rate only for a sort that moves them:
+    # a frame that sorts by depth first moves a fifth, and its share is of those.
     defined, defined_passes = defined_sort_bytes(pairs, tiles)
     pass_bytes = sort_pass_bytes(pairs, passes, st.key_bits)
     moved = pairs * 8 + pass_bytes   # the histogram reads every key once
@@ -584,7 +587,8 @@ def sort_stress_leg(torch, raster, scenes, _abi, reps):
             "sort_gkeys_per_s": round(pairs / (sort_ms * 1e-3) / 1e9, 3),
             "sort_bytes": int(defined), "sort_bytes_passes": defined_passes,
             "sort_GB/s": round(defined / (sort_ms * 1e-3) / 1e9, 1),
-            "sort_hbm_frac": round(defined / (sort_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+            "depth_first": st.depth_sort_ms > 0.0,
+            "sort_hbm_frac": round((moved if st.depth_sort_ms > 0.0 else defined) / (sort_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "moved_bytes": int(moved), "moved_GB/s": round(moved / (sort_ms * 1e-3) / 1e9, 1),
             "moved_hbm_frac": round(moved / (sort_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "passes_ms": round(float(ms[4]), 4),
@@ -657,7 +661,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=10)
     ap.add_argument("--count", type=int, default=3_000_000, help="splats (the workload is 3,000,000)")
     ap.add_argument("--cpu-seconds", type=float, default=15.0, help="CPU-baseline budget; 0 skips it")
-    ap.add_argument("--blend-batch", type=int, default=256, help="records in each quadrant's LDS list: 64, 128 or 256")
+    ap.add_argument("--blend-batch", type=int, default=256, help="64, 128 or 256: accepted, of no effect on the blend")
     ap.add_argument("--tile-size", type=int, default=16, help="pixels a tile's side: 8, 16 (the reference's) or 32")
     ap.add_argument("--sweeps", type=int, default=1, help="1: the blend-setting and tile-size comparisons; 0 skips them")
     ap.add_argument("--image-pixels", type=int, default=65536,
@@ -770,18 +774,17 @@ def main():
     stages["blend"]["TFLOP/s"] = round(walk_steps * 64 * WALK_FLOPS / (stages["blend"]["ms"] * 1e-3) / 1e12, 3)
     roofline = roofline_of(dominant, stages, passes)
     copy_gbs = copy_bandwidth_gbs(torch)
-    # The blend at each batch depth and launch order, split blends and the frame
-    # at each tile size, for the record (--sweeps 0 skips them).
+    # The blend at each launch order, split blends and the frame at each tile
+    # size, for the record (--sweeps 0 skips them).
     variants, tile_sizes = {}, {}
     if args.sweeps:
-        for batch in (64, 128, 256):
-            for order in (0, 1):
-                vs = raster.RenderSettings(**{**timed.__dict__, "blend_batch": batch, "tile_order": order})
-                acc_v = np.zeros(8)
-                for _ in range(10):
-                    rast.render(proj, inst, vs, targets)
-                    acc_v += rast.debug(_abi.DEBUG_KERNEL_MS)
-                variants[f"batch{batch}_{'index_order' if order == 0 else 'heavy_first'}"] = round(float(acc_v[6] / 10), 4)
+        for order in (0, 1):
+            vs = raster.RenderSettings(**{**timed.__dict__, "tile_order": order})
+            acc_v = np.zeros(8)
+            for _ in range(10):
+                rast.render(proj, inst, vs, targets)
+                acc_v += rast.debug(_abi.DEBUG_KERNEL_MS)
+            variants["index_order" if order == 0 else "heavy_first"] = round(float(acc_v[6] / 10), 4)
         # Heavy tiles split across waves: the blend at each segment length (0: never split).
         for segment in (0, 256, 512, 1024, 2048):
             vs = raster.RenderSettings(**{**timed.__dict__, "blend_segment": segment})

@@ -729,7 +729,7 @@ void TileRasterizer::enqueueViews(std::span<const SplatInstance> instances, cons
     const uint32_t* pairSlots = values_[sorted].as<uint32_t>();
     const uint32_t* slotOfPair = training ? pairSlot_.as<uint32_t>() : nullptr;
     mark(7);
-    // A persistent blend keeps about 24 one-wave workgroups on each CU.
+    // A persistent blend keeps about 24 waves on each CU (six workgroups of four).
     const bool keepWalk = training || settings.keepWalkState;
     kern::blendViews(settings.depthMode, settings.persistentBlend, computeUnits_ * 24u, params,
                      views, viewCount, tiles, tileShiftOf(settings.tileSize), slots, ranges_.as<uint2>(), pairSlots,

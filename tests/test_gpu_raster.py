@@ -219,9 +219,10 @@ def test_errors_carry_the_reference_codes(rast, cloud):
     assert rast.debug(_abi.DEBUG_COUNTS)[2] == gpu["counts"][2]
 
 
-@pytest.mark.parametrize("batch,order", [(64, 0), (64, 1), (128, 0), (128, 1), (256, 0), (256, 1)])
-def test_every_batch_depth_and_tile_order_draws_the_same_frame(rast, cloud, batch, order):
-    """Batch depth and launch order are performance parameters only."""
+@pytest.mark.parametrize("batch,order", [(256, 0), (256, 1), (64, 1)])
+def test_every_tile_order_draws_the_same_frame(rast, cloud, batch, order):
+    """The launch order is a performance parameter only; blend_batch is accepted
+    at values other than its default and changes nothing."""
     cam, _ = CAMERAS["perspective"]
     s = raster.RenderSettings(width=W, height=HGT, blend_batch=batch, tile_order=order)
     inst = [(cloud, np.eye(4), raster.SplatEdit())]
