@@ -384,13 +384,20 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
     w.accum = addColour<R0 + 1>(colour, weight[1], w.accum);
     w.accum = addColour<R0 + 2>(colour, weight[2], w.accum);
     w.accum = addColour<R0 + 3>(colour, weight[3], w.accum);
+    if constexpr (TRACK) {
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        if constexpr (TRACK) w.lastIn = ok[k] ? first + static_cast<int32_t>(R0 + k) : w.lastIn;
-        if constexpr (DEPTH_MODE == 1) {
-            const bool at = ok[k] & (1.0f - t[k + 1] >= w.depthAt);
-            w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
-            w.depthAt = at ? __builtin_inff() : w.depthAt;
+        for (uint32_t k = 0; k < 4; ++k) w.lastIn = ok[k] ? first + static_cast<int32_t>(R0 + k) : w.lastIn;
+    }
+    if constexpr (DEPTH_MODE == 1) {
+        // T only falls, so a group whose last T finds no pixel's depth holds
+        // none; each pixel's is found once.
+        if (__ballot(walks & (1.0f - t[4] >= w.depthAt)) != 0) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const bool at = ok[k] & (1.0f - t[k + 1] >= w.depthAt);
+                w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
+                w.depthAt = at ? __builtin_inff() : w.depthAt;
+            }
         }
     }
     w.t = walks ? t[4] : w.t;
