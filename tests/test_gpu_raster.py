@@ -594,6 +594,27 @@ def test_a_large_and_a_small_view_in_turn_keep_their_own_order():
     assert torch.equal(images[0], images[1]) and torch.equal(images[0], images[2])
 
 
+def test_a_frame_duplicated_in_vain_bins_as_the_oracle():
+    """A large frame of a shape not drawn before, on a rasteriser whose buffers
+    hold its pairs: they are duplicated before the counts are known, and so many
+    that sorting by depth first still gains. Pairs and ranges are the oracle's,
+    the images and walk state a fresh rasteriser's."""
+    rast = raster.TileRasterizer()
+    cam = _cam((0.0, 0.0, 4.0), (0.0, 0.0, 0.0), focal=30.0)
+    inst = [(_broad_splats(60_011, 3, -2.7), np.eye(4), raster.SplatEdit())]
+    wide = raster.RenderSettings(width=2400, height=1350, time_stages=True)
+    new = raster.RenderSettings(width=2160, height=1215, time_stages=True)
+    assert H.run_gpu(cam, wide, inst, rast)["stats"].depth_sort_ms > 0.0
+    gpu = H.run_gpu(cam, new, inst, rast)
+    ora = H.run_oracle(cam, new, inst)
+    assert 3 * ora["pairs"] > 30_000_000 + 10 * ora["visible"]
+    assert gpu["stats"].depth_sort_ms > 0.0
+    H.assert_bit_exact(dict(gpu, stats=None), ora)
+    fresh = H.run_gpu(cam, new, inst, raster.TileRasterizer())
+    for name in ("colour", "depth", "final_t", "last_count"):
+        np.testing.assert_array_equal(gpu[name].view(np.uint32), fresh[name].view(np.uint32))
+
+
 def test_one_splat_over_millions_of_tiles_draws_as_at_larger_tiles():
     """A single drawn splat past the pair count where slots are sorted by depth
     first: there is nothing to sort, and its pairs are its own. 6.25M 8-pixel
