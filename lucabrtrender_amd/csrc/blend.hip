@@ -12,9 +12,8 @@
 //      group, and leaves once its 64 pixels are opaque. Records and lists hold
 //      two rounds, so one barrier a round is enough.
 // A tile's four quadrants share one gather and one staging of its pairs. With a
-// wave of its own for each quadrant, each gathered and tested all of them: 27M
-// cache accesses a launch against 7.5M, and half of the vector instructions,
-// on 3M splats at 1920x1080.
+// wave of its own for each quadrant, each gathered and tested all of them: 26.9M
+// cache accesses a launch against 7.4M on 3M splats at 1920x1080.
 // A record's Gaussian is expanded about the quadrant's centre and scaled to the
 // exponent's base 2, log2(opacity) added: at a pixel (u, v) from the
 // centre q = A u^2 + B u v + C v^2 + D u + E v + F, the pixel is inside the
@@ -23,17 +22,17 @@
 // scaled power by float rounding only (below 2e-4 on footprints from a quarter
 // pixel to 300 pixels wide, centres up to 3.5 sigma outside the quadrant).
 //
-// What bounds it: the walk, by vector and matrix issue (a group of four records
-// about 250 cycles of a SIMD; the f32 matrix products and the vector FMAs do
-// not overlap), and, where one tile holds many times the others' pairs, that
-// tile's serial chain (about 480 cycles a group when a wave has a SIMD to
-// itself). Form and colour sums on FMAs with the records read from the LDS by
-// broadcast took 96 LDS cycles a group for each of the CU's four SIMDs, more
-// than the arithmetic. Blend time, that form against this one: 3M clustered
-// splats at 1920x1080 225 against 178 us, 2M splats in 64 views 5.30 against
-// 4.43 ms, 1M opaque splats at 1571x877 91 against 78 us. Broadcasting the
-// records by DPP operands instead took 198 us on the first, 4.96 ms on the
-// second.
+// What bounds it: vector issue in the walk (busy 61% of a launch on 3M splats at
+// 1920x1080, the matrix cores 12%; 67 vector instructions a group of four
+// records, staging included), and between its instructions the chain through T,
+// the rounds' gathers and barriers and the launch's last tiles. A wave a quadrant
+// with form and colours on FMAs, the records read from the LDS by broadcast,
+// issued 84.2M vector instructions a launch there against 57.0M, and 10.7M LDS
+// instructions against 5.7M. Blend time, that form against this one: 3M clustered
+// splats at 1920x1080 232 against 197 us, with 1M discs 217 against 178; 2M
+// splats in 64 views 4.93 against 4.11 ms; 1M splats at 1571x877 with the
+// threshold depth 95 against 77 us. Broadcasting the records by DPP operands
+// instead took 198 us where six matrix products for the form took 178.
 //
 // Per pixel it is the reference's splatBlend walk (shaders/lrt/splat/
 // splat_blend.slang:23-108, splat-only entry :110-114): skip past the cutoff,
