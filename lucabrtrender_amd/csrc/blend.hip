@@ -29,9 +29,9 @@
 // with form and colours on FMAs, the records read from the LDS by broadcast,
 // issued 84.2M vector instructions a launch there against 57.0M, and 10.7M LDS
 // instructions against 5.7M. Blend time, that form against this one: 3M clustered
-// splats at 1920x1080 232 against 197 us, with 1M discs 217 against 178; 2M
-// splats in 64 views 4.93 against 4.11 ms; 1M splats at 1571x877 with the
-// threshold depth 95 against 77 us. Broadcasting the records by DPP operands
+// splats at 1920x1080 232 against 194 us, with 1M discs 217 against 179; 2M
+// splats in 64 views 4.93 against 4.10 ms; 1M splats at 1571x877 with the
+// threshold depth 95 against 75 us. Broadcasting the records by DPP operands
 // instead took 198 us where six matrix products for the form took 178.
 //
 // Per pixel it is the reference's splatBlend walk (shaders/lrt/splat/
@@ -311,10 +311,10 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
     for (uint32_t k = 0; k < 4; ++k) {
         const float power2 = __builtin_amdgcn_exp2f(q[k]);
         if constexpr (COMPOSITE) {
-            const float a = __builtin_fminf(kAlphaMax, bound[k] * power2);
+            const float a = bound[k] * power2;
             inside[k] = q[k] >= 0.0f;
             passes[k] = inside[k] & (a >= 1.0f / 255.0f);
-            alpha[k] = passes[k] ? a : 0.0f;
+            alpha[k] = passes[k] ? __builtin_fminf(kAlphaMax, a) : 0.0f;
         } else {
             passes[k] = q[k] >= bound[k];
             alpha[k] = passes[k] ? __builtin_fminf(kAlphaMax, power2) : 0.0f;
@@ -342,11 +342,11 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
                     w.opaqueIn = hit ? first + static_cast<int32_t>(R0 + k) : w.opaqueIn;
                     stop(hit);
                 } else {
-                    const bool ok = (w.t >= kTMin) & passes[k];
-                    weight[k] = w.t * (ok ? alpha[k] : 0.0f);
+                    const bool here = w.t >= kTMin;
+                    weight[k] = (here ? w.t : 0.0f) * alpha[k];
                     w.t = w.t - weight[k];
                     if constexpr (DEPTH_MODE == 1) {
-                        const bool at = ok & (1.0f - w.t >= w.depthAt);
+                        const bool at = here & passes[k] & (1.0f - w.t >= w.depthAt);
                         w.depthIn = at ? first + static_cast<int32_t>(R0 + k) : w.depthIn;
                         w.depthAt = at ? __builtin_inff() : w.depthAt;
                     }
@@ -405,7 +405,8 @@ __device__ __forceinline__ void walkGroup(WalkLane& w, Vec4 q, float colour, flo
 // Up to sixteen records, whose A, B and C lanes 0 .. 15 hold and whose colours
 // `colour` does (lane l: channel l & 3 of record l / 4), four a group in order,
 // while there are records and the wave has a pixel that walks; the next group's
-// form is computed while this one is blended. Returns the records walked.
+// form is computed, and its bounds read, while this one is blended. Returns the
+// records walked.
 template <uint32_t DEPTH_MODE, bool COMPOSITE, bool TRACK>
 __device__ __forceinline__ uint32_t walkSixteen(WalkLane& w, uint32_t records, const float form[3], float colour,
                                                 float u, float v, const float4 (*chunk)[kLanes / 4], uint32_t at,
@@ -413,15 +414,23 @@ __device__ __forceinline__ uint32_t walkSixteen(WalkLane& w, uint32_t records, c
                                                 int32_t first) {
     uint32_t walked = 0;
     Vec4 q = formOf<0>(form, u, v, chunk, at);
+    float4 bound = chunk[3][at];
+    float4 reach = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (COMPOSITE) reach = chunkReach[0];
     const auto group = [&](auto g) -> bool {
         constexpr uint32_t G = decltype(g)::value;
         if (G * kGroup >= records) return false;
-        Vec4 next = q;
-        if constexpr (G + 1 < 16 / kGroup) next = formOf<G + 1>(form, u, v, chunk, at);
-        float4 reach = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if constexpr (COMPOSITE) reach = chunkReach[G];
-        walkGroup<DEPTH_MODE, COMPOSITE, TRACK, G>(w, q, colour, chunk[3][at + G], reach, stopZ, discs, first);
-        q = next;
+        Vec4 nextQ = q;
+        float4 nextBound = bound, nextReach = reach;
+        if constexpr (G + 1 < 16 / kGroup) {
+            nextQ = formOf<G + 1>(form, u, v, chunk, at);
+            nextBound = chunk[3][at + G + 1];
+            if constexpr (COMPOSITE) nextReach = chunkReach[G + 1];
+        }
+        walkGroup<DEPTH_MODE, COMPOSITE, TRACK, G>(w, q, colour, bound, reach, stopZ, discs, first);
+        q = nextQ;
+        bound = nextBound;
+        reach = nextReach;
         walked += kGroup;
         return __ballot(w.t >= kTMin) != 0;
     };
